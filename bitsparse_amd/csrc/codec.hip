@@ -11,6 +11,7 @@
 #include "bs_device.h"
 #include "bs_host.h"
 #include "compact.h"
+#include "tile_rows.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -669,15 +670,16 @@ void compress_stream_kernel(CompressArgs a)
         // column (< 8 N elements: the host takes this path only when 8 N
         // elements of the widest operand fit 32 bits)
         const uint64_t t_org = (uint64_t)tm * 64 * (uint64_t)a.N + (uint64_t)tn * 64;
+        const int64_t rows_t = a.M - (int64_t)tm * 64;      // rows of the tile inside the matrix (>= 1)
         const uint32_t r_in = (uint32_t)(lane >> 3) * (uint32_t)a.N;
         const uint32_t c_in = (uint32_t)(min(col0, a.N - 8) - (int64_t)tn * 64);
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             const int64_t row = row0 + 8 * k;
             if constexpr (VEC) {
-                // rows past the matrix read the tile's first row (in range)
+                // a row past the matrix reads an in-range row of the tile
                 const uint32_t lo = (row < a.M ? r_in : 0u) + c_in;
-                d[k] = ld_chunk<NT, RawIn>(a.dense + (t_org + (uint64_t)(8 * k) * (uint64_t)a.N) * INB +
+                d[k] = ld_chunk<NT, RawIn>(a.dense + (t_org + (uint64_t)row_step(k, rows_t) * (uint64_t)a.N) * INB +
                                            (uint64_t)(lo * (uint32_t)INB));
             } else {
                 d[k] = tile_ok ? load_chunk<INB, false>(a.dense, a.M, a.N, row, col0) : RawIn{};
