@@ -353,7 +353,6 @@ def test_to_fp8(dev, shape):
     assert qt.shape == x.T.shape and (bits(qt.contiguous()) == qo.T).all()
 
 
-@pytest.mark.skip(reason="a GPU memory fault ended the full GPU test run after this test was added; no cause found yet, so it stays off the GPU")
 def test_to_fp8_misaligned_input(dev):
     """A contiguous view starting 2 bytes into its storage, of odd length: the
     amax and the quantizer take their per-element paths (no 16-byte vectors),

@@ -168,7 +168,6 @@ def _relu2_special_inputs(dev, B=304, D=192, H=528, seed=9):
     return [t.to(dev) for t in (x, W1, W2, dY)]
 
 
-@pytest.mark.skip(reason="a GPU memory fault ended the full GPU test run after this test was added; no cause found yet, so it stays off the GPU")
 @pytest.mark.parametrize("storage", ["bf16", "e4m3fn"])
 def test_relu2_square_fused_into_compress(dev, monkeypatch, storage):
     """Relu2Linear with the square written back by the compress pass (and,
@@ -210,7 +209,6 @@ def test_relu2_square_fused_into_compress(dev, monkeypatch, storage):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (name, special)
 
 
-@pytest.mark.skip(reason="a GPU memory fault ended the full GPU test run after this test was added; no cause found yet, so it stays off the GPU")
 @pytest.mark.parametrize("k", [1.0, 0.5, 3.0, -2.0, 0.0])
 def test_relu2_amax_derived_from_relu_amax(dev, k):
     """amax|bf16(bf16(r*r) * k)| from amax|relu(z)| (bs_amax_relu2_from)
