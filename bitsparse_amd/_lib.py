@@ -17,7 +17,7 @@ LIB_NAME = "libbitsparse_hip.so"
 # BITSPARSE_HIP_LIB points at another build of the same sources (tuning sweeps)
 LIB_PATH = os.environ.get("BITSPARSE_HIP_LIB") or os.path.join(
     os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 BS_OK = 0
 BS_ERR_INVALID = 1
@@ -83,6 +83,8 @@ _SIGNATURES = {
     "bs_compress_noalloc": [_vp, _int, _i64, _i64, _int, _int, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _int,
                             _vp, _vp, _int, _vp, _vp, _vp],
     "bs_compress_noalloc_max_tiles": [],
+    "bs_col_sum_workspace_bytes": [_i64, _i64],
+    "bs_col_sum": [_vp, _i64, _i64, _vp, _vp, _i64, _vp],
     "bs_launch_timing": [_int],
     "bs_nontemporal_min_bytes": [_i64],
     "bs_launch_timing_read": [_vp, _vp, _int, _vp],
@@ -96,6 +98,7 @@ _RESTYPES = {
     "bs_gemm_compressed_b_packed_workspace_bytes": _i64,
     "bs_compress_noalloc_max_tiles": _i64,
     "bs_linear_relu_compress_max_n": _i64,
+    "bs_col_sum_workspace_bytes": _i64,
     "bs_nontemporal_min_bytes": _i64,
     "bs_workspace_amax_slot": _vp,
     "bs_workspace_fallback_counter": _vp,

@@ -141,6 +141,22 @@ class MatmulFp8(Function):
         return grad_a, grad_b, None, None
 
 
+def linear_fp8_backward(x: Tensor, W: Tensor, grad_z: Tensor, need_x: bool,
+                        need_W: bool) -> tuple[Tensor | None, Tensor | None]:
+    """(grad of x, grad of W) of z = matmul(x, W.T, True) for bf16 x and W:
+    ``MatmulFp8``'s backward with its operands quantized again, W's gradient
+    in W's own layout."""
+    g = Fp8Operand(*to_fp8(grad_z))
+    grad_x = grad_W = None
+    if need_x:
+        w = as_fp8_operand(W, None)
+        grad_x = _as_input_dtype(fp8_gemm(g, w, _grad_dtype(w.codes.dtype)), x.dtype)
+    if need_W:
+        a = as_fp8_operand(x, None)
+        grad_W = _as_input_dtype(fp8_gemm(g.T, a, _grad_dtype(a.codes.dtype)), W.dtype)
+    return grad_x, grad_W
+
+
 def _as_input_dtype(grad: Tensor, in_dtype: torch.dtype) -> Tensor:
     """An e4m3fn gradient of a bf16 input widened to bf16 by the HIP kernel
     (exact; the cast autograd would otherwise make with torch's float8 copy)."""

@@ -12,15 +12,17 @@ from __future__ import annotations
 
 import torch
 from torch import Tensor
-from torch.autograd import Function
+from torch.autograd import Function, forward_ad
 
+from . import config
 from .bitsparse import BitsparseTensor, TensorBuffer
 from .config import RELU2_SCALE
-from .fp8 import is_fp8, matmul, to_fp8
+from .fp8 import Fp8Operand, as_fp8_operand, fp8_gemm, is_fp8, linear_fp8_backward, matmul, to_fp8
 from .src.functions import (fused_linear_relu_ok, linear_relu_and_compress, relu2_and_compress,
                             relu2_fused_ok, relu2_quantize_and_compress, relu_and_compress,
                             relu_quantize_and_compress)
-from .src.hip_operators import mask_with_bitmask_, quantize_e4m3fn, relu2_grad_sparse_, relu2_square_amax_
+from .src.hip_operators import (col_sum, col_sum_supported, mask_with_bitmask_, quantize_e4m3fn,
+                                relu2_grad_sparse_, relu2_square_amax_)
 from .src.sparse_matmul import AspB, AspRelu2B
 
 # FFNRelu / FFNRelu2 with bf16 storage into a TensorBuffer run the up-projection
@@ -40,6 +42,11 @@ class ReluLinear(Function):
                 dtype: torch.dtype = torch.bfloat16):
         ctx.dtype = dtype
         ctx.save_for_backward(W)
+        y, ctx.h_sparse = ReluLinear.activate_and_project(z, W, sparse_data, pack_sbit, dtype)
+        return y
+
+    @staticmethod
+    def activate_and_project(z, W, sparse_data, pack_sbit, dtype) -> tuple[Tensor, BitsparseTensor]:
         # h = z.relu_() fused into the compress pass (z is still updated in place)
         if is_fp8(dtype):
             # any fp8 dtype stores e4m3fn codes + scale: the reference quantizes
@@ -48,10 +55,7 @@ class ReluLinear(Function):
         else:
             scale = None
             h, h_sparse = relu_and_compress(z, sparse_data, pack_sbit)
-
-        ctx.h_sparse = h_sparse
-        y = matmul(h, W.T, is_fp8(dtype), a_scale=scale)
-        return y
+        return matmul(h, W.T, is_fp8(dtype), a_scale=scale), h_sparse
 
     @staticmethod
     @torch.compiler.disable
@@ -89,6 +93,9 @@ class FFNRelu:
         bs_dims = x.shape[:-1]
         x = x.reshape(-1, x.shape[-1])
 
+        if _block_ok(x, W1, W2, b1, b2):
+            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, pack_sbit, dtype, False)
+            return y.reshape(*bs_dims, y.shape[-1])
         if not is_fp8(dtype) and not pack_sbit and USE_FUSED_UP and fused_linear_relu_ok(x, W1, b1, sparse_data):
             y = _UpReluLinear.apply(x, W1, b1, W2, sparse_data, False)
         else:
@@ -114,6 +121,11 @@ class Relu2Linear(Function):
                 storage_dtype: torch.dtype = torch.bfloat16):
         ctx.dtype = storage_dtype
         ctx.save_for_backward(W)
+        y, ctx.h_sparse = Relu2Linear.activate_and_project(z, W, sparse_data, pack_sbit, storage_dtype)
+        return y
+
+    @staticmethod
+    def activate_and_project(z, W, sparse_data, pack_sbit, storage_dtype) -> tuple[Tensor, BitsparseTensor]:
         # h = z.relu_() fused into the compress pass (z is still updated in place)
         fused_sq = relu2_fused_ok(z, sparse_data, pack_sbit, RELU2_SCALE)
         if is_fp8(storage_dtype):
@@ -127,10 +139,9 @@ class Relu2Linear(Function):
                 _, _, h_sparse = relu_quantize_and_compress(z, sparse_data, pack_sbit, dense_out=False)
                 # h.square_(); h.mul_(k) and the amax of to_fp8(h) in one pass
                 epoch = relu2_square_amax_(z, RELU2_SCALE)
-            ctx.h_sparse = h_sparse
             # h ends up in z, as the reference's in-place ops leave it
             h8, h_scale = quantize_e4m3fn(z, epoch)
-            return matmul(h8, W.T, True, a_scale=h_scale)
+            return matmul(h8, W.T, True, a_scale=h_scale), h_sparse
         if fused_sq:
             h_sparse = relu2_and_compress(z, sparse_data, RELU2_SCALE)
             h = z
@@ -142,8 +153,7 @@ class Relu2Linear(Function):
             else:
                 h.square_()
                 h.mul_(RELU2_SCALE)
-        ctx.h_sparse = h_sparse
-        return matmul(h, W.T, False)
+        return matmul(h, W.T, False), h_sparse
 
     @staticmethod
     @torch.compiler.disable
@@ -178,6 +188,9 @@ class FFNRelu2:
               storage_dtype: torch.dtype = torch.bfloat16):
         bs_dims = x.shape[:-1]
         x = x.reshape(-1, x.shape[-1])
+        if _block_ok(x, W1, W2, b1, b2):
+            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, pack_sbit, storage_dtype, True)
+            return y.reshape(*bs_dims, y.shape[-1])
         if (not is_fp8(storage_dtype) and not pack_sbit and USE_FUSED_UP
                 and fused_linear_relu_ok(x, W1, b1, sparse_data)):
             y = _UpReluLinear.apply(x, W1, b1, W2, sparse_data, True)
@@ -190,6 +203,93 @@ class FFNRelu2:
         if b2 is not None:
             y = y + b2
         return y
+
+
+# ------------------------------------------------------------
+# the whole block as one autograd node
+# ------------------------------------------------------------
+def _plain(t: Tensor) -> bool:
+    return type(t) in (Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.bfloat16
+
+
+def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor | None) -> bool:
+    """The MLP block runs as one node (``_FFNBlock``): plain bf16 matrices on
+    the GPU and bias rows, outside autocast, tracing, forward-mode AD and the
+    options that choose another path.  Everything else takes the layers'
+    separate nodes, with their errors."""
+    if not (_plain(x) and _plain(W1) and _plain(W2)) or USE_FUSED_UP or config.CACHE_FP8_MATMUl:
+        return False
+    if x.dim() != 2 or W1.dim() != 2 or W2.dim() != 2 or 0 in x.shape or 0 in W1.shape or 0 in W2.shape:
+        return False
+    if x.shape[1] != W1.shape[1] or W1.shape[0] != W2.shape[1]:
+        return False
+    if not (W1.is_contiguous() and W2.is_contiguous() and x.device == W1.device == W2.device):
+        return False
+    for b, n in ((b1, W1.shape[0]), (b2, W2.shape[0])):
+        if b is not None and not (_plain(b) and b.shape == (n,) and b.is_contiguous() and b.device == x.device):
+            return False
+    return (not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
+            and not torch.compiler.is_compiling())
+
+
+class _FFNBlock(Function):
+    """y = act(x @ W1.T + b1) @ W2.T + b2 with act(z) = relu(z) or
+    k * relu(z)^2 saved compressed: the products, quantizations and kernels of
+    the nodes it stands for (``matmul``, the bias adds, ``ReluLinear`` /
+    ``Relu2Linear``), in their order and with their roundings.  What the one
+    node adds is what crosses them: bias gradients are column sums of the
+    gradients at hand."""
+
+    @staticmethod
+    def forward(ctx, x, W1, b1, W2, b2, sparse_data, pack_sbit, dtype, square):
+        fp8 = is_fp8(dtype)
+        ctx.save_for_backward(x, W1, W2)
+        ctx.fp8, ctx.square = fp8, square
+        if fp8:
+            z = fp8_gemm(as_fp8_operand(x, None), as_fp8_operand(W1.T, None), torch.bfloat16)
+        else:
+            z = x @ W1.T
+        if b1 is not None:
+            z = z + b1
+        down = Relu2Linear if square else ReluLinear
+        y, ctx.h_sparse = down.activate_and_project(z, W2, sparse_data, pack_sbit, dtype)
+        return y if b2 is None else y + b2
+
+    @staticmethod
+    @torch.compiler.disable
+    def backward(ctx, grad_output: Tensor):
+        x, W1, W2 = ctx.saved_tensors
+        h: BitsparseTensor = ctx.h_sparse
+        ctx.h_sparse = None
+        need_x, need_W1, need_b1, need_W2, need_b2 = ctx.needs_input_grad[:5]
+        grad_x = grad_W1 = grad_b1 = grad_W2 = grad_b2 = None
+        if need_b2:
+            grad_b2 = _col_sum(grad_output)
+        scale = None
+        if ctx.fp8:
+            grad_output, scale = to_fp8(grad_output)
+        if need_W2:
+            product = AspRelu2B if ctx.square else AspB
+            grad_W2 = product(grad_output.T, h, A_scale=scale)
+        if need_x or need_W1 or need_b1:
+            if ctx.fp8:
+                grad_h = fp8_gemm(Fp8Operand(grad_output, scale), as_fp8_operand(W2, None), torch.bfloat16)
+            else:
+                grad_h = grad_output @ W2
+            grad_z = relu2_grad_sparse_(grad_h, h) if ctx.square else mask_with_bitmask_(grad_h, h)
+            if need_b1:
+                grad_b1 = _col_sum(grad_z)
+            if ctx.fp8:
+                grad_x, grad_W1 = linear_fp8_backward(x, W1, grad_z, need_x, need_W1)
+            else:
+                grad_x = grad_z.mm(W1) if need_x else None
+                grad_W1 = grad_z.t().mm(x) if need_W1 else None   # W1's own layout, as autograd forms it
+        return grad_x, grad_W1, grad_b1, grad_W2, grad_b2, None, None, None, None
+
+
+def _col_sum(g: Tensor) -> Tensor:
+    # a graph of this gradient (create_graph) needs torch's own sum
+    return col_sum(g) if col_sum_supported(g) and not torch.is_grad_enabled() else g.sum(0)
 
 
 # ------------------------------------------------------------

@@ -453,6 +453,24 @@ def _check_grad(grad: Tensor, sparse: BitsparseTensor, what: str) -> None:
         raise ValueError(f"{what}: grad shape {tuple(grad.shape)} != {tuple(sparse.shape)}")
 
 
+def col_sum_supported(x: Tensor) -> bool:
+    """Whether ``col_sum`` takes x as it is."""
+    return (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and x.is_contiguous() and x.shape[0] > 0
+            and x.shape[1] > 0 and x.shape[1] % 8 == 0 and x.data_ptr() % 16 == 0 and x.numel() < 2 ** 31)
+
+
+def col_sum(x: Tensor) -> Tensor:
+    """x.sum(0) of a bf16 matrix (``col_sum_supported``), in fp32, rounded once."""
+    R, C = x.shape
+    L = _lib.load()
+    out = torch.empty(C, device=x.device, dtype=torch.bfloat16)
+    need = L.bs_col_sum_workspace_bytes(R, C)
+    part = torch.empty(need, device=x.device, dtype=torch.uint8)
+    check(L.bs_col_sum(x.data_ptr(), R, C, out.data_ptr(), part.data_ptr(), need, stream_handle(x.device)),
+          "bs_col_sum")
+    return out
+
+
 def mask_with_bitmask_(grad: Tensor, sparse: BitsparseTensor) -> Tensor:
     """grad <- grad * bitmask, in place.  Reference: triton_operators.py:165-175."""
     _check_grad(grad, sparse, "mask_with_bitmask_")

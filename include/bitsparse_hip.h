@@ -531,6 +531,18 @@ int bs_compress_noalloc(const void* dense, int in_dtype, int64_t M, int64_t N, i
 int64_t bs_compress_noalloc_max_tiles(void);
 
 /*
+ * Column sums of a bf16 [R, C] matrix (row-major, contiguous, 16-byte
+ * aligned, C % 8 == 0, R >= 1): out[c] = bf16(sum over r of x[r, c]), summed
+ * in fp32 (partial sums of row blocks, added in order).  workspace: at least
+ * bs_col_sum_workspace_bytes(R, C) bytes, any contents.  Replaces the
+ * grad.sum(0) autograd makes for the bias adds of lib_sparse/layers.py:86-94
+ * and :169-177.
+ */
+int64_t bs_col_sum_workspace_bytes(int64_t R, int64_t C);
+int bs_col_sum(const void* x, int64_t R, int64_t C, void* out, void* workspace, int64_t workspace_bytes,
+               void* stream);
+
+/*
  * bs_stream_probe — no counterpart in the reference: a measurement kernel, the
  * floor of the codec kernels' HBM access mix.  mode 0 (compress mix): read the
  * [M, N] bf16 matrix `dense` in the compress kernel's load pattern (8 tiles per
