@@ -102,6 +102,16 @@ __device__ __forceinline__ uint32_t f32_to_bf16(float f)
     return __builtin_bit_cast(uint16_t, (__bf16)f);
 }
 
+// the two bf16 halves of a + those of b, each sum rounded once
+__device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b)
+{
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const f32x2 s = {__uint_as_float(a << 16) + __uint_as_float(b << 16),
+                     __uint_as_float(a & 0xffff0000u) + __uint_as_float(b & 0xffff0000u)};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(s, bf16x2));
+}
+
 // e4m3fn bits -> fp32 (exact). 0x7f / 0xff are NaN.
 __device__ __forceinline__ float e4m3_to_f32(uint32_t b)
 {

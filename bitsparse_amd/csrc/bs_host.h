@@ -71,6 +71,12 @@ hipError_t stream_device(hipStream_t stream, int* dev);
 int amax_launch(const void* x, int64_t n, void* workspace, int64_t workspace_bytes, uint32_t epoch,
                 void* stream, bool relu, bool check_capture);
 
+// The second pass of column sums and of per-workgroup maxima: out[c] (bf16,
+// with part) = sum over S partial rows of part[., c]; with maxima, their
+// largest into the amax slot under `epoch`.  Either may be null.
+int sums_finish_launch(const float* part, int64_t S, int64_t C, void* out, const uint32_t* maxima, int64_t nmax,
+                       uint64_t* slot, uint32_t epoch, hipStream_t stream);
+
 // Records a formatted message for bs_last_error() and returns `code`.
 int set_error(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 void clear_error();

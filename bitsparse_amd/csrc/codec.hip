@@ -113,13 +113,39 @@ __device__ __forceinline__ uint2 quant_chunk(const uint4 v, float scale, float r
     return uint2{p[0] | (p[1] << 16), p[2] | (p[3] << 16)};
 }
 
-// entry i of each half stands for magnitude base + i - 1 (the end entries
-// for every magnitude past them); scale from the amax slot
-__global__ __launch_bounds__(256) void qtab_build_kernel(const uint64_t* slot, uint32_t epoch, uint8_t* qtab)
+// The same rule for the scale of h = bf16(bf16(r * r) * k) over the tensor
+// whose amax|r| the slot holds (r >= 0 or NaN, k finite: |h| is non-decreasing
+// in r, so amax|h| is that of the largest r).
+__device__ __forceinline__ float relu2_scale_from_slot(const uint64_t* slot, uint32_t epoch, float k)
 {
-    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+    uint64_t s = *slot;
+    const uint32_t m = ((uint32_t)(s >> 32) == epoch) ? (uint32_t)s & 0x7fffu : 0u;
+    float sc = bf16_to_f32(relu2_sq_bits(m, k) & 0x7fffu) / 448.0f;
+    return (sc < 1e-9f) ? 1e-9f : sc;
+}
+
+// z + b of 8 bf16 values, each sum rounded to bf16 as torch's add rounds it
+__device__ __forceinline__ uint4 add_bias_chunk(const uint4 z, const uint4 b)
+{
+    const uint32_t w[4] = {z.x, z.y, z.z, z.w}, c[4] = {b.x, b.y, b.z, b.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = add_bf16x2(w[i], c[i]);
+    return uint4{o[0], o[1], o[2], o[3]};
+}
+
+// entry i of each half stands for magnitude base + i - 1 (the end entries
+// for every magnitude past them); scale from the amax slot, for the second
+// table (blocks from kQtabBlocks on) that of h = k r^2
+constexpr int kQtabBlocks = (kQtabEntries + 255) / 256;
+__global__ __launch_bounds__(256) void qtab_build_kernel(const uint64_t* slot, uint32_t epoch, uint8_t* qtab,
+                                                         float k)
+{
+    const bool h = blockIdx.x >= kQtabBlocks;
+    const int i = (int)((blockIdx.x - (h ? kQtabBlocks : 0)) * 256 + threadIdx.x);
     if (i >= kQtabEntries) return;
-    const float scale = scale_from_slot(slot, epoch);
+    const float scale = h ? relu2_scale_from_slot(slot, epoch, k) : scale_from_slot(slot, epoch);
+    if (h) qtab += kQtabBytes;
     const int m = min(max(qtab_offset(scale) + i, 0), 0x7fff);
     const uint32_t c = f32_to_e4m3(bf16_to_f32((uint32_t)m) / scale);
     if (scale != scale) {
@@ -173,8 +199,23 @@ struct CompressArgs {
     uint32_t* fallbacks;
     uint64_t patience;          // look-back wait (s_memrealtime ticks) before counting a unit itself
     const uint8_t* qtab;        // quantize: the code table (kQtabBytes), copied into LDS
-    float relu_k;               // RSQ: relu_out receives bf16(bf16(r * r) * relu_k), r = relu(dense)
+    float relu_k;               // WB_SQUARE / WB_ACT_SQUARE: h = bf16(bf16(r * r) * relu_k), r = relu(dense)
+    const uint16_t* bias;       // WB_ACT*: nullable, dense + bias is the pre-activation
+    float* h_scale_out;         // WB_ACT_SQUARE, quantizing: scale of h's codes
 };
+
+// What the fused pass writes back beside the compressed form of r, and what
+// it reads:
+//   WB_RELU        relu_out (nullable) receives r
+//   WB_SQUARE      relu_out receives the ReLU^2 layer's h = k r^2
+//   WB_ACT         the activation step inside an MLP block, whose
+//                  pre-activation nothing else reads: bias (nullable) is added
+//                  first, and only what the down-projection multiplies is
+//                  written -- r to relu_out, or (quantizing) its codes
+//   WB_ACT_SQUARE  the same for h: h to relu_out, or (quantizing) the e4m3fn
+//                  codes of h, whose scale follows from the amax of r because
+//                  |h| is non-decreasing in r
+enum { WB_RELU = 0, WB_SQUARE = 1, WB_ACT = 2, WB_ACT_SQUARE = 3 };
 
 // 200 us at the 100 MHz s_memrealtime clock: waiting longer than this for a
 // predecessor makes the waiter count that predecessor's tiles itself (a
@@ -592,16 +633,19 @@ __device__ __forceinline__ void packed_unit_edges(const CompressArgs& a, int64_t
 #endif
 
 // NT: nontemporal loads of the dense input and stores of the value slots.
-// RSQ: the fused ReLU's write-back is the ReLU^2 layer's in-place square
-// (relu2_sq_bits of relu(dense)); the compressed form is that of relu(dense).
-template <int IN_T, bool QUANT, bool VEC, int MODE, int U, bool PACKED, bool NT, bool RSQ = false>
+// WB: what is written back (above); the compressed form is that of relu(dense).
+template <int IN_T, bool QUANT, bool VEC, int MODE, int U, bool PACKED, bool NT, int WB = WB_RELU>
 __global__ __launch_bounds__(64 * U) __attribute__((amdgpu_waves_per_eu(
     QUANT ? BS_QUANT_WAVES_PER_EU : (PACKED ? BS_PACKED_WAVES_PER_EU : BS_STREAM_WAVES_PER_EU))))
 void compress_stream_kernel(CompressArgs a)
 {
     static_assert(!(QUANT && MODE == MODE_VALS), "the values pass copies stored values");
     static_assert(!PACKED || MODE == MODE_FUSED, "the packed stream is written by the fused pass");
-    static_assert(!RSQ || (IN_T == DT_BF16 && MODE == MODE_FUSED && !PACKED), "the ReLU^2 write-back");
+    static_assert(WB == WB_RELU || (IN_T == DT_BF16 && MODE == MODE_FUSED), "the ReLU^2 write-back");
+    constexpr bool ACT = WB == WB_ACT || WB == WB_ACT_SQUARE;
+    static_assert(!ACT || VEC, "the activation step takes vector loads");
+    constexpr bool RSQ = WB == WB_SQUARE || (WB == WB_ACT_SQUARE && !QUANT), HCODES = WB == WB_ACT_SQUARE && QUANT;
+    constexpr int kTabs = HCODES ? 2 : 1;   // code tables: r's, and h's behind it
     constexpr bool WRITE_VALS = MODE != MODE_COUNT;
     using TR = CompressTraits<IN_T, QUANT>;
     constexpr int INB = TR::INB, OUTB = TR::OUTB;
@@ -619,7 +663,7 @@ void compress_stream_kernel(CompressArgs a)
     // the quantizer's code table is read only while the chunks are masked,
     // the value rings only after the look-back's barrier: they share LDS
     constexpr int kRingBytes = WRITE_VALS ? U * kRingElems * OUTB : 16;
-    constexpr int kShared = QUANT && kQtabBytes > kRingBytes ? kQtabBytes : kRingBytes;
+    constexpr int kShared = QUANT && kTabs * kQtabBytes > kRingBytes ? kTabs * kQtabBytes : kRingBytes;
     __shared__ __align__(16) uint8_t s_area[kShared];
     uint8_t* const s_ring = s_area;
     uint8_t* const s_qtab = s_area;
@@ -636,6 +680,9 @@ void compress_stream_kernel(CompressArgs a)
     if constexpr (QUANT) scale = scale_from_slot(a.amax_slot, a.amax_epoch);
     const float rcp = 1.0f / scale;
     const int qoff = QUANT ? qtab_offset(scale) : 0;
+    float h_scale = 1.0f;
+    if constexpr (HCODES) h_scale = relu2_scale_from_slot(a.amax_slot, a.amax_epoch, a.relu_k);
+    const int hoff = HCODES ? qtab_offset(h_scale) : 0;
     int64_t start = 0;
     if (a.offset_in) start = *a.offset_in;
     if (a.align8) start = (start + 7) & ~(int64_t)7;
@@ -698,11 +745,18 @@ void compress_stream_kernel(CompressArgs a)
         }
         if constexpr (QUANT) {
             // the code table into LDS, behind the dense loads (16-byte copies)
-            for (int i = tid; i < kQtabBytes / 16; i += 64 * U)
+            for (int i = tid; i < kTabs * kQtabBytes / 16; i += 64 * U)
                 reinterpret_cast<uint4*>(s_qtab)[i] = reinterpret_cast<const uint4*>(a.qtab)[i];
             __syncthreads();
         }
         if constexpr (MODE != MODE_VALS) {
+            if constexpr (ACT) {
+                if (a.bias != nullptr) {
+                    const uint4 b = *reinterpret_cast<const uint4*>(a.bias + (uint64_t)tn * 64 + c_in);
+#pragma unroll
+                    for (int k = 0; k < 8; k++) d[k] = add_bias_chunk(d[k], b);
+                }
+            }
             if (a.relu) {
 #pragma unroll
                 for (int k = 0; k < 8; k++) d[k] = relu_chunk<IN_T>(d[k]);
@@ -735,7 +789,12 @@ void compress_stream_kernel(CompressArgs a)
                             else
                                 st_chunk<false, RawIn>(a.relu_out + ko * INB + (uint64_t)(lo * (uint32_t)INB), d[k]);
                         }
-                        if constexpr (QUANT) {
+                        if constexpr (HCODES) {
+                            if (8 * k < rows_in)
+                                st_chunk<false, RawOut>(a.dense_q_out + ko + (uint64_t)lo,
+                                                        quant_chunk_tab(relu2_sq_chunk(d[k], a.relu_k),
+                                                                        s_qtab + kQtabBytes, hoff));
+                        } else if constexpr (QUANT) {
                             if (a.dense_q_out != nullptr && 8 * k < rows_in)
                                 st_chunk<false, RawOut>(a.dense_q_out + ko + (uint64_t)lo, o[k]);
                         }
@@ -847,6 +906,9 @@ void compress_stream_kernel(CompressArgs a)
             }
             if constexpr (QUANT) {
                 if (u == 0 && lane == 0 && a.scale_out) *a.scale_out = scale;
+                if constexpr (HCODES) {
+                    if (u == 0 && lane == 0 && a.h_scale_out) *a.h_scale_out = h_scale;
+                }
             }
         }
         if constexpr (WRITE_VALS) {
@@ -1138,7 +1200,60 @@ struct GatherArgs {
     uint32_t num_tiles;
     float relu2_scale;
     const float* scale;
+    float* col_part;       // SUMS: nullable, [tile rows, K] column sums of the written gradient
+    uint32_t* wg_max;      // SUMS: nullable, per workgroup, the largest magnitude written (bf16 bits)
 };
+
+// Column sums and amax of the gradient a workgroup writes, for the bias
+// gradient and the fp8 quantizer that read it next: both are taken from the
+// registers it is stored from, which saves two reads of the matrix (26 and
+// 23 us at 4096 x 16384) for ~4 us here.  cs[j][e]: this thread's sum of
+// column e of its chunks of tile j (fp32, two rows), mx its largest magnitude.
+// `lds`: U * 8 KiB, free once every thread is here.  Tile t's 64 sums go to
+// row t / grid_n of col_part.
+template <int U>
+__device__ __forceinline__ void write_grad_sums(const float (&cs)[U][8], uint32_t mx, float* lds, uint32_t t0,
+                                                int ntiles, uint32_t grid_n, int64_t K, float* col_part,
+                                                uint32_t* wg_max, int tid)
+{
+    __shared__ uint32_t s_mx[kThreads / 64];
+    const uint32_t wmx = wave_max_u32(mx);
+    if ((tid & 63) == 0) s_mx[tid >> 6] = wmx;
+    __syncthreads();
+    if (wg_max != nullptr && tid == 0) wg_max[blockIdx.x] = max(max(s_mx[0], s_mx[1]), max(s_mx[2], s_mx[3]));
+    if (col_part == nullptr) return;
+#pragma unroll
+    for (int j = 0; j < U; j++)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+            *reinterpret_cast<float4*>(&lds[(j * 32 + (tid >> 3)) * 64 + (tid & 7) * 8 + e]) =
+                float4{cs[j][e], cs[j][e + 1], cs[j][e + 2], cs[j][e + 3]};
+    __syncthreads();
+    for (int i = tid; i < ntiles * 64; i += kThreads) {
+        const int j = i >> 6, c = i & 63;
+        float a = 0.f, b = 0.f;
+#pragma unroll
+        for (int r = 0; r < 32; r += 2) {
+            a += lds[(j * 32 + r) * 64 + c];
+            b += lds[(j * 32 + r + 1) * 64 + c];
+        }
+        const uint32_t tm = (t0 + j) / grid_n, tn = (t0 + j) - tm * grid_n;
+        const int64_t col = (int64_t)tn * 64 + c;
+        if (col < K) col_part[(int64_t)tm * K + col] = a + b;
+    }
+}
+
+// adds a written chunk to its column sums and the magnitude maximum
+__device__ __forceinline__ void grad_sums_add(float (&cs)[8], uint32_t& mx, const uint4 v)
+{
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        cs[2 * i] += __uint_as_float(w[i] << 16);
+        cs[2 * i + 1] += __uint_as_float(w[i] & 0xffff0000u);
+        mx = max(mx, max(w[i] & 0x7fffu, (w[i] >> 16) & 0x7fffu));
+    }
+}
 
 // Stage the value run of tiles [t0, t0+ntiles) in LDS; returns its phase.
 // The run is [vo + prefix[t0], vo + prefix[t0+ntiles]).
@@ -1607,7 +1722,8 @@ __global__ __launch_bounds__(kThreads) void decompress_fp8_kernel(GatherArgs a, 
 
 // grad = bit ? bf16(grad * (2k * r)) : 0, then optionally grad = bf16(grad * bf16(scale))
 // NT: nontemporal gradient loads / stores and staging loads.
-template <int V_T, bool HAS_SCALE, bool VEC, int U, bool PACKED, bool NT>
+// SUMS: also the column sums and the amax of what is written (write_grad_sums).
+template <int V_T, bool HAS_SCALE, bool VEC, int U, bool PACKED, bool NT, bool SUMS = false>
 __global__ __launch_bounds__(kThreads) void relu2_grad_kernel(GatherArgs a)
 {
     constexpr int VB = V_T == DT_BF16 ? 2 : 1;
@@ -1666,6 +1782,8 @@ __global__ __launch_bounds__(kThreads) void relu2_grad_kernel(GatherArgs a)
     if constexpr (HAS_SCALE) sb = bf16_to_f32(f32_to_bf16(sc));
     const uint32_t zero_x = HAS_SCALE ? f32_to_bf16(0.0f * sb) : 0u;
     const float k2 = 2.0f * a.relu2_scale;
+    float cs[SUMS ? U : 1][8] = {};
+    uint32_t mx = 0;
 #pragma unroll
     for (int j = 0; j < U; j++) {
         if (j >= ntiles) break;
@@ -1690,18 +1808,30 @@ __global__ __launch_bounds__(kThreads) void relu2_grad_kernel(GatherArgs a)
             int64_t row, col0;
             chunk_pos(t0 + j, a.grid_n, h * 256 + tid, row, col0);
             store_chunk<2, VEC, NT>(a.out, a.rows, a.K, row, col0, ov);
+            if constexpr (SUMS) {
+                if (row < a.rows && col0 < a.K) grad_sums_add(cs[j], mx, ov);
+            }
         }
+    }
+    if constexpr (SUMS) {
+        static_assert(VEC, "the sums take whole chunks");
+        __syncthreads();                    // the staged values are done with
+        float* lds = WIDEN ? reinterpret_cast<float*>(s_rv) : reinterpret_cast<float*>(s_vals);
+        static_assert((WIDEN ? sizeof(s_rv) : sizeof(s_vals)) >= (size_t)U * 8192, "room for the sums");
+        write_grad_sums<U>(cs, mx, lds, t0, ntiles, a.grid_n, a.K, a.col_part, a.wg_max, tid);
     }
 }
 
 // ===========================================================================
 // ReLU mask gradient (in place)
 // ===========================================================================
-// NT: nontemporal gradient loads / stores.
-template <bool VEC, int U, bool NT>
+// NT: nontemporal gradient loads / stores.  SUMS: also the column sums and
+// the amax of the masked gradient, whose kept chunks are then read too.
+template <bool VEC, int U, bool NT, bool SUMS = false>
 __global__ __launch_bounds__(kThreads) void relu_grad_kernel(uint8_t* grad, int64_t M, int64_t N,
                                                              uint32_t grid_n, uint32_t T,
-                                                             const uint8_t* bitmask)
+                                                             const uint8_t* bitmask, float* col_part = nullptr,
+                                                             uint32_t* wg_max = nullptr)
 {
     const int tid = threadIdx.x;
     const uint32_t t0 = blockIdx.x * U;
@@ -1711,26 +1841,32 @@ __global__ __launch_bounds__(kThreads) void relu_grad_kernel(uint8_t* grad, int6
     for (int j = 0; j < U; j++)
 #pragma unroll
         for (int h = 0; h < 2; h++)
-            m[j][h] = j < ntiles ? bitmask[(size_t)(t0 + j) * kTileBytes + h * 256 + tid] : 0xffu;
+            m[j][h] = j < ntiles ? bitmask[(size_t)(t0 + j) * kTileBytes + h * 256 + tid] : (SUMS ? 0u : 0xffu);
     uint4 g[U][2];
 #pragma unroll
     for (int j = 0; j < U; j++)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             g[j][h] = uint4{0u, 0u, 0u, 0u};
-            if (m[j][h] != 0u && m[j][h] != 0xffu) {
+            if (m[j][h] != 0u && (SUMS || m[j][h] != 0xffu)) {
                 int64_t row, col0;
                 chunk_pos(t0 + j, grid_n, h * 256 + tid, row, col0);
                 g[j][h] = load_chunk<2, VEC, NT>(grad, M, N, row, col0);
             }
         }
+    float cs[SUMS ? U : 1][8] = {};
+    uint32_t mx = 0;
 #pragma unroll
     for (int j = 0; j < U; j++)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const uint32_t mm = m[j][h];
-            if (mm == 0xffu) continue;    // all kept: nothing to write
             uint4 v = g[j][h];
+            if (mm == 0xffu) {            // all kept: nothing to write
+                if constexpr (SUMS) grad_sums_add(cs[j], mx, v);
+                continue;
+            }
+            if (SUMS && j >= ntiles) continue;
             // byte mask -> 16-bit lane masks (all-zero byte stores zeros)
             uint32_t k0 = ((mm & 1u) ? 0xffffu : 0u) | ((mm & 2u) ? 0xffff0000u : 0u);
             uint32_t k1 = ((mm & 4u) ? 0xffffu : 0u) | ((mm & 8u) ? 0xffff0000u : 0u);
@@ -1740,7 +1876,14 @@ __global__ __launch_bounds__(kThreads) void relu_grad_kernel(uint8_t* grad, int6
             int64_t row, col0;
             chunk_pos(t0 + j, grid_n, h * 256 + tid, row, col0);
             store_chunk<2, VEC, NT>(grad, M, N, row, col0, v);
+            // (bits past the matrix are clear, so such a chunk adds nothing)
+            if constexpr (SUMS) grad_sums_add(cs[j], mx, v);
         }
+    if constexpr (SUMS) {
+        static_assert(VEC, "the sums take whole chunks");
+        __shared__ __align__(16) float lds[U * 32 * 64];
+        write_grad_sums<U>(cs, mx, lds, t0, ntiles, grid_n, N, col_part, wg_max, tid);
+    }
 }
 
 // Empty input (T = 0): prefix = [0]; the cursor outputs take the input
@@ -1784,49 +1927,48 @@ constexpr int kStreamU = BS_STREAM_U;
 // 32-bit byte offset below 8 rows of N elements of `eb` bytes.
 static bool vec_rows_fit(int64_t N, int eb) { return 8 * N * (int64_t)eb < (int64_t(1) << 32); }
 
-template <int IN_T, bool QUANT, int MODE, bool PACKED>
-static hipError_t launch_compress_mode(const CompressArgs& a, bool vec, bool nt, hipStream_t st, bool rsq = false)
+template <int IN_T, bool QUANT, int MODE, bool PACKED, int WB>
+static hipError_t launch_compress_wb(const CompressArgs& a, bool vec, bool nt, hipStream_t st)
 {
-    const uint32_t units = (a.tend - a.tile0 + kStreamU - 1) / kStreamU;
+    const dim3 units((a.tend - a.tile0 + kStreamU - 1) / kStreamU), threads(64 * kStreamU);
     // the streaming hint is built for the fused pass over a vector-loadable input
     constexpr bool kHasNt = MODE == MODE_FUSED;
-    if constexpr (IN_T == DT_BF16 && MODE == MODE_FUSED && !PACKED) {
-        if (rsq) {
-            if (vec && nt)
-                launch_timed(0, compress_stream_kernel<IN_T, QUANT, true, MODE, kStreamU, PACKED, true, true>,
-                             dim3(units), dim3(64 * kStreamU), 0, st, a);
-            else if (vec)
-                launch_timed(0, compress_stream_kernel<IN_T, QUANT, true, MODE, kStreamU, PACKED, false, true>,
-                             dim3(units), dim3(64 * kStreamU), 0, st, a);
-            else
-                launch_timed(0, compress_stream_kernel<IN_T, QUANT, false, MODE, kStreamU, PACKED, false, true>,
-                             dim3(units), dim3(64 * kStreamU), 0, st, a);
-            return hipGetLastError();
-        }
-    }
     if (vec && nt && kHasNt)
-        launch_timed(0, compress_stream_kernel<IN_T, QUANT, true, MODE, kStreamU, PACKED, kHasNt>, dim3(units),
-                     dim3(64 * kStreamU), 0, st, a);
+        launch_timed(0, compress_stream_kernel<IN_T, QUANT, true, MODE, kStreamU, PACKED, kHasNt, WB>, units, threads,
+                     0, st, a);
     else if (vec)
-        launch_timed(0, compress_stream_kernel<IN_T, QUANT, true, MODE, kStreamU, PACKED, false>, dim3(units),
-                     dim3(64 * kStreamU), 0, st, a);
-    else
-        launch_timed(0, compress_stream_kernel<IN_T, QUANT, false, MODE, kStreamU, PACKED, false>, dim3(units),
-                     dim3(64 * kStreamU), 0, st, a);
+        launch_timed(0, compress_stream_kernel<IN_T, QUANT, true, MODE, kStreamU, PACKED, false, WB>, units, threads, 0,
+                     st, a);
+    else if constexpr (WB == WB_RELU || WB == WB_SQUARE)      // (the activation step's host side asks for vec)
+        launch_timed(0, compress_stream_kernel<IN_T, QUANT, false, MODE, kStreamU, PACKED, false, WB>, units, threads,
+                     0, st, a);
     return hipGetLastError();
+}
+
+template <int IN_T, bool QUANT, int MODE, bool PACKED>
+static hipError_t launch_compress_mode(const CompressArgs& a, bool vec, bool nt, hipStream_t st, int wb)
+{
+    if constexpr (IN_T == DT_BF16 && MODE == MODE_FUSED) {
+        if constexpr (!PACKED) {
+            if (wb == WB_SQUARE) return launch_compress_wb<IN_T, QUANT, MODE, PACKED, WB_SQUARE>(a, vec, nt, st);
+        }
+        if (wb == WB_ACT) return launch_compress_wb<IN_T, QUANT, MODE, PACKED, WB_ACT>(a, vec, nt, st);
+        if (wb == WB_ACT_SQUARE) return launch_compress_wb<IN_T, QUANT, MODE, PACKED, WB_ACT_SQUARE>(a, vec, nt, st);
+    }
+    return launch_compress_wb<IN_T, QUANT, MODE, PACKED, WB_RELU>(a, vec, nt, st);
 }
 
 template <int MODE, bool PACKED = false>
 static hipError_t launch_compress(const CompressArgs& a, int in_dtype, bool quant, bool vec, bool nt,
-                                  hipStream_t st, bool rsq = false)
+                                  hipStream_t st, int wb = WB_RELU)
 {
     if constexpr (MODE != MODE_VALS) {
-        if (quant) return launch_compress_mode<DT_BF16, true, MODE, PACKED>(a, vec, nt, st, rsq);
+        if (quant) return launch_compress_mode<DT_BF16, true, MODE, PACKED>(a, vec, nt, st, wb);
     }
     switch (in_dtype) {
-    case DT_BF16: return launch_compress_mode<DT_BF16, false, MODE, PACKED>(a, vec, nt, st, rsq);
-    case DT_E4M3FN: return launch_compress_mode<DT_E4M3FN, false, MODE, PACKED>(a, vec, nt, st);
-    default: return launch_compress_mode<DT_E5M2, false, MODE, PACKED>(a, vec, nt, st);
+    case DT_BF16: return launch_compress_mode<DT_BF16, false, MODE, PACKED>(a, vec, nt, st, wb);
+    case DT_E4M3FN: return launch_compress_mode<DT_E4M3FN, false, MODE, PACKED>(a, vec, nt, st, wb);
+    default: return launch_compress_mode<DT_E5M2, false, MODE, PACKED>(a, vec, nt, st, wb);
     }
 }
 
@@ -1880,15 +2022,17 @@ static int compress_impl(const void* dense, int in_dtype, int64_t M, int64_t N, 
                          int32_t* err_flags, void* workspace, int64_t workspace_bytes,
                          uint32_t epoch, void* stream, bool relu, void* relu_out, bool packed = false,
                          bool check_capture = true, const std::function<int()>& before_launch = nullptr,
-                         bool relu_sq = false, float relu_k = 1.0f)
+                         int wb = WB_RELU, float relu_k = 1.0f, const void* bias = nullptr,
+                         float* h_scale_out = nullptr)
 {
-    if (relu_sq) {
+    if (wb == WB_SQUARE) {
         // the ReLU^2 write-back: bf16 pre-activation, values into a buffer
         if (!relu || relu_out == nullptr || in_dtype != DT_BF16 || packed || !write_vals)
             return set_error(BS_ERR_INVALID, "bs_compress_relu2: needs a bf16 pre-activation, relu_out and "
                                              "write_vals = 1");
-        if (!std::isfinite(relu_k)) return set_error(BS_ERR_INVALID, "bs_compress_relu2: k must be finite");
     }
+    if (wb != WB_RELU && !std::isfinite(relu_k))
+        return set_error(BS_ERR_INVALID, "bs_compress_relu2: k must be finite");
     if (packed) {
         // vals is the packed stream and vals_capacity its size in bytes
         if (!write_vals) return set_error(BS_ERR_INVALID, "bs_compress_packed: write_vals must be 1");
@@ -1968,6 +2112,8 @@ static int compress_impl(const void* dense, int in_dtype, int64_t M, int64_t N, 
     a.relu = relu ? 1 : 0;
     a.relu_out = (uint8_t*)relu_out;
     a.relu_k = relu_k;
+    a.bias = (const uint16_t*)bias;
+    a.h_scale_out = h_scale_out;
     a.status = reinterpret_cast<uint64_t*>((uint8_t*)workspace + kWsHeaderBytes);
     a.epoch = epoch;
     a.err = err_flags;
@@ -1982,8 +2128,8 @@ static int compress_impl(const void* dense, int in_dtype, int64_t M, int64_t N, 
     if (quantize) {
         // the code table of this call's scale, built after the amax it reads
         uint8_t* qtab = (uint8_t*)workspace + ws_qtab_offset(T);
-        hipLaunchKernelGGL(qtab_build_kernel, dim3((kQtabEntries + 255) / 256), dim3(256), 0, st, amax_slot, amax_epoch,
-                           qtab);
+        hipLaunchKernelGGL(qtab_build_kernel, dim3(kQtabBlocks * (wb == WB_ACT_SQUARE ? 2 : 1)), dim3(256), 0, st,
+                           amax_slot, amax_epoch, qtab, relu_k);
         a.qtab = qtab;
     }
     const int inb = in_dtype == DT_BF16 ? 2 : 1;
@@ -1991,8 +2137,8 @@ static int compress_impl(const void* dense, int in_dtype, int64_t M, int64_t N, 
                (dense_q_out == nullptr || aligned8(dense_q_out)) &&
                (relu_out == nullptr || ((uintptr_t)relu_out) % (8 * inb) == 0);
     const bool nt = use_nontemporal(M * N * inb);
-    hipError_t e = packed     ? launch_compress<MODE_FUSED, true>(a, in_dtype, quantize != 0, vec, nt, st)
-                 : write_vals ? launch_compress<MODE_FUSED>(a, in_dtype, quantize != 0, vec, nt, st, relu_sq)
+    hipError_t e = packed     ? launch_compress<MODE_FUSED, true>(a, in_dtype, quantize != 0, vec, nt, st, wb)
+                 : write_vals ? launch_compress<MODE_FUSED>(a, in_dtype, quantize != 0, vec, nt, st, wb)
                               : launch_compress<MODE_COUNT>(a, in_dtype, quantize != 0, vec, nt, st);
     if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_compress launch: %s", hipGetErrorString(e));
     return BS_OK;
@@ -2039,7 +2185,42 @@ extern "C" int bs_compress_relu2(const void* preact, int quantize, int64_t M, in
     return compress_impl(preact, DT_BF16, M, N, quantize, amax_slot, amax_epoch, scale_out, dense_q_out,
                          bitmask, prefix, vals, vals_capacity, vals_offset_in, 0, vals_offset_out, nullptr, 1,
                          err_flags, workspace, workspace_bytes, epoch, stream, true, relu_out, false, true, nullptr,
-                         true, k);
+                         WB_SQUARE, k);
+}
+
+extern "C" int64_t bs_compress_act_workspace_bytes(int64_t M, int64_t N)
+{
+    const int64_t w = bs_compress_workspace_bytes(M, N);
+    return w < 0 ? w : w + kQtabBytes;      // the code table of h behind that of r
+}
+
+extern "C" int bs_compress_act(const void* preact, const void* bias, int64_t M, int64_t N, int square, float k,
+                               int quantize, const uint64_t* amax_slot, uint32_t amax_epoch, float* scale_out,
+                               void* codes_out, float* codes_scale_out, void* h_out, uint8_t* bitmask,
+                               uint32_t* prefix, void* vals, int64_t vals_capacity, int packed,
+                               const int64_t* vals_offset_in, int64_t* vals_offset_out, int64_t* vals_start_out,
+                               int32_t* err_flags, void* workspace, int64_t workspace_bytes, uint32_t epoch,
+                               void* stream)
+{
+    clear_error();
+    if (M <= 0 || N <= 0) return set_error(BS_ERR_INVALID, "bs_compress_act: empty input");
+    if (N % 8 != 0 || !aligned16(preact) || !vec_rows_fit(N, 2))
+        return set_error(BS_ERR_INVALID, "bs_compress_act: needs N %% 8 == 0, N < 2^28 and a 16-byte aligned input");
+    if (bias != nullptr && !aligned16(bias)) return set_error(BS_ERR_INVALID, "bs_compress_act: bias misaligned");
+    if (h_out != nullptr && !aligned16(h_out)) return set_error(BS_ERR_INVALID, "bs_compress_act: h_out misaligned");
+    if (quantize ? (codes_out == nullptr || !aligned8(codes_out) || h_out != nullptr) : h_out == nullptr)
+        return set_error(BS_ERR_INVALID, "bs_compress_act: quantize writes codes_out (8-byte aligned) and no h_out, "
+                                         "else h_out is written");
+    if (quantize && amax_slot == nullptr) return set_error(BS_ERR_INVALID, "bs_compress_act: null amax slot");
+    if ((uint64_t)M * (uint64_t)N >= kMaxElemsUntested)
+        return set_error(BS_ERR_INVALID, "bs_compress_act: M*N must be < 2^31");
+    if (workspace_bytes < bs_compress_act_workspace_bytes(M, N))
+        return set_error(BS_ERR_INVALID, "bs_compress_act: workspace too small");
+    const int wb = square ? WB_ACT_SQUARE : WB_ACT;
+    return compress_impl(preact, DT_BF16, M, N, quantize, amax_slot, amax_epoch, scale_out, codes_out, bitmask, prefix,
+                         vals, vals_capacity, vals_offset_in, packed, vals_offset_out, vals_start_out, 1, err_flags,
+                         workspace, workspace_bytes, epoch, stream, true, h_out, packed != 0, true, nullptr, wb,
+                         square ? k : 1.0f, bias, codes_scale_out);
 }
 
 extern "C" int bs_compress_packed(const void* dense, int in_dtype, int64_t M, int64_t N, int quantize,
@@ -2378,6 +2559,92 @@ extern "C" int bs_relu2_grad_packed(void* grad, int64_t M, int64_t N, const void
 {
     return relu2_grad_impl(grad, M, N, stream_bytes, vals_dtype, stream_nbytes, bitmask, prefix, vals_offset,
                            relu2_scale, scale, stream, true);
+}
+
+// The gradient kernels with their sums.  workspace: [tile rows, N] fp32
+// column sums, then a magnitude per workgroup (2 tiles each).
+static int64_t grad_wgs(int64_t M, int64_t N) { return (((M + 63) / 64) * ((N + 63) / 64) + kGatherU - 1) / kGatherU; }
+
+extern "C" int64_t bs_grad_sums_workspace_bytes(int64_t M, int64_t N)
+{
+    if (M <= 0 || N <= 0) return 0;
+    return ((M + 63) / 64) * N * 4 + grad_wgs(M, N) * 4;
+}
+
+template <int V_T, bool SC, bool PK>
+static void launch_relu2_sums_t(const GatherArgs& a, uint32_t blocks, bool nt, hipStream_t st)
+{
+    if (nt)
+        hipLaunchKernelGGL((relu2_grad_kernel<V_T, SC, true, kGatherU, PK, true, true>), dim3(blocks), dim3(kThreads), 0,
+                           st, a);
+    else
+        hipLaunchKernelGGL((relu2_grad_kernel<V_T, SC, true, kGatherU, PK, false, true>), dim3(blocks), dim3(kThreads), 0,
+                           st, a);
+}
+
+extern "C" int bs_act_grad_sums(void* grad, int64_t M, int64_t N, int square, const void* vals, int vals_dtype,
+                                int64_t vals_numel, int packed, const uint8_t* bitmask, const uint32_t* prefix,
+                                const int64_t* vals_offset, float relu2_scale, const float* scale, void* bias_grad,
+                                void* amax_workspace, uint32_t amax_epoch, void* workspace, int64_t workspace_bytes,
+                                void* stream)
+{
+    clear_error();
+    const char* fn = "bs_act_grad_sums";
+    if (M <= 0 || N <= 0) return set_error(BS_ERR_INVALID, "%s: empty gradient", fn);
+    if (grad == nullptr || bitmask == nullptr) return set_error(BS_ERR_INVALID, "%s: null pointer", fn);
+    if (square) {
+        if (int rc = check_gather(vals, vals_dtype, vals_numel, bitmask, prefix, fn, packed != 0)) return rc;
+    }
+    if (N % 8 != 0 || !aligned16(grad))
+        return set_error(BS_ERR_INVALID, "%s: needs N %% 8 == 0 and a 16-byte aligned gradient", fn);
+    if ((uint64_t)M * (uint64_t)N >= kMaxElemsUntested) return set_error(BS_ERR_INVALID, "%s: M*N must be < 2^31", fn);
+    if (workspace == nullptr || (((uintptr_t)workspace) & 3u) || workspace_bytes < bs_grad_sums_workspace_bytes(M, N))
+        return set_error(BS_ERR_INVALID, "%s: workspace too small or misaligned", fn);
+    hipStream_t st = (hipStream_t)stream;
+    uint64_t* slot = nullptr;
+    if (amax_workspace != nullptr) {
+        if (amax_epoch == 0 || amax_epoch >= (1u << 30)) return set_error(BS_ERR_INVALID, "%s: epoch out of range", fn);
+        if (int rc = refuse_capture(st, fn)) return rc;
+        slot = reinterpret_cast<uint64_t*>((uint8_t*)amax_workspace + kWsAmaxOffset);
+    }
+    const int64_t grid_m = (M + 63) / 64, wgs = grad_wgs(M, N);
+    GatherArgs a{};
+    a.vals = (const uint8_t*)vals;
+    a.vals_numel = vals_numel;
+    a.bitmask = bitmask;
+    a.prefix = prefix;
+    a.vals_offset = vals_offset;
+    a.out = (uint8_t*)grad;
+    a.grid_n = (uint32_t)((N + 63) / 64);
+    a.K = N;
+    a.rows = M;
+    a.num_tiles = (uint32_t)(grid_m * a.grid_n);
+    a.relu2_scale = relu2_scale;
+    a.scale = scale;
+    a.col_part = bias_grad ? (float*)workspace : nullptr;
+    a.wg_max = slot ? (uint32_t*)workspace + grid_m * N : nullptr;
+    const bool nt = use_nontemporal(2 * M * N);
+    if (!square) {
+        if (nt)
+            hipLaunchKernelGGL((relu_grad_kernel<true, kGatherU, true, true>), dim3((uint32_t)wgs), dim3(kThreads), 0, st,
+                               a.out, M, N, a.grid_n, a.num_tiles, bitmask, a.col_part, a.wg_max);
+        else
+            hipLaunchKernelGGL((relu_grad_kernel<true, kGatherU, false, true>), dim3((uint32_t)wgs), dim3(kThreads), 0,
+                               st, a.out, M, N, a.grid_n, a.num_tiles, bitmask, a.col_part, a.wg_max);
+    } else {
+#define BS_R2S(V_T, SC)                                                                    \
+    do {                                                                                   \
+        if (packed) launch_relu2_sums_t<V_T, SC, true>(a, (uint32_t)wgs, nt, st);          \
+        else launch_relu2_sums_t<V_T, SC, false>(a, (uint32_t)wgs, nt, st);                \
+    } while (0)
+        if (vals_dtype == DT_BF16 && scale == nullptr) BS_R2S(DT_BF16, false);
+        else if (vals_dtype == DT_E4M3FN && scale != nullptr) BS_R2S(DT_E4M3FN, true);
+        else return set_error(BS_ERR_INVALID, "%s: bf16 values without a scale, or e4m3fn values with one", fn);
+#undef BS_R2S
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(BS_ERR_HIP, "%s launch: %s", fn, hipGetErrorString(e));
+    return sums_finish_launch(a.col_part, grid_m, N, bias_grad, a.wg_max, wgs, slot, amax_epoch, st);
 }
 
 extern "C" int bs_pack_bits(const void* raw, int vals_dtype, const uint32_t* count_ptr, int64_t count_max,

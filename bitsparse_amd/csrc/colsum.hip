@@ -64,13 +64,31 @@ __global__ __launch_bounds__(kSumThreads) void col_sum_part_kernel(const uint16_
     }
 }
 
-// out[c] = bf16(sum over rows p < S of part[p, c]): 64 columns per workgroup,
-// the four waves taking every fourth partial row.
-__global__ __launch_bounds__(kSumThreads) void col_sum_finish_kernel(const float* part, int64_t S, int64_t C,
-                                                                     uint16_t* out)
+// Workgroups below col_blocks: out[c] = bf16(sum over rows p < S of part[p, c]),
+// 64 columns each, the four waves taking every fourth partial row.  The
+// others: the largest of `maxima` (bf16 magnitude bits) into the amax slot.
+constexpr int kMaxBlocks = 16;
+__global__ __launch_bounds__(kSumThreads) void sums_finish_kernel(const float* part, int64_t S, int64_t C,
+                                                                  uint16_t* out, uint32_t col_blocks,
+                                                                  const uint32_t* maxima, int64_t nmax,
+                                                                  uint64_t* slot, uint32_t epoch)
 {
     __shared__ float s_acc[4][64];
+    __shared__ uint32_t s_mx[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (blockIdx.x >= col_blocks) {
+        const int64_t stride = (int64_t)(gridDim.x - col_blocks) * kSumThreads;
+        uint32_t m = 0;
+        for (int64_t i = (int64_t)(blockIdx.x - col_blocks) * kSumThreads + threadIdx.x; i < nmax; i += stride)
+            m = max(m, maxima[i]);
+        m = wave_max_u32(m);
+        if (lane == 0) s_mx[wave] = m;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            atomicMax((unsigned long long*)slot, (unsigned long long)(((uint64_t)epoch << 32) |
+                                                                      max(max(s_mx[0], s_mx[1]), max(s_mx[2], s_mx[3]))));
+        return;
+    }
     const int64_t c = (int64_t)blockIdx.x * 64 + lane;
     float t = 0.f;
     if (c < C)
@@ -88,6 +106,18 @@ static int64_t col_sum_splits(int64_t R, int64_t C)
 {
     const int64_t groups = (C + kSumCols - 1) / kSumCols;
     return std::max<int64_t>(1, std::min<int64_t>((2048 + groups - 1) / groups, R / 64));
+}
+
+int sums_finish_launch(const float* part, int64_t S, int64_t C, void* out, const uint32_t* maxima, int64_t nmax,
+                       uint64_t* slot, uint32_t epoch, hipStream_t stream)
+{
+    const uint32_t cb = part ? (uint32_t)((C + 63) / 64) : 0u;
+    const uint32_t mb = maxima ? (uint32_t)std::min<int64_t>((nmax + 1023) / 1024, kMaxBlocks) : 0u;
+    if (cb + mb == 0) return BS_OK;
+    hipLaunchKernelGGL(sums_finish_kernel, dim3(cb + mb), dim3(kSumThreads), 0, stream, part, S, C, (uint16_t*)out, cb,
+                       maxima, nmax, slot, epoch);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? BS_OK : set_error(BS_ERR_HIP, "sums_finish launch: %s", hipGetErrorString(e));
 }
 
 }  // namespace bs
@@ -120,9 +150,7 @@ extern "C" int bs_col_sum(const void* x, int64_t R, int64_t C, void* out, void* 
     hipStream_t st = (hipStream_t)stream;
     auto kernel = use_nontemporal(2 * R * C) ? col_sum_part_kernel<true> : col_sum_part_kernel<false>;
     hipLaunchKernelGGL(kernel, grid, dim3(kSumThreads), 0, st, (const uint16_t*)x, R, C, rows_per, (float*)workspace);
-    hipLaunchKernelGGL(col_sum_finish_kernel, dim3((uint32_t)((C + 63) / 64)), dim3(kSumThreads), 0, st,
-                       (const float*)workspace, S, C, (uint16_t*)out);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_col_sum launch: %s", hipGetErrorString(e));
-    return BS_OK;
+    return sums_finish_launch((const float*)workspace, S, C, out, nullptr, 0, nullptr, 0, st);
 }

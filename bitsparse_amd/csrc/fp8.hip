@@ -5,6 +5,7 @@
 // with one correctly rounded fp32 division per value: the quantize pass reads
 // each code from a table of the scale's 24-exponent window (quant_chunk_tab),
 // which every workgroup builds in LDS from exact divisions.
+#include <algorithm>
 #include <cmath>
 
 #include "bs_device.h"
@@ -67,6 +68,52 @@ __global__ __launch_bounds__(kFp8Threads) void amax_bf16_kernel(const uint16_t* 
     }
     for (int64_t j = nvec * 8 + (int64_t)blockIdx.x * kFp8Threads + tid; j < n; j += stride)
         m = max(m, mag_bits<RELU>((uint32_t)x[j]));
+    m = wave_max_u32(m);
+    if ((tid & 63) == 0) s_w[tid >> 6] = m;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < kFp8Threads / 64; w++) m = max(m, s_w[w]);
+        atomicMax((unsigned long long*)slot, (unsigned long long)(((uint64_t)epoch << 32) | m));
+    }
+}
+
+// amax of relu(bf16(x + bias)) of a [rows, 8 nc] matrix: the amax of an MLP
+// block's activation straight from the up-projection's product, so that the
+// biased pre-activation is never written (the add is repeated by the compress).
+// A thread keeps one column chunk (its stride is a whole number of rows).
+template <bool NT>
+__global__ __launch_bounds__(kFp8Threads) void amax_bias_relu_kernel(const uint16_t* x, int64_t rows, uint32_t nc,
+                                                                     const uint16_t* bias, uint64_t* slot,
+                                                                     uint32_t epoch)
+{
+    __shared__ uint32_t s_w[kFp8Threads / 64];
+    const int tid = threadIdx.x;
+    const int64_t t = (int64_t)blockIdx.x * kFp8Threads + tid;
+    const int64_t rstep = (int64_t)gridDim.x * kFp8Threads / nc;      // rows per pass (>= 1: host)
+    const int64_t r0 = t / nc, c = t - r0 * nc;
+    const uint4* xv = reinterpret_cast<const uint4*>(x) + c;
+    uint32_t m = 0;
+    if (r0 < rstep) {
+        const uint4 b = reinterpret_cast<const uint4*>(bias)[c];
+        const uint32_t bw[4] = {b.x, b.y, b.z, b.w};
+        auto take = [&](const uint4 v) __attribute__((always_inline)) {
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint32_t s = add_bf16x2(w[k], bw[k]);
+                m = max(m, max(mag_bits<true>(s & 0xffffu), mag_bits<true>(s >> 16)));
+            }
+        };
+        int64_t r = r0;
+        for (; r + (kAmaxUnroll - 1) * rstep < rows; r += kAmaxUnroll * rstep) {
+            uint4 v[kAmaxUnroll];
+#pragma unroll
+            for (int u = 0; u < kAmaxUnroll; u++) v[u] = ld16<NT>(xv + (r + u * rstep) * nc);
+#pragma unroll
+            for (int u = 0; u < kAmaxUnroll; u++) take(v[u]);
+        }
+        for (; r < rows; r += rstep) take(ld16<NT>(xv + r * nc));
+    }
     m = wave_max_u32(m);
     if ((tid & 63) == 0) s_w[tid >> 6] = m;
     __syncthreads();
@@ -394,6 +441,38 @@ extern "C" int bs_amax_relu(const void* preact, int64_t n, void* workspace, int6
 {
     clear_error();
     return amax_launch(preact, n, workspace, workspace_bytes, epoch, stream, true, true);
+}
+
+extern "C" int bs_amax_bias_relu(const void* x, int64_t M, int64_t N, const void* bias, void* workspace,
+                                 int64_t workspace_bytes, uint32_t epoch, void* stream)
+{
+    clear_error();
+    if (M <= 0 || N <= 0) return set_error(BS_ERR_INVALID, "bs_amax_bias_relu: empty input");
+    if (workspace == nullptr || workspace_bytes < kWsHeaderBytes)
+        return set_error(BS_ERR_INVALID, "bs_amax_bias_relu: workspace too small");
+    if (epoch == 0 || epoch >= (1u << 30)) return set_error(BS_ERR_INVALID, "bs_amax_bias_relu: epoch out of range");
+    if (x == nullptr || bias == nullptr) return set_error(BS_ERR_INVALID, "bs_amax_bias_relu: null pointer");
+    if (N % 8 != 0 || (((uintptr_t)x) & 15u) || (((uintptr_t)bias) & 15u))
+        return set_error(BS_ERR_INVALID, "bs_amax_bias_relu: needs N %% 8 == 0 and 16-byte aligned operands");
+    if ((uint64_t)M * (uint64_t)N >= kMaxElemsUntested)
+        return set_error(BS_ERR_INVALID, "bs_amax_bias_relu: M*N must be < 2^31");
+    if (int rc = refuse_capture((hipStream_t)stream, "bs_amax_bias_relu")) return rc;
+    uint64_t* slot = reinterpret_cast<uint64_t*>((uint8_t*)workspace + kWsAmaxOffset);
+    int dev = 0, cus = 0;
+    if (stream_device((hipStream_t)stream, &dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    // two workgroups per CU (few atomics meet on the slot), and at least one
+    // row of chunks per pass
+    const int64_t nc = N / 8;
+    const int64_t grid = std::max<int64_t>(std::min<int64_t>(grid_for(M * N), 2 * cus),
+                                           (nc + kFp8Threads - 1) / kFp8Threads);
+    auto kernel = use_nontemporal(2 * M * N) ? amax_bias_relu_kernel<true> : amax_bias_relu_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kFp8Threads), 0, (hipStream_t)stream, (const uint16_t*)x, M,
+                       (uint32_t)nc, (const uint16_t*)bias, slot, epoch);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_amax_bias_relu launch: %s", hipGetErrorString(e));
+    return BS_OK;
 }
 
 extern "C" int bs_quantize_e4m3fn(const void* x, int64_t n, void* q_out, float* scale_out,

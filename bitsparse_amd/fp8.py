@@ -141,12 +141,11 @@ class MatmulFp8(Function):
         return grad_a, grad_b, None, None
 
 
-def linear_fp8_backward(x: Tensor, W: Tensor, grad_z: Tensor, need_x: bool,
+def linear_fp8_backward(x: Tensor, W: Tensor, g: Fp8Operand | None, need_x: bool,
                         need_W: bool) -> tuple[Tensor | None, Tensor | None]:
-    """(grad of x, grad of W) of z = matmul(x, W.T, True) for bf16 x and W:
-    ``MatmulFp8``'s backward with its operands quantized again, W's gradient
-    in W's own layout."""
-    g = Fp8Operand(*to_fp8(grad_z))
+    """(grad of x, grad of W) of z = matmul(x, W.T, True) for bf16 x and W
+    and z's gradient g in fp8: ``MatmulFp8``'s backward with its operands
+    quantized again, W's gradient in W's own layout."""
     grad_x = grad_W = None
     if need_x:
         w = as_fp8_operand(W, None)

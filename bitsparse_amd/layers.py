@@ -18,11 +18,11 @@ from . import config
 from .bitsparse import BitsparseTensor, TensorBuffer
 from .config import RELU2_SCALE
 from .fp8 import Fp8Operand, as_fp8_operand, fp8_gemm, is_fp8, linear_fp8_backward, matmul, to_fp8
-from .src.functions import (fused_linear_relu_ok, linear_relu_and_compress, relu2_and_compress,
-                            relu2_fused_ok, relu2_quantize_and_compress, relu_and_compress,
+from .src.functions import (activate_and_compress, activate_ok, fused_linear_relu_ok, linear_relu_and_compress,
+                            relu2_and_compress, relu2_fused_ok, relu2_quantize_and_compress, relu_and_compress,
                             relu_quantize_and_compress)
-from .src.hip_operators import (col_sum, col_sum_supported, mask_with_bitmask_, quantize_e4m3fn,
-                                relu2_grad_sparse_, relu2_square_amax_)
+from .src.hip_operators import (act_grad_sums_, act_grad_sums_supported, col_sum, col_sum_supported,
+                                mask_with_bitmask_, quantize_e4m3fn, relu2_grad_sparse_, relu2_square_amax_)
 from .src.sparse_matmul import AspB, AspRelu2B
 
 # FFNRelu / FFNRelu2 with bf16 storage into a TensorBuffer run the up-projection
@@ -249,10 +249,15 @@ class _FFNBlock(Function):
             z = fp8_gemm(as_fp8_operand(x, None), as_fp8_operand(W1.T, None), torch.bfloat16)
         else:
             z = x @ W1.T
-        if b1 is not None:
-            z = z + b1
-        down = Relu2Linear if square else ReluLinear
-        y, ctx.h_sparse = down.activate_and_project(z, W2, sparse_data, pack_sbit, dtype)
+        if activate_ok(z, b1, sparse_data, RELU2_SCALE):
+            h, scale, ctx.h_sparse = activate_and_compress(z, b1, sparse_data, pack_sbit, fp8, square)
+            y = (fp8_gemm(Fp8Operand(h, scale), as_fp8_operand(W2.T, None), torch.bfloat16) if fp8
+                 else h @ W2.T)
+        else:
+            if b1 is not None:
+                z = z + b1
+            down = Relu2Linear if square else ReluLinear
+            y, ctx.h_sparse = down.activate_and_project(z, W2, sparse_data, pack_sbit, dtype)
         return y if b2 is None else y + b2
 
     @staticmethod
@@ -276,11 +281,21 @@ class _FFNBlock(Function):
                 grad_h = fp8_gemm(Fp8Operand(grad_output, scale), as_fp8_operand(W2, None), torch.bfloat16)
             else:
                 grad_h = grad_output @ W2
-            grad_z = relu2_grad_sparse_(grad_h, h) if ctx.square else mask_with_bitmask_(grad_h, h)
-            if need_b1:
-                grad_b1 = _col_sum(grad_z)
+            need_g = ctx.fp8 and (need_x or need_W1)
+            g8 = None
+            if (need_b1 or need_g) and not torch.is_grad_enabled() and act_grad_sums_supported(grad_h, h, ctx.square):
+                grad_z = grad_h
+                grad_b1, epoch = act_grad_sums_(grad_z, h, ctx.square, need_b1, need_g)
+                if need_g:
+                    g8 = Fp8Operand(*quantize_e4m3fn(grad_z, epoch))
+            else:
+                grad_z = relu2_grad_sparse_(grad_h, h) if ctx.square else mask_with_bitmask_(grad_h, h)
+                if need_b1:
+                    grad_b1 = _col_sum(grad_z)
+                if need_g:
+                    g8 = as_fp8_operand(grad_z, None)
             if ctx.fp8:
-                grad_x, grad_W1 = linear_fp8_backward(x, W1, grad_z, need_x, need_W1)
+                grad_x, grad_W1 = linear_fp8_backward(x, W1, g8, need_x, need_W1)
             else:
                 grad_x = grad_z.mm(W1) if need_x else None
                 grad_W1 = grad_z.t().mm(x) if need_W1 else None   # W1's own layout, as autograd forms it

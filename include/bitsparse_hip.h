@@ -531,6 +531,61 @@ int bs_compress_noalloc(const void* dense, int in_dtype, int64_t M, int64_t N, i
 int64_t bs_compress_noalloc_max_tiles(void);
 
 /*
+ * The activation step inside an MLP block: r = relu(bf16(preact + bias)) is
+ * compressed (bs_compress_relu, or bs_compress_packed with packed = 1) and
+ * only what the down-projection multiplies is written: r, or with square = 1
+ * h = bf16(bf16(r * r) * k), k finite.
+ *   bias       bf16 [N], 16-byte aligned; nullable: none
+ *   quantize   0: bf16 values; h_out (bf16 [M, N], 16-byte aligned, may alias
+ *              preact) receives r or h, codes_out is not used.
+ *              1: e4m3fn values with the scale of amax|r|, which the amax
+ *              slot holds under amax_epoch (bs_amax_bias_relu, or
+ *              bs_amax_relu without a bias); h_out must be null; codes_out
+ *              (uint8 [M, N], 8-byte aligned) receives the e4m3fn codes of r
+ *              (their scale is scale_out) or of h, as to_fp8 makes them, with
+ *              their scale in codes_scale_out.
+ * M, N >= 1, N % 8 == 0, preact 16-byte aligned, M * N < 2^31; workspace of
+ * bs_compress_act_workspace_bytes(M, N) bytes; the other arguments as for
+ * bs_compress (packed: the stream and its bytes, as for bs_compress_packed).
+ * Refused while `stream` is capturing.  Replaces z = z + b1; h = z.relu_();
+ * [to_fp8(h)]; dense_to_tilesparse(h); [h.square_(); h.mul_(k); to_fp8(h)] of
+ * lib_sparse/layers.py:29-39, :86-89, :107-119, :169-172.
+ */
+int64_t bs_compress_act_workspace_bytes(int64_t M, int64_t N);
+int bs_compress_act(const void* preact, const void* bias, int64_t M, int64_t N, int square, float k,
+                    int quantize, const uint64_t* amax_slot, uint32_t amax_epoch, float* scale_out,
+                    void* codes_out, float* codes_scale_out, void* h_out, uint8_t* bitmask,
+                    uint32_t* prefix, void* vals, int64_t vals_capacity, int packed,
+                    const int64_t* vals_offset_in, int64_t* vals_offset_out, int64_t* vals_start_out,
+                    int32_t* err_flags, void* workspace, int64_t workspace_bytes, uint32_t epoch,
+                    void* stream);
+
+/*
+ * amax of relu(bf16(x + bias)) of a bf16 [M, N] matrix into the amax slot of
+ * `workspace` under `epoch` (as bs_amax_relu of the biased matrix, which is
+ * not written).  M, N >= 1, N % 8 == 0, x and bias 16-byte aligned.
+ */
+int bs_amax_bias_relu(const void* x, int64_t M, int64_t N, const void* bias, void* workspace,
+                      int64_t workspace_bytes, uint32_t epoch, void* stream);
+
+/*
+ * bs_relu_grad (square = 0) or bs_relu2_grad (square = 1; raw or packed
+ * values: bf16 without a scale, e4m3fn with one) in place, with what the
+ * backward reads next taken from the gradient as it is written: bias_grad
+ * (bf16 [N], nullable) receives its column sums (fp32, rounded once), and
+ * with amax_workspace (nullable) its amax goes to that workspace's amax slot
+ * under amax_epoch (then refused while `stream` is capturing).  M, N >= 1,
+ * N % 8 == 0, grad 16-byte aligned; workspace: at least
+ * bs_grad_sums_workspace_bytes(M, N) bytes, any contents.
+ */
+int64_t bs_grad_sums_workspace_bytes(int64_t M, int64_t N);
+int bs_act_grad_sums(void* grad, int64_t M, int64_t N, int square, const void* vals, int vals_dtype,
+                     int64_t vals_numel, int packed, const uint8_t* bitmask, const uint32_t* prefix,
+                     const int64_t* vals_offset, float relu2_scale, const float* scale, void* bias_grad,
+                     void* amax_workspace, uint32_t amax_epoch, void* workspace, int64_t workspace_bytes,
+                     void* stream);
+
+/*
  * Column sums of a bf16 [R, C] matrix (row-major, contiguous, 16-byte
  * aligned, C % 8 == 0, R >= 1): out[c] = bf16(sum over r of x[r, c]), summed
  * in fp32 (partial sums of row blocks, added in order).  workspace: at least

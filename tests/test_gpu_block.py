@@ -1,0 +1,139 @@
+"""The MLP block's single node and its activation / gradient kernels against
+the separate steps they stand for, bit for bit (column sums: fp32 order)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+E4M3 = torch.float8_e4m3fn
+
+
+def _z(shape, seed, special, dev):
+    g = torch.Generator().manual_seed(seed)
+    z = torch.randn(shape, generator=g).to(torch.bfloat16)
+    b = (0.5 * torch.randn(shape[1], generator=g)).to(torch.bfloat16)
+    if special:
+        f = z.view(torch.int16).view(-1)
+        n = f.numel()
+        # -0, +Inf, -Inf, largest finite, a value whose square overflows, denormals
+        for i, v in enumerate((-32768, 0x7f80, -128, 0x7f7f, 0x5f80, 1, 0x0080)):
+            f[(i * 977 + 13) % n] = v
+    return z.to(dev), b.to(dev)
+
+
+def _same(a, b, what):
+    assert a.shape == b.shape and torch.equal(a.view(torch.uint8), b.view(torch.uint8)), what
+
+
+# one tile, short last tile rows and columns, a row of several workgroups
+@pytest.mark.parametrize("shape", [(1, 8), (64, 64), (65, 72), (80, 1416), (304, 528), (1000, 1024)])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed", "e4m3_packed"])
+@pytest.mark.parametrize("special", [False, True])
+def test_activation_step(dev, shape, bias, square, store, special):
+    from bitsparse_amd.bitsparse import TensorBuffer
+    from bitsparse_amd.fp8 import to_fp8
+    from bitsparse_amd.src import functions as F
+    fp8, pack = store.startswith("e4m3"), store.endswith("packed")
+    z, b = _z(shape, 3, special and not fp8, dev)
+    n = z.numel()
+    size = (n * (7 if fp8 else 15) + 7) // 8 + 16 if pack else n * (1 if fp8 else 2)
+    bufs = [TensorBuffer(size, device=dev, dtype=E4M3 if fp8 else torch.bfloat16, pack_sbit=pack) for _ in range(2)]
+    zz = z + b if bias else z.clone()
+    if fp8:
+        q, scale, want = F.relu_quantize_and_compress(zz, bufs[0], pack)
+        operand, oscale = (q, scale) if not square else to_fp8(zz.square().mul_(1.0))
+    else:
+        operand, want = F.relu_and_compress(zz, bufs[0], pack)
+        oscale = None
+        if square:
+            operand = operand.square().mul_(1.0)
+    assert F.activate_ok(z, b if bias else None, bufs[1], 1.0)
+    got_operand, got_scale, got = F.activate_and_compress(z, b if bias else None, bufs[1], pack, fp8, square)
+    _same(want.bitmask, got.bitmask, "bitmask")
+    _same(want.prefix, got.prefix, "prefix")
+    _same(bufs[0].vals, bufs[1].vals, "values")
+    _same(bufs[0].offset, bufs[1].offset, "cursor")
+    _same(want.vals_offset.reshape(1), got.vals_offset.reshape(1), "start")
+    _same(operand, got_operand, "operand")
+    if fp8:
+        _same(want.scale.reshape(1), got.scale.reshape(1), "stored scale")
+        _same(oscale.reshape(1), got_scale.reshape(1), "operand scale")
+
+
+def test_codes_of_an_overflowing_square(dev):
+    """r finite, k r^2 past bf16's range: the scale of h is infinite, as to_fp8 has it."""
+    from bitsparse_amd.bitsparse import TensorBuffer
+    from bitsparse_amd.fp8 import to_fp8
+    from bitsparse_amd.src import functions as F
+    z, _ = _z((70, 136), 4, False, dev)
+    z[3, 5] = 2.0e25
+    buf = TensorBuffer(z.numel(), device=dev, dtype=E4M3)
+    want, wscale = to_fp8(z.relu().square().mul_(1.0))
+    got, gscale, _ = F.activate_and_compress(z, None, buf, False, True, True)
+    _same(wscale.reshape(1), gscale.reshape(1), "scale")
+    _same(want, got, "codes")
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (64, 64), (65, 72), (80, 1416), (1000, 1024), (4100, 192)])
+@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed", "e4m3_packed"])
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("zeros", [0.0, 0.5, 1.0])
+def test_gradient_sums(dev, shape, store, square, zeros):
+    from bitsparse_amd.src import functions as F
+    from bitsparse_amd.src import hip_operators as H
+    z, _ = _z(shape, 6, False, dev)
+    z = z.abs() + 1 if zeros == 0.0 else (-z.abs() if zeros == 1.0 else z)
+    pack = store.endswith("packed")
+    if store.startswith("e4m3"):
+        sp = F.quantize_and_compress(z.relu(), None, pack)[2]
+    else:
+        sp = F.dense_to_tilesparse(z.relu(), None, None, pack)
+    g = torch.randn(shape, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to(dev)
+    want = g.clone()
+    (H.relu2_grad_sparse_ if square else H.mask_with_bitmask_)(want, sp)
+    assert H.act_grad_sums_supported(g, sp, square)
+    sums, epoch = H.act_grad_sums_(g, sp, square, True, True)
+    q, scale = H.quantize_e4m3fn(g, epoch)
+    _same(want, g, "gradient")
+    wq, wscale = H.quantize_e4m3fn(want, H.amax_into_workspace(want))
+    _same(wscale.reshape(1), scale.reshape(1), "scale")
+    _same(wq, q, "codes")
+    w64 = want.double().sum(0)
+    bound = shape[0] * 2.0 ** -24 * want.double().abs().sum(0) + 2.0 ** -8 * w64.abs() + 1e-30
+    assert ((sums.double() - w64).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed"])
+@pytest.mark.parametrize("use_buffer", [False, True])
+def test_block_equals_the_separate_nodes(dev, square, store, use_buffer, monkeypatch):
+    """y, dx, dW1, dW2 bit for bit; the bias gradients to their rounding."""
+    from bitsparse_amd import layers
+    from bitsparse_amd.bitsparse import TensorBuffer
+    g = torch.Generator().manual_seed(11)
+    T, D, Hn = 208, 144, 528
+    fp8, pack = store == "e4m3", store.endswith("packed")
+    x = torch.randn((2, T // 2, D), generator=g).to(torch.bfloat16).to(dev)
+    W1 = (0.1 * torch.randn((Hn, D), generator=g)).to(torch.bfloat16).to(dev)
+    W2 = (0.1 * torch.randn((D, Hn), generator=g)).to(torch.bfloat16).to(dev)
+    b1 = (0.1 * torch.randn(Hn, generator=g)).to(torch.bfloat16).to(dev)
+    b2 = (0.1 * torch.randn(D, generator=g)).to(torch.bfloat16).to(dev)
+    dY = torch.randn((2, T // 2, D), generator=g).to(torch.bfloat16).to(dev)
+    dt = E4M3 if fp8 else torch.bfloat16
+    layer, kw = (layers.FFNRelu2, "storage_dtype") if square else (layers.FFNRelu, "dtype")
+    outs = []
+    for block in (True, False):
+        if not block:
+            monkeypatch.setattr(layers, "_block_ok", lambda *a: False)
+        p = [t.clone().requires_grad_() for t in (x, W1, W2, b1, b2)]
+        buf = TensorBuffer(2 * T * Hn + 64, device=dev, dtype=dt, pack_sbit=pack) if use_buffer else None
+        y = layer.apply(p[0], p[1], p[2], p[3], p[4], sparse_data=buf, pack_sbit=pack, **{kw: dt})
+        y.backward(dY)
+        outs.append([y.detach()] + [t.grad for t in p])
+    for a, b, name in zip(outs[0][:4], outs[1][:4], ("y", "dx", "dW1", "dW2")):
+        _same(a, b, name)
+    for a, b, name in zip(outs[0][4:], outs[1][4:], ("db1", "db2")):
+        # two bf16 roundings of fp32 sums
+        assert ((a - b).double().abs() <= 2.0 ** -7 * b.double().abs() + 1e-2).all(), name
