@@ -91,8 +91,17 @@ __global__ __launch_bounds__(kSumThreads) void sums_finish_kernel(const float* p
     }
     const int64_t c = (int64_t)blockIdx.x * 64 + lane;
     float t = 0.f;
-    if (c < C)
-        for (int64_t p = wave; p < S; p += 4) t += part[p * C + c];
+    if (c < C) {
+        int64_t p = wave;
+        for (; p + 28 < S; p += 32) {                  // eight loads in flight
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = part[(p + 4 * u) * C + c];
+#pragma unroll
+            for (int u = 0; u < 8; u++) t += v[u];
+        }
+        for (; p < S; p += 4) t += part[p * C + c];
+    }
     s_acc[wave][lane] = t;
     __syncthreads();
     if (wave == 0 && c < C)

@@ -92,7 +92,9 @@ __global__ __launch_bounds__(kFp8Threads) void amax_bias_relu_kernel(const uint1
     const int64_t rstep = (int64_t)gridDim.x * kFp8Threads / nc;      // rows per pass (>= 1: host)
     const int64_t r0 = t / nc, c = t - r0 * nc;
     const uint4* xv = reinterpret_cast<const uint4*>(x) + c;
-    uint32_t m = 0;
+    typedef short i16x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 m2 = {0, 0};
     if (r0 < rstep) {
         const uint4 b = reinterpret_cast<const uint4*>(bias)[c];
         const uint32_t bw[4] = {b.x, b.y, b.z, b.w};
@@ -100,8 +102,12 @@ __global__ __launch_bounds__(kFp8Threads) void amax_bias_relu_kernel(const uint1
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const uint32_t s = add_bf16x2(w[k], bw[k]);
-                m = max(m, max(mag_bits<true>(s & 0xffffu), mag_bits<true>(s >> 16)));
+                // relu of a half keeps it iff its saturating int16 sum with 127 is
+                // not negative (positives, and NaNs of either sign): packed ops
+                const i16x2 s = __builtin_bit_cast(i16x2, add_bf16x2(w[k], bw[k]));
+                const i16x2 drop = __builtin_elementwise_add_sat(s, (i16x2)(short)127) >> (i16x2)(short)15;
+                const u16x2 r = __builtin_bit_cast(u16x2, s & ~drop) & (u16x2)(unsigned short)0x7fff;
+                m2 = __builtin_elementwise_max(m2, r);
             }
         };
         int64_t r = r0;
@@ -114,6 +120,7 @@ __global__ __launch_bounds__(kFp8Threads) void amax_bias_relu_kernel(const uint1
         }
         for (; r < rows; r += rstep) take(ld16<NT>(xv + r * nc));
     }
+    uint32_t m = max((uint32_t)m2.x, (uint32_t)m2.y);
     m = wave_max_u32(m);
     if ((tid & 63) == 0) s_w[tid >> 6] = m;
     __syncthreads();
@@ -266,6 +273,70 @@ __global__ __launch_bounds__(256) void transpose_u8_kernel(const uint8_t* in, in
 #pragma unroll
         for (int i = 0; i < 4; i++)
             if (orow + i < C && ocol < R) *reinterpret_cast<uint32_t*>(out + (orow + i) * ld_out + ocol) = o[i];
+    }
+}
+
+// Quantize of a [R, C] matrix straight into the transposed layout (qt [C, R],
+// row-major) that hipBLASLt's fp8 path wants of the operands of a backward
+// product, and with BOTH also row-major (q [R, C]): the codes go through LDS
+// on their way out instead of being written, read and written again by
+// transpose_u8_kernel (64 MiB each way for a 4096 x 16384 weight).  Bound by
+// its one read and its writes; tile, swizzle and 4 x 4 byte transpose are
+// transpose_u8_kernel's, the codes the quantizer's table's.  A workgroup walks
+// several tiles so that building its table (1 us) is spread over them.
+// Needs C % 8 == 0, R % 4 == 0, 16-byte aligned x, 8-byte aligned q.
+template <bool BOTH, bool NT>
+__global__ __launch_bounds__(kFp8Threads) void quantize_t_kernel(const uint16_t* x, int64_t R, int64_t C, uint8_t* q,
+                                                                 uint8_t* qt, float* scale_out, const uint64_t* slot,
+                                                                 uint32_t epoch, uint32_t tiles_c, uint32_t ntiles)
+{
+    __shared__ __align__(16) uint8_t s_tab[kQtabBytes];
+    __shared__ __align__(16) uint32_t s[kTrTile * 32];
+    const float scale = fp8_scale_from_slot(slot, epoch);
+    const int t = threadIdx.x;
+    if (blockIdx.x == 0 && t == 0) *scale_out = scale;
+    const int qoff = qtab_offset(scale);
+    const int cc = 8 * (t % 16), d0 = cc / 4;          // the thread's columns in the tile, as dword columns
+    const int rb = t % 32;                             // transposed side: input rows 4 rb .. 4 rb + 3 (swizzle rb)
+    bool built = false;
+    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const uint32_t tr = tile / tiles_c, tc = tile - tr * tiles_c;
+        const int64_t r0 = (int64_t)tr * kTrTile, c = (int64_t)tc * kTrTile + cc;
+        uint4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            // rows and columns past the matrix read an in-range chunk; nothing of it is stored
+            const int64_t r = min(r0 + t / 16 + 16 * i, R - 1);
+            v[i] = ld16<NT>(x + r * C + min(c, C - 8));
+        }
+        if (!built) {
+            qtab_build_lds(s_tab, scale, 1.0f / scale, t);
+            built = true;
+        }
+        __syncthreads();                               // the table; the last tile's reads of s
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int rr = t / 16 + 16 * i, sw = (rr >> 2) & 31;
+            const uint2 o = quant_chunk_tab(v[i], s_tab, qoff);
+            // dwords d0, d0 + 1 at d0 ^ sw, (d0 + 1) ^ sw: one aligned pair, swapped by an odd swizzle
+            *reinterpret_cast<uint2*>(&s[rr * 32 + ((d0 ^ sw) & ~1)]) = (sw & 1) ? uint2{o.y, o.x} : o;
+            if constexpr (BOTH) {
+                if (r0 + rr < R && c < C) st8<NT>(q + (r0 + rr) * C + c, o);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const int cb = t / 32 + 8 * p;             // input dword column: columns 4 cb .. 4 cb + 3
+            uint32_t a[4], o[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) a[k] = s[(4 * rb + k) * 32 + (cb ^ rb)];
+            transpose4x4_bytes(a, o);
+            const int64_t orow = (int64_t)tc * kTrTile + 4 * cb, ocol = r0 + 4 * rb;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (orow + i < C && ocol < R) *reinterpret_cast<uint32_t*>(qt + (orow + i) * R + ocol) = o[i];
+        }
     }
 }
 
@@ -492,6 +563,34 @@ extern "C" int bs_quantize_e4m3fn(const void* x, int64_t n, void* q_out, float* 
                        (const uint16_t*)x, n, (uint8_t*)q_out, scale_out, slot, epoch);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_quantize_e4m3fn launch: %s", hipGetErrorString(e));
+    return BS_OK;
+}
+
+extern "C" int bs_quantize_e4m3fn_t(const void* x, int64_t R, int64_t C, void* q_out, void* qt_out, float* scale_out,
+                                    const void* workspace, int64_t workspace_bytes, uint32_t epoch, void* stream)
+{
+    clear_error();
+    if (R <= 0 || C <= 0) return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: empty input");
+    if (workspace == nullptr || workspace_bytes < kWsHeaderBytes)
+        return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: workspace too small");
+    if (x == nullptr || qt_out == nullptr || scale_out == nullptr)
+        return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: null pointer");
+    if (C % 8 != 0 || R % 4 != 0 || (((uintptr_t)x) & 15u) || (((uintptr_t)q_out) & 7u) || (((uintptr_t)qt_out) & 3u))
+        return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: needs C %% 8 == 0, R %% 4 == 0 and aligned operands");
+    if ((uint64_t)R * (uint64_t)C >= kMaxElemsUntested)
+        return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: R*C must be < 2^31");
+    const uint64_t* slot = reinterpret_cast<const uint64_t*>((const uint8_t*)workspace + kWsAmaxOffset);
+    const uint32_t tiles_c = (uint32_t)((C + kTrTile - 1) / kTrTile);
+    const uint32_t ntiles = (uint32_t)((R + kTrTile - 1) / kTrTile) * tiles_c;
+    // six workgroups' tiles and tables fit a CU's LDS at once
+    const uint32_t grid = std::min<uint32_t>(ntiles, 1536);
+    const bool nt = use_nontemporal(2 * R * C);
+    auto kernel = q_out ? (nt ? quantize_t_kernel<true, true> : quantize_t_kernel<true, false>)
+                        : (nt ? quantize_t_kernel<false, true> : quantize_t_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFp8Threads), 0, (hipStream_t)stream, (const uint16_t*)x, R, C,
+                       (uint8_t*)q_out, (uint8_t*)qt_out, scale_out, slot, epoch, tiles_c, ntiles);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_quantize_e4m3fn_t launch: %s", hipGetErrorString(e));
     return BS_OK;
 }
 

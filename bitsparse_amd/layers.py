@@ -17,12 +17,14 @@ from torch.autograd import Function, forward_ad
 from . import config
 from .bitsparse import BitsparseTensor, TensorBuffer
 from .config import RELU2_SCALE
-from .fp8 import Fp8Operand, as_fp8_operand, fp8_gemm, is_fp8, linear_fp8_backward, matmul, to_fp8
+from .fp8 import (Fp8Operand, as_fp8_operand, as_right_operand, fp8_gemm, is_fp8, linear_fp8_backward, matmul,
+                  to_fp8)
 from .src.functions import (activate_and_compress, activate_ok, fused_linear_relu_ok, linear_relu_and_compress,
                             relu2_and_compress, relu2_fused_ok, relu2_quantize_and_compress, relu_and_compress,
                             relu_quantize_and_compress)
 from .src.hip_operators import (act_grad_sums_, act_grad_sums_supported, col_sum, col_sum_supported,
-                                mask_with_bitmask_, quantize_e4m3fn, relu2_grad_sparse_, relu2_square_amax_)
+                                mask_with_bitmask_, quantize_e4m3fn, quantize_e4m3fn_t, quantize_t_supported,
+                                relu2_grad_sparse_, relu2_square_amax_)
 from .src.sparse_matmul import AspB, AspRelu2B
 
 # FFNRelu / FFNRelu2 with bf16 storage into a TensorBuffer run the up-projection
@@ -278,28 +280,38 @@ class _FFNBlock(Function):
             grad_W2 = product(grad_output.T, h, A_scale=scale)
         if need_x or need_W1 or need_b1:
             if ctx.fp8:
-                grad_h = fp8_gemm(Fp8Operand(grad_output, scale), as_fp8_operand(W2, None), torch.bfloat16)
+                grad_h = fp8_gemm(Fp8Operand(grad_output, scale), as_right_operand(W2), torch.bfloat16)
             else:
                 grad_h = grad_output @ W2
             need_g = ctx.fp8 and (need_x or need_W1)
-            g8 = None
+            g8 = gt8 = None
             if (need_b1 or need_g) and not torch.is_grad_enabled() and act_grad_sums_supported(grad_h, h, ctx.square):
                 grad_z = grad_h
                 grad_b1, epoch = act_grad_sums_(grad_z, h, ctx.square, need_b1, need_g)
                 if need_g:
-                    g8 = Fp8Operand(*quantize_e4m3fn(grad_z, epoch))
+                    g8, gt8 = _quantized_both_ways(grad_z, epoch, need_x, need_W1)
             else:
                 grad_z = relu2_grad_sparse_(grad_h, h) if ctx.square else mask_with_bitmask_(grad_h, h)
                 if need_b1:
                     grad_b1 = _col_sum(grad_z)
                 if need_g:
                     g8 = as_fp8_operand(grad_z, None)
+                    gt8 = g8.T
             if ctx.fp8:
-                grad_x, grad_W1 = linear_fp8_backward(x, W1, g8, need_x, need_W1)
+                grad_x, grad_W1 = linear_fp8_backward(x, W1, g8, gt8, need_x, need_W1)
             else:
                 grad_x = grad_z.mm(W1) if need_x else None
                 grad_W1 = grad_z.t().mm(x) if need_W1 else None   # W1's own layout, as autograd forms it
         return grad_x, grad_W1, grad_b1, grad_W2, grad_b2, None, None, None, None
+
+
+def _quantized_both_ways(g: Tensor, epoch: int, rows: bool, cols: bool) -> tuple[Fp8Operand | None, Fp8Operand | None]:
+    """(g in fp8, its transpose in fp8), each row-major, from the amax of ``epoch``."""
+    if cols and quantize_t_supported(g):
+        q, qt, scale = quantize_e4m3fn_t(g, epoch, rows)
+        return (Fp8Operand(q, scale) if rows else None), Fp8Operand(qt, scale)
+    g8 = Fp8Operand(*quantize_e4m3fn(g, epoch))
+    return g8, g8.T
 
 
 def _col_sum(g: Tensor) -> Tensor:
