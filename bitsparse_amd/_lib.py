@@ -84,7 +84,6 @@ _SIGNATURES = {
     "bs_compress_noalloc": [_vp, _int, _i64, _i64, _int, _int, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _int,
                             _vp, _vp, _int, _vp, _vp, _vp],
     "bs_compress_noalloc_max_tiles": [],
-    "bs_compress_act_workspace_bytes": [_i64, _i64],
     "bs_compress_act": [_vp, _vp, _i64, _i64, _int, _f32, _int, _vp, _u32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64,
                         _int, _vp, _vp, _vp, _vp, _vp, _i64, _u32, _vp],
     "bs_amax_bias_relu": [_vp, _i64, _i64, _vp, _vp, _i64, _u32, _vp],
@@ -106,7 +105,6 @@ _RESTYPES = {
     "bs_gemm_compressed_b_packed_workspace_bytes": _i64,
     "bs_compress_noalloc_max_tiles": _i64,
     "bs_linear_relu_compress_max_n": _i64,
-    "bs_compress_act_workspace_bytes": _i64,
     "bs_grad_sums_workspace_bytes": _i64,
     "bs_col_sum_workspace_bytes": _i64,
     "bs_nontemporal_min_bytes": _i64,

@@ -392,4 +392,34 @@ __device__ __forceinline__ uint2 quant_chunk_tab(const uint4 v, const uint8_t* q
     return uint2{p[0] | (p[1] << 16), p[2] | (p[3] << 16)};
 }
 
+// The activation step's pair table: entry i (as above, positive magnitudes
+// only) holds the code of r in its low byte and that of h(r) in its high one.
+// It serves a tensor whose scale of h is finite: its r (>= 0) are then finite
+// too, h(r) of everything below the window is under 2^-40 of amax|h| and
+// converts to a zero, and nothing lies above the window but r's own NaN code
+// (which no finite tensor looks up).
+__device__ __forceinline__ void pair_codes_tab(const uint4 v, const uint16_t* tab, int qoff, uint2& r, uint2& h)
+{
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const u16x2 lo = (u16x2)(unsigned short)(qoff > 0 ? qoff : 0);
+    const u16x2 hi = (u16x2)(unsigned short)(qoff + kQtabEntries - 1);
+    const u16x2 off = (u16x2)(unsigned short)(uint32_t)qoff;
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t p[4];
+    uint32_t rr[4], hh[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const u16x2 m = __builtin_bit_cast(u16x2, w[k]) & (u16x2)(unsigned short)0x7fff;
+        const uint32_t ii = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_elementwise_max(m, lo), hi) - off);
+        p[k] = (uint32_t)tab[ii & 0xffffu] | ((uint32_t)tab[ii >> 16] << 16);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k += 2) {
+        rr[k] = __builtin_amdgcn_perm(p[k + 1], p[k], 0x06040200u);
+        hh[k] = __builtin_amdgcn_perm(p[k + 1], p[k], 0x07050301u);
+    }
+    r = uint2{rr[0], rr[2]};
+    h = uint2{hh[0], hh[2]};
+}
+
 }  // namespace bs

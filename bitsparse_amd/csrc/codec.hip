@@ -135,26 +135,55 @@ __device__ __forceinline__ uint4 add_bias_chunk(const uint4 z, const uint4 b)
 }
 
 // entry i of each half stands for magnitude base + i - 1 (the end entries
-// for every magnitude past them); scale from the amax slot, for the second
-// table (blocks from kQtabBlocks on) that of h = k r^2
-constexpr int kQtabBlocks = (kQtabEntries + 255) / 256;
-__global__ __launch_bounds__(256) void qtab_build_kernel(const uint64_t* slot, uint32_t epoch, uint8_t* qtab,
-                                                         float k)
+// for every magnitude past them); scale from the amax slot
+__device__ __forceinline__ uint32_t qtab_entry(int m, float scale)
 {
-    const bool h = blockIdx.x >= kQtabBlocks;
-    const int i = (int)((blockIdx.x - (h ? kQtabBlocks : 0)) * 256 + threadIdx.x);
-    if (i >= kQtabEntries) return;
-    const float scale = h ? relu2_scale_from_slot(slot, epoch, k) : scale_from_slot(slot, epoch);
-    if (h) qtab += kQtabBytes;
-    const int m = min(max(qtab_offset(scale) + i, 0), 0x7fff);
     const uint32_t c = f32_to_e4m3(bf16_to_f32((uint32_t)m) / scale);
-    if (scale != scale) {
-        qtab[i] = 0x7fu;
-        qtab[kQtabEntries + i] = m > 0x7f80 ? 0xffu : 0x7fu;
-    } else {
-        qtab[i] = (uint8_t)c;
-        qtab[kQtabEntries + i] = (uint8_t)(c | 0x80u);
+    return scale != scale ? 0x7fu : c;
+}
+__global__ __launch_bounds__(256) void qtab_build_kernel(const uint64_t* slot, uint32_t epoch, uint8_t* qtab)
+{
+    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (i >= kQtabEntries) return;
+    const float scale = scale_from_slot(slot, epoch);
+    const int m = min(max(qtab_offset(scale) + i, 0), 0x7fff);
+    const uint32_t c = qtab_entry(m, scale);
+    qtab[i] = (uint8_t)c;
+    // (a NaN scale gives x's own NaN for a NaN x, else the scale's)
+    qtab[kQtabEntries + i] = (uint8_t)(scale != scale && m <= 0x7f80 ? 0x7fu : c | 0x80u);
+}
+
+// The pair table (pair_codes_tab): the code of r and that of h = k r^2
+__global__ __launch_bounds__(256) void pair_tab_build_kernel(const uint64_t* slot, uint32_t epoch, uint16_t* tab,
+                                                             float k)
+{
+    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (i >= kQtabEntries) return;
+    const float scale = scale_from_slot(slot, epoch), h_scale = relu2_scale_from_slot(slot, epoch, k);
+    const int m = min(max(qtab_offset(scale) + i, 0), 0x7fff);
+    const uint32_t hc = f32_to_e4m3(bf16_to_f32(relu2_sq_bits((uint32_t)m, k)) / h_scale);
+    tab[i] = (uint16_t)(qtab_entry(m, scale) | (hc << 8));
+}
+
+// The codes of a chunk of r >= 0 (or NaN) and of its h where the scale of h is
+// infinite or NaN (an Inf or NaN in the tensor, or a square past bf16's
+// range), from what the pair table gave: a NaN r keeps its sign; h is a zero
+// over an infinite scale unless it is infinite, and a NaN over a NaN one.
+__device__ __forceinline__ void codes_nonfinite_scale(const uint4 v, float k, float h_scale, uint2& r, uint2& h)
+{
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    r.x |= __builtin_amdgcn_perm(w[1], w[0], 0x07050301u) & 0x80808080u;
+    r.y |= __builtin_amdgcn_perm(w[3], w[2], 0x07050301u) & 0x80808080u;
+    const bool nan_s = h_scale != h_scale;
+    const uint32_t inf_code = f32_to_e4m3(__uint_as_float(0x7f800000u) / h_scale);
+    uint32_t o[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const uint32_t b = relu2_sq_bits((w[e >> 1] >> (16 * (e & 1))) & 0xffffu, k), mag = b & 0x7fffu;
+        const uint32_t c = nan_s ? 0x7fu : ((b >> 8) & 0x80u) | (mag < 0x7f80u ? 0u : mag == 0x7f80u ? inf_code : 0x7fu);
+        o[e >> 2] |= c << (8 * (e & 3));
     }
+    h = uint2{o[0], o[1]};
 }
 
 // Chunk geometry inside tile t of a [*, N] matrix.
@@ -223,7 +252,13 @@ enum { WB_RELU = 0, WB_SQUARE = 1, WB_ACT = 2, WB_ACT_SQUARE = 3 };
 // behind slow predecessors stay well below it).  The environment variable
 // BITSPARSE_LOOKBACK_PATIENCE (ticks) overrides it; 0 makes every wait take
 // the fallback, which is how the tests exercise that path.
+// Counting reads the dense input, which an in-place write-back may have
+// replaced by then.  relu(z) counts as z does; the ReLU^2 layer's in-place
+// square does not (a square can underflow, k can be negative), so that form
+// waits up to kInPlaceSquareTicks (10 s, whatever the variable says) and
+// flags bit 2 of *err if it has to count after all.
 constexpr uint64_t kLookbackPatienceTicks = 20000;
+constexpr uint64_t kInPlaceSquareTicks = 1000000000;
 
 template <int IN_T, bool QUANT>
 struct CompressTraits {
@@ -302,7 +337,9 @@ __device__ __forceinline__ typename Raw<DT == DT_BF16 ? 2 : 1>::T relu_chunk(typ
 
 // Nonzero count of compress unit q computed straight from the dense input by
 // one wave (look-back fallback).
-template <int IN_T, bool QUANT, bool VEC, int U>
+// ACT: the bias is added as the unit adds it (every chunk of a row inside the
+// matrix; those past it count nothing).
+template <int IN_T, bool QUANT, bool VEC, int U, bool ACT>
 __device__ uint32_t unit_count_wave(const CompressArgs& a, uint32_t q, float scale, int lane)
 {
     using TR = CompressTraits<IN_T, QUANT>;
@@ -313,6 +350,10 @@ __device__ uint32_t unit_count_wave(const CompressArgs& a, uint32_t q, float sca
         int64_t row, col0;
         chunk_pos(t0 + (k >> 9), a.grid_n, (int)(k & 511), row, col0);
         auto d = load_chunk<TR::INB, VEC>(a.dense, a.M, a.N, row, col0);
+        if constexpr (ACT) {
+            if (a.bias != nullptr && row < a.M && col0 < a.N)
+                d = add_bias_chunk(d, *reinterpret_cast<const uint4*>(a.bias + col0));
+        }
         if constexpr (IN_T == DT_BF16 && !QUANT) {
             // count only (no mask byte): few live registers on this rare path
             const uint32_t w[4] = {d.x, d.y, d.z, d.w};
@@ -346,7 +387,7 @@ __device__ __forceinline__ uint64_t bcast_lane0(uint64_t v)
 // dense input instead.  Returns the exclusive prefix of unit u in every lane.
 constexpr int kGroupUnits = 64;
 
-template <int IN_T, bool QUANT, bool VEC, int U>
+template <int IN_T, bool QUANT, bool VEC, int U, bool ACT>
 __device__ uint32_t wave_lookback_grouped(const CompressArgs& a, uint32_t u, uint32_t unit_total,
                                           float scale, int lane)
 {
@@ -408,8 +449,9 @@ __device__ uint32_t wave_lookback_grouped(const CompressArgs& a, uint32_t u, uin
                 break;
             }
             if (wall_clock64() - since > a.patience) {
-                excl += unit_count_wave<IN_T, QUANT, VEC, U>(a, (uint32_t)pos, scale, lane);
+                excl += unit_count_wave<IN_T, QUANT, VEC, U, ACT>(a, (uint32_t)pos, scale, lane);
                 if (lane == 0 && a.fallbacks) atomicAdd(a.fallbacks, 1u);
+                if (lane == 0 && a.err && a.patience == kInPlaceSquareTicks) atomicOr(a.err, 4);
                 break;
             }
             __builtin_amdgcn_s_sleep(4);
@@ -645,7 +687,6 @@ void compress_stream_kernel(CompressArgs a)
     constexpr bool ACT = WB == WB_ACT || WB == WB_ACT_SQUARE;
     static_assert(!ACT || VEC, "the activation step takes vector loads");
     constexpr bool RSQ = WB == WB_SQUARE || (WB == WB_ACT_SQUARE && !QUANT), HCODES = WB == WB_ACT_SQUARE && QUANT;
-    constexpr int kTabs = HCODES ? 2 : 1;   // code tables: r's, and h's behind it
     constexpr bool WRITE_VALS = MODE != MODE_COUNT;
     using TR = CompressTraits<IN_T, QUANT>;
     constexpr int INB = TR::INB, OUTB = TR::OUTB;
@@ -663,7 +704,7 @@ void compress_stream_kernel(CompressArgs a)
     // the quantizer's code table is read only while the chunks are masked,
     // the value rings only after the look-back's barrier: they share LDS
     constexpr int kRingBytes = WRITE_VALS ? U * kRingElems * OUTB : 16;
-    constexpr int kShared = QUANT && kTabs * kQtabBytes > kRingBytes ? kTabs * kQtabBytes : kRingBytes;
+    constexpr int kShared = QUANT && kQtabBytes > kRingBytes ? kQtabBytes : kRingBytes;
     __shared__ __align__(16) uint8_t s_area[kShared];
     uint8_t* const s_ring = s_area;
     uint8_t* const s_qtab = s_area;
@@ -682,7 +723,6 @@ void compress_stream_kernel(CompressArgs a)
     const int qoff = QUANT ? qtab_offset(scale) : 0;
     float h_scale = 1.0f;
     if constexpr (HCODES) h_scale = relu2_scale_from_slot(a.amax_slot, a.amax_epoch, a.relu_k);
-    const int hoff = HCODES ? qtab_offset(h_scale) : 0;
     int64_t start = 0;
     if (a.offset_in) start = *a.offset_in;
     if (a.align8) start = (start + 7) & ~(int64_t)7;
@@ -745,7 +785,7 @@ void compress_stream_kernel(CompressArgs a)
         }
         if constexpr (QUANT) {
             // the code table into LDS, behind the dense loads (16-byte copies)
-            for (int i = tid; i < kTabs * kQtabBytes / 16; i += 64 * U)
+            for (int i = tid; i < kQtabBytes / 16; i += 64 * U)
                 reinterpret_cast<uint4*>(s_qtab)[i] = reinterpret_cast<const uint4*>(a.qtab)[i];
             __syncthreads();
         }
@@ -775,8 +815,15 @@ void compress_stream_kernel(CompressArgs a)
                 o[k] = d[k];
                 m = tile_ok ? vm[k] & 0xffu : 0u;
             } else {
-                m = stream_chunk_mask<IN_T, QUANT, QUANT>(d[k], o[k], scale, rcp, s_qtab, qoff) &
-                    (8 * k < rows_in ? 0xffu : 0u);
+                uint2 h8;
+                if constexpr (HCODES) {
+                    pair_codes_tab(d[k], reinterpret_cast<const uint16_t*>(s_qtab), qoff, o[k], h8);
+                    if (!(h_scale < __builtin_inff())) codes_nonfinite_scale(d[k], a.relu_k, h_scale, o[k], h8);
+                    m = mask_fp8x8<DT_E4M3FN>(o[k]);
+                } else {
+                    m = stream_chunk_mask<IN_T, QUANT, QUANT>(d[k], o[k], scale, rcp, s_qtab, qoff);
+                }
+                m &= 8 * k < rows_in ? 0xffu : 0u;
                 if (tile_ok) {
                     if constexpr (VEC) {
                         // in range, the lane's unclamped place in the tile
@@ -791,9 +838,7 @@ void compress_stream_kernel(CompressArgs a)
                         }
                         if constexpr (HCODES) {
                             if (8 * k < rows_in)
-                                st_chunk<false, RawOut>(a.dense_q_out + ko + (uint64_t)lo,
-                                                        quant_chunk_tab(relu2_sq_chunk(d[k], a.relu_k),
-                                                                        s_qtab + kQtabBytes, hoff));
+                                st_chunk<false, RawOut>(a.dense_q_out + ko + (uint64_t)lo, h8);
                         } else if constexpr (QUANT) {
                             if (a.dense_q_out != nullptr && 8 * k < rows_in)
                                 st_chunk<false, RawOut>(a.dense_q_out + ko + (uint64_t)lo, o[k]);
@@ -880,7 +925,7 @@ void compress_stream_kernel(CompressArgs a)
         if (MODE != MODE_VALS && wave == 0) {
             uint32_t excl = 0;
             if (u != 0) {
-                excl = wave_lookback_grouped<IN_T, QUANT, VEC, U>(a, u, unit_total, scale, lane);
+                excl = wave_lookback_grouped<IN_T, QUANT, VEC, U, ACT>(a, u, unit_total, scale, lane);
                 if (lane == 0) st_relaxed(&a.status[u], pack_status(a.epoch, kFlagInc, excl + unit_total));
             }
             if (lane == 0 && ((u + 1) & (kGroupUnits - 1)) == 0)
@@ -2124,12 +2169,17 @@ static int compress_impl(const void* dense, int in_dtype, int64_t M, int64_t N, 
         const unsigned long long v = strtoull(ev, &end, 10);
         if (end != ev) a.patience = (uint64_t)v;
     }
+    if (wb == WB_SQUARE && relu_out == dense) a.patience = kInPlaceSquareTicks;
     a.gstat = a.status + (T + kStreamU - 1) / kStreamU;
     if (quantize) {
         // the code table of this call's scale, built after the amax it reads
         uint8_t* qtab = (uint8_t*)workspace + ws_qtab_offset(T);
-        hipLaunchKernelGGL(qtab_build_kernel, dim3(kQtabBlocks * (wb == WB_ACT_SQUARE ? 2 : 1)), dim3(256), 0, st,
-                           amax_slot, amax_epoch, qtab, relu_k);
+        if (wb == WB_ACT_SQUARE)
+            hipLaunchKernelGGL(pair_tab_build_kernel, dim3((kQtabEntries + 255) / 256), dim3(256), 0, st, amax_slot,
+                               amax_epoch, (uint16_t*)qtab, relu_k);
+        else
+            hipLaunchKernelGGL(qtab_build_kernel, dim3((kQtabEntries + 255) / 256), dim3(256), 0, st, amax_slot,
+                               amax_epoch, qtab);
         a.qtab = qtab;
     }
     const int inb = in_dtype == DT_BF16 ? 2 : 1;
@@ -2188,12 +2238,6 @@ extern "C" int bs_compress_relu2(const void* preact, int quantize, int64_t M, in
                          WB_SQUARE, k);
 }
 
-extern "C" int64_t bs_compress_act_workspace_bytes(int64_t M, int64_t N)
-{
-    const int64_t w = bs_compress_workspace_bytes(M, N);
-    return w < 0 ? w : w + kQtabBytes;      // the code table of h behind that of r
-}
-
 extern "C" int bs_compress_act(const void* preact, const void* bias, int64_t M, int64_t N, int square, float k,
                                int quantize, const uint64_t* amax_slot, uint32_t amax_epoch, float* scale_out,
                                void* codes_out, float* codes_scale_out, void* h_out, uint8_t* bitmask,
@@ -2211,11 +2255,11 @@ extern "C" int bs_compress_act(const void* preact, const void* bias, int64_t M, 
     if (quantize ? (codes_out == nullptr || !aligned8(codes_out) || h_out != nullptr) : h_out == nullptr)
         return set_error(BS_ERR_INVALID, "bs_compress_act: quantize writes codes_out (8-byte aligned) and no h_out, "
                                          "else h_out is written");
+    if (h_out == preact && (square || bias != nullptr))
+        return set_error(BS_ERR_INVALID, "bs_compress_act: h_out may alias preact only without a bias or square");
     if (quantize && amax_slot == nullptr) return set_error(BS_ERR_INVALID, "bs_compress_act: null amax slot");
     if ((uint64_t)M * (uint64_t)N >= kMaxElemsUntested)
         return set_error(BS_ERR_INVALID, "bs_compress_act: M*N must be < 2^31");
-    if (workspace_bytes < bs_compress_act_workspace_bytes(M, N))
-        return set_error(BS_ERR_INVALID, "bs_compress_act: workspace too small");
     const int wb = square ? WB_ACT_SQUARE : WB_ACT;
     return compress_impl(preact, DT_BF16, M, N, quantize, amax_slot, amax_epoch, scale_out, codes_out, bitmask, prefix,
                          vals, vals_capacity, vals_offset_in, packed, vals_offset_out, vals_start_out, 1, err_flags,

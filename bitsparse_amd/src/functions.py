@@ -362,7 +362,7 @@ def activate_and_compress(z: Tensor, bias: Tensor | None, sparse_data: TensorBuf
     """The activation step of an MLP block on its up-projection z, which
     nothing reads afterwards: r = relu(z + bias) compressed into
     ``sparse_data`` and the down-projection's operand -- r, or with ``square``
-    k r^2; in bf16 (written over z), or with ``fp8`` as e4m3fn codes with their
+    k r^2; in bf16 (over z, or new), or with ``fp8`` as e4m3fn codes with their
     scale (``to_fp8`` of it).  Bit for bit the separate bias add,
     relu_[quantize_]and_compress, square and quantize.  Needs ``activate_ok``.
     Returns (operand, its scale or None, compressed r)."""
@@ -388,8 +388,9 @@ def activate_and_compress(z: Tensor, bias: Tensor | None, sparse_data: TensorBuf
         fused = dict(codes_out=operand, scale_out=scale, amax_epoch=epoch,
                      codes_scale_out=operand_scale if square else None)
     else:
-        operand = z
-        fused = dict(h_out=z)
+        # over z where that leaves a recount of z (the look-back's fallback) right
+        operand = z if bias is None and not square else torch.empty_like(z)
+        fused = dict(h_out=operand)
     ops.compress_act_into(z, bias, square, bitmask, prefix, sparse_data.vals, pack_sbit, cursor, advanced, start,
                           sparse_data.err_flags, **fused)
     sparse_data.advance(advanced)

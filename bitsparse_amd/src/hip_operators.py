@@ -327,7 +327,7 @@ def compress_act_into(z: Tensor, bias: Tensor | None, square: bool, bitmask: Ten
     quantize = codes_out is not None
     L = _lib.load()
     ws = _lib.workspace_for(z.device)
-    ws.ensure(L.bs_compress_act_workspace_bytes(M, N))
+    ws.ensure(L.bs_compress_workspace_bytes(M, N))
     epoch = ws.next_epoch()
     check(L.bs_compress_act(z.data_ptr(), ptr(bias), M, N, int(square), float(RELU2_SCALE), int(quantize),
                             ws.amax_slot_ptr() if quantize else None, amax_epoch, ptr(scale_out), ptr(codes_out),

@@ -545,8 +545,9 @@ int64_t bs_compress_noalloc_max_tiles(void);
  * only what the down-projection multiplies is written: r, or with square = 1
  * h = bf16(bf16(r * r) * k), k finite.
  *   bias       bf16 [N], 16-byte aligned; nullable: none
- *   quantize   0: bf16 values; h_out (bf16 [M, N], 16-byte aligned, may alias
- *              preact) receives r or h, codes_out is not used.
+ *   quantize   0: bf16 values; h_out (bf16 [M, N], 16-byte aligned; may alias
+ *              preact only without bias and square: a look-back fallback
+ *              counts from preact) receives r or h, codes_out is not used.
  *              1: e4m3fn values with the scale of amax|r|, which the amax
  *              slot holds under amax_epoch (bs_amax_bias_relu, or
  *              bs_amax_relu without a bias); h_out must be null; codes_out
@@ -554,13 +555,12 @@ int64_t bs_compress_noalloc_max_tiles(void);
  *              (their scale is scale_out) or of h, as to_fp8 makes them, with
  *              their scale in codes_scale_out.
  * M, N >= 1, N % 8 == 0, preact 16-byte aligned, M * N < 2^31; workspace of
- * bs_compress_act_workspace_bytes(M, N) bytes; the other arguments as for
+ * bs_compress_workspace_bytes(M, N) bytes; the other arguments as for
  * bs_compress (packed: the stream and its bytes, as for bs_compress_packed).
  * Refused while `stream` is capturing.  Replaces z = z + b1; h = z.relu_();
  * [to_fp8(h)]; dense_to_tilesparse(h); [h.square_(); h.mul_(k); to_fp8(h)] of
  * lib_sparse/layers.py:29-39, :86-89, :107-119, :169-172.
  */
-int64_t bs_compress_act_workspace_bytes(int64_t M, int64_t N);
 int bs_compress_act(const void* preact, const void* bias, int64_t M, int64_t N, int square, float k,
                     int quantize, const uint64_t* amax_slot, uint32_t amax_epoch, float* scale_out,
                     void* codes_out, float* codes_scale_out, void* h_out, uint8_t* bitmask,

@@ -36,7 +36,7 @@ def test_activation_step(dev, shape, bias, square, store, special):
     from bitsparse_amd.fp8 import to_fp8
     from bitsparse_amd.src import functions as F
     fp8, pack = store.startswith("e4m3"), store.endswith("packed")
-    z, b = _z(shape, 3, special and not fp8, dev)
+    z, b = _z(shape, 3, special, dev)
     n = z.numel()
     size = (n * (7 if fp8 else 15) + 7) // 8 + 16 if pack else n * (1 if fp8 else 2)
     bufs = [TensorBuffer(size, device=dev, dtype=E4M3 if fp8 else torch.bfloat16, pack_sbit=pack) for _ in range(2)]
@@ -62,18 +62,55 @@ def test_activation_step(dev, shape, bias, square, store, special):
         _same(oscale.reshape(1), got_scale.reshape(1), "operand scale")
 
 
-def test_codes_of_an_overflowing_square(dev):
-    """r finite, k r^2 past bf16's range: the scale of h is infinite, as to_fp8 has it."""
+@pytest.mark.parametrize("value", [2.0e25, 3.0e-25, float("inf"), float("nan"), -float("nan"), None])
+@pytest.mark.parametrize("k", [1.0, 0.37, -2.0, 0.0])
+def test_codes_of_the_square(dev, value, k, monkeypatch):
+    """The codes of h = k r^2 over the whole range of scales: a square past
+    bf16's range (an infinite scale), all squares underflowing, Inf, NaN of
+    either sign, an all-negative pre-activation; k of either sign and 0."""
     from bitsparse_amd.bitsparse import TensorBuffer
     from bitsparse_amd.fp8 import to_fp8
     from bitsparse_amd.src import functions as F
+    from bitsparse_amd.src import hip_operators as H
+    monkeypatch.setattr(H, "RELU2_SCALE", k)
     z, _ = _z((70, 136), 4, False, dev)
-    z[3, 5] = 2.0e25
-    buf = TensorBuffer(z.numel(), device=dev, dtype=E4M3)
-    want, wscale = to_fp8(z.relu().square().mul_(1.0))
-    got, gscale, _ = F.activate_and_compress(z, None, buf, False, True, True)
-    _same(wscale.reshape(1), gscale.reshape(1), "scale")
-    _same(want, got, "codes")
+    if value is None:
+        z = -z.abs()
+    elif value == 3.0e-25:
+        z = z * value
+    else:
+        z[3, 5] = value
+    bufs = [TensorBuffer(z.numel(), device=dev, dtype=E4M3) for _ in range(2)]
+    r = z.clone()
+    want_sp = F.relu_quantize_and_compress(r, bufs[0], False)[2]
+    want, wscale = to_fp8(r.square().mul_(k))
+    got, gscale, sp = F.activate_and_compress(z, None, bufs[1], False, True, True)
+    _same(wscale.reshape(1), gscale.reshape(1), "scale of h")
+    _same(want, got, "codes of h")
+    _same(want_sp.scale.reshape(1), sp.scale.reshape(1), "scale")
+    _same(want_sp.bitmask, sp.bitmask, "bitmask")
+    _same(bufs[0].vals, bufs[1].vals, "values")
+
+
+@pytest.mark.parametrize("store", ["bf16", "e4m3"])
+def test_activation_step_lookback_fallback(dev, store, monkeypatch):
+    """With no patience every wait counts its predecessors from the dense
+    input, where the bias has to be added too (and rows past the matrix, whose
+    bias alone may be positive, count nothing)."""
+    from bitsparse_amd.bitsparse import TensorBuffer
+    from bitsparse_amd.src import functions as F
+    z, b = _z((72, 64 * 40), 12, False, dev)
+    b = b.abs()
+    dt = E4M3 if store == "e4m3" else torch.bfloat16
+    outs = []
+    for patience in (None, "0"):
+        if patience is not None:
+            monkeypatch.setenv("BITSPARSE_LOOKBACK_PATIENCE", patience)
+        buf = TensorBuffer(2 * z.numel(), device=dev, dtype=dt)
+        sp = F.activate_and_compress(z.clone(), b, buf, False, store == "e4m3", True)[2]
+        outs.append((sp.prefix, buf.vals, buf.offset))
+    for x, y, what in zip(*outs, ("prefix", "values", "cursor")):
+        _same(x, y, what)
 
 
 @pytest.mark.parametrize("shape", [(1, 8), (64, 64), (65, 72), (80, 1416), (1000, 1024), (4100, 192)])
