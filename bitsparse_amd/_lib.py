@@ -116,6 +116,25 @@ _lib = None
 _lock = threading.Lock()
 
 
+_native_module = None
+
+
+def native():
+    """The native host path (csrc/native.cpp, built as ``_native``), bound to
+    the library this module loaded."""
+    global _native_module
+    if _native_module is None:
+        load()
+        try:
+            from . import _native
+        except ImportError as e:
+            raise ImportError(f"bitsparse_amd/_native is missing or does not load ({e}): build it with "
+                              f"`python -c 'import __graft_entry__ as g; g.build()'`") from e
+        _native.init(LIB_PATH)
+        _native_module = _native
+    return _native_module
+
+
 class LaunchTimer:
     """Kernel durations of this thread's compress / decompress launches,
     recorded by the library at each kernel's own start and end
@@ -205,68 +224,11 @@ def require_device(t: torch.Tensor, what: str) -> None:
 
 # ---------------------------------------------------------------------------
 # per-(device, stream) workspace for the single-pass compress and the amax
+# (the native module's Workspace: an epoch counter over zero-initialised
+# device scratch)
 # ---------------------------------------------------------------------------
 _EPOCH_LIMIT = (1 << 30) - 1
 
 
-class Workspace:
-    """Zero-initialised device scratch with an epoch counter.
-
-    Each compress / amax call takes a fresh epoch; status words written under
-    older epochs are ignored by the kernels, so the buffer never needs
-    clearing between calls.  When the epoch counter wraps the buffer is
-    zeroed again.
-    """
-
-    def __init__(self, device: torch.device):
-        self.device = device
-        self.buf = torch.zeros(0, dtype=torch.uint8, device=device)
-        self.epoch = 0
-
-    def ensure(self, nbytes: int) -> None:
-        if self.buf.numel() < nbytes:
-            # grow geometrically; the old contents (amax slot, status words of
-            # earlier epochs) move along and the new tail is zero, so epochs
-            # already handed out stay meaningful
-            size = max(nbytes, 2 * self.buf.numel(), 1 << 16)
-            new = torch.zeros(size, dtype=torch.uint8, device=self.device)
-            if self.buf.numel():
-                new[:self.buf.numel()].copy_(self.buf)
-            self.buf = new
-
-    def next_epoch(self, reserve: int = 1) -> int:
-        """A fresh epoch.  ``reserve`` = how many epochs the caller's sequence
-        takes in total (the amax of a quantizing compress reserves 2), so the
-        wrap -- which zeroes the buffer, amax slot included -- never falls
-        between the amax and the compress that reads it."""
-        if self.epoch + reserve > _EPOCH_LIMIT:
-            self.buf.zero_()
-            self.epoch = 0
-        self.epoch += 1
-        return self.epoch
-
-    @property
-    def nbytes(self) -> int:
-        return self.buf.numel()
-
-    def amax_slot_ptr(self) -> int:
-        return load().bs_workspace_amax_slot(self.buf.data_ptr(), self.nbytes)
-
-    def fallback_count(self) -> int:
-        """Look-back fallbacks recorded in this workspace (synchronises)."""
-        if self.buf.numel() < 12:
-            return 0
-        return int(self.buf[8:12].view(torch.int32).item())
-
-
-_workspaces: dict[tuple[int, int], Workspace] = {}
-
-
-def workspace_for(device: torch.device) -> Workspace:
-    dev = device.index if device.index is not None else torch.cuda.current_device()
-    key = (dev, torch.cuda.current_stream(device).cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None:
-        ws = Workspace(torch.device("cuda", dev))
-        _workspaces[key] = ws
-    return ws
+def workspace_for(device: torch.device):
+    return native().workspace(-1 if device.index is None else device.index)

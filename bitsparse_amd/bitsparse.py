@@ -129,7 +129,6 @@ class TensorBuffer:
     lib_sparse/bitsparse.py:90-117.
     """
     vals: Tensor
-    offset: Tensor
 
     def __init__(self, size: int, device="cuda", dtype=torch.bfloat16,
                  pack_sbit: bool = False, *, inplace_offset: bool = False):
@@ -149,15 +148,26 @@ class TensorBuffer:
                 raise ValueError("raw TensorBuffer size must be a multiple of dtype size")
             numel = self.size // torch.empty((), dtype=dtype).element_size()
             self.vals = torch.zeros(numel, device=self.device, dtype=self.dtype)
-        self.offset = torch.zeros(1, device=self.device, dtype=torch.int64)
+        self._offset = torch.zeros(1, device=self.device, dtype=torch.int64)
         self.err_flags = torch.zeros(1, device=self.device, dtype=torch.int32)
+
+    @property
+    def offset(self) -> Tensor:
+        """The cursor, a 1-element int64 tensor (after a reset, made when first asked for)."""
+        if self._offset is None:
+            self._offset = torch.zeros(1, device=self.device, dtype=torch.int64)
+        return self._offset
+
+    @offset.setter
+    def offset(self, value: Tensor) -> None:
+        self._offset = value
 
     def reset_buffer(self):
         """Start filling from offset 0 again (once per training step)."""
         if self.inplace_offset:
             self.offset.zero_()
         else:
-            self.offset = torch.zeros(1, device=self.device, dtype=torch.int64)
+            self._offset = None      # 0: a compress needs no tensor filled with it
 
     def cursor(self) -> tuple[Tensor, Tensor]:
         """(start, out) for one compress into this buffer: the kernel reads the

@@ -63,5 +63,26 @@ def build_library(verbose: bool = False, out: str | None = None,
     return out
 
 
+def build_native(verbose: bool = False) -> str:
+    """Compile csrc/native.cpp (host code against torch's C++ API) into
+    bitsparse_amd/_native.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    out = os.path.join(PKG, "_native.so")
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc = cpp_extension.include_paths() + [os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+                                           sysconfig.get_paths()["include"], INCLUDE]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-DTORCH_EXTENSION_NAME=_native", "-DTORCH_API_INCLUDE_EXTENSION_H",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + [f"-I{d}" for d in inc] +
+         [os.path.join(CSRC, "native.cpp"), "-o", out + ".tmp", f"-L{libs}", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+          "-lc10", "-lc10_hip", "-ltorch_python", "-ldl"], verbose)
+    os.replace(out + ".tmp", out)
+    return out
+
+
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_native(verbose=True))

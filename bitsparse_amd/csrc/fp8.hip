@@ -16,14 +16,12 @@ namespace bs {
 constexpr int kFp8Threads = 256;
 
 // max over |x| as bf16 magnitude bits; NaN patterns sort above Inf, so a NaN
-// anywhere wins the max and the decoded amax is NaN.  Bound by the read: each
-// thread keeps four independent 16-byte loads in flight per pass, in
-// workgroups of 1024 threads, two per CU.  That fills every wave slot (with
-// 256 threads, the 8 MiB in flight were too few: 64M elements 34 us) and
-// still sends only some 500 device-scope atomicMax to the one slot, the only
-// serialised step (8 workgroups per CU of 256 threads: 44 us).
+// anywhere wins the max and the decoded amax is NaN.  Each thread keeps four
+// independent 16-byte loads in flight per pass; the grid is a few workgroups
+// per CU, so the per-workgroup device-scope atomicMax on the one slot (the
+// only serialised step) stays at a few hundred.  (Workgroups of 1024 threads,
+// which fill every wave slot: 1.5 us slower per call at 4096 x 16384.)
 constexpr int kAmaxUnroll = 4;
-constexpr int kAmaxThreads = 1024;
 
 // RELU: amax of relu(x) (x <= 0 counts as 0; NaN is kept by relu, so it still wins).
 template <bool RELU>
@@ -36,16 +34,16 @@ __device__ __forceinline__ uint32_t mag_bits(uint32_t b)
 
 // NT: nontemporal loads of x.
 template <bool RELU, bool NT>
-__global__ __launch_bounds__(kAmaxThreads) void amax_bf16_kernel(const uint16_t* x, int64_t n,
+__global__ __launch_bounds__(kFp8Threads) void amax_bf16_kernel(const uint16_t* x, int64_t n,
                                                                 uint64_t* slot, uint32_t epoch)
 {
-    __shared__ uint32_t s_w[kAmaxThreads / 64];
+    __shared__ uint32_t s_w[kFp8Threads / 64];
     const int tid = threadIdx.x;
     uint32_t m = 0;
     const int64_t nvec = ((((uintptr_t)x) & 15u) == 0) ? n / 8 : 0;
-    const int64_t stride = (int64_t)gridDim.x * kAmaxThreads;
+    const int64_t stride = (int64_t)gridDim.x * kFp8Threads;
     const uint4* xv = reinterpret_cast<const uint4*>(x);
-    int64_t i = (int64_t)blockIdx.x * kAmaxThreads + tid;
+    int64_t i = (int64_t)blockIdx.x * kFp8Threads + tid;
     for (; i + (kAmaxUnroll - 1) * stride < nvec; i += kAmaxUnroll * stride) {
         uint4 v[kAmaxUnroll];
 #pragma unroll
@@ -69,13 +67,13 @@ __global__ __launch_bounds__(kAmaxThreads) void amax_bf16_kernel(const uint16_t*
             m = max(m, mag_bits<RELU>(w[k] >> 16));
         }
     }
-    for (int64_t j = nvec * 8 + (int64_t)blockIdx.x * kAmaxThreads + tid; j < n; j += stride)
+    for (int64_t j = nvec * 8 + (int64_t)blockIdx.x * kFp8Threads + tid; j < n; j += stride)
         m = max(m, mag_bits<RELU>((uint32_t)x[j]));
     m = wave_max_u32(m);
     if ((tid & 63) == 0) s_w[tid >> 6] = m;
     __syncthreads();
     if (tid == 0) {
-        for (int w = 1; w < kAmaxThreads / 64; w++) m = max(m, s_w[w]);
+        for (int w = 1; w < kFp8Threads / 64; w++) m = max(m, s_w[w]);
         atomicMax((unsigned long long*)slot, (unsigned long long)(((uint64_t)epoch << 32) | m));
     }
 }
@@ -85,14 +83,14 @@ __global__ __launch_bounds__(kAmaxThreads) void amax_bf16_kernel(const uint16_t*
 // biased pre-activation is never written (the add is repeated by the compress).
 // A thread keeps one column chunk (its stride is a whole number of rows).
 template <bool NT>
-__global__ __launch_bounds__(kAmaxThreads) void amax_bias_relu_kernel(const uint16_t* x, int64_t rows, uint32_t nc,
+__global__ __launch_bounds__(kFp8Threads) void amax_bias_relu_kernel(const uint16_t* x, int64_t rows, uint32_t nc,
                                                                      const uint16_t* bias, uint64_t* slot,
                                                                      uint32_t epoch)
 {
-    __shared__ uint32_t s_w[kAmaxThreads / 64];
+    __shared__ uint32_t s_w[kFp8Threads / 64];
     const int tid = threadIdx.x;
-    const int64_t t = (int64_t)blockIdx.x * kAmaxThreads + tid;
-    const int64_t rstep = (int64_t)gridDim.x * kAmaxThreads / nc;      // rows per pass (>= 1: host)
+    const int64_t t = (int64_t)blockIdx.x * kFp8Threads + tid;
+    const int64_t rstep = (int64_t)gridDim.x * kFp8Threads / nc;      // rows per pass (>= 1: host)
     const int64_t r0 = t / nc, c = t - r0 * nc;
     const uint4* xv = reinterpret_cast<const uint4*>(x) + c;
     typedef short i16x2 __attribute__((ext_vector_type(2)));
@@ -128,7 +126,7 @@ __global__ __launch_bounds__(kAmaxThreads) void amax_bias_relu_kernel(const uint
     if ((tid & 63) == 0) s_w[tid >> 6] = m;
     __syncthreads();
     if (tid == 0) {
-        for (int w = 1; w < kAmaxThreads / 64; w++) m = max(m, s_w[w]);
+        for (int w = 1; w < kFp8Threads / 64; w++) m = max(m, s_w[w]);
         atomicMax((unsigned long long*)slot, (unsigned long long)(((uint64_t)epoch << 32) | m));
     }
 }
@@ -210,7 +208,7 @@ static uint32_t grid_for(int64_t n)
 // amax: a chunk per thread, at most two workgroups per CU
 static uint32_t amax_grid(int64_t n, int cus)
 {
-    return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((n / 8 + kAmaxThreads - 1) / kAmaxThreads, 2 * cus));
+    return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((n / 8 + kFp8Threads - 1) / kFp8Threads, 2 * cus));
 }
 
 // the quantize pass: at least 8 chunks per thread where n allows (each
@@ -501,7 +499,7 @@ int bs::amax_launch(const void* x, int64_t n, void* workspace, int64_t workspace
     const bool nt = use_nontemporal(2 * n);
     auto kernel = relu ? (nt ? amax_bf16_kernel<true, true> : amax_bf16_kernel<true, false>)
                        : (nt ? amax_bf16_kernel<false, true> : amax_bf16_kernel<false, false>);
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kAmaxThreads), 0, (hipStream_t)stream, (const uint16_t*)x, n,
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFp8Threads), 0, (hipStream_t)stream, (const uint16_t*)x, n,
                        slot, epoch);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_amax launch: %s", hipGetErrorString(e));
@@ -544,9 +542,9 @@ extern "C" int bs_amax_bias_relu(const void* x, int64_t M, int64_t N, const void
     // two workgroups per CU (few atomics meet on the slot), and at least one
     // row of chunks per pass
     const int64_t nc = N / 8;
-    const int64_t grid = std::max<int64_t>(amax_grid(M * N, cus), (nc + kAmaxThreads - 1) / kAmaxThreads);
+    const int64_t grid = std::max<int64_t>(amax_grid(M * N, cus), (nc + kFp8Threads - 1) / kFp8Threads);
     auto kernel = use_nontemporal(2 * M * N) ? amax_bias_relu_kernel<true> : amax_bias_relu_kernel<false>;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kAmaxThreads), 0, (hipStream_t)stream, (const uint16_t*)x, M,
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kFp8Threads), 0, (hipStream_t)stream, (const uint16_t*)x, M,
                        (uint32_t)nc, (const uint16_t*)bias, slot, epoch);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_amax_bias_relu launch: %s", hipGetErrorString(e));

@@ -1,0 +1,508 @@
+// Native host path of the codec calls and of the MLP block's forward and
+// backward: the allocations and the calls into libbitsparse_hip.so and torch
+// without the interpreter between the launches.  At the small sizes the host
+// work is the whole time (a 128-token block step: 300 us of Python for 60 us
+// of kernels).  Every tensor lives on the current stream of its device; a
+// backward runs on its forward's stream (autograd sets it).
+#include <dlfcn.h>
+#include <torch/extension.h>
+
+#include <ATen/core/grad_mode.h>
+#include <ATen/hip/HIPContext.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <map>
+#include <memory>
+#include <mutex>
+
+#include "bitsparse_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+// ---------------------------------------------------------------------------
+// libbitsparse_hip.so (the path Python loads, so that both use one library)
+// ---------------------------------------------------------------------------
+#define BS_FUNCS(F)                                                                                              \
+    F(bs_last_error) F(bs_compress_workspace_bytes) F(bs_compress) F(bs_compress_relu) F(bs_compress_packed)     \
+    F(bs_compress_act) F(bs_amax) F(bs_amax_relu) F(bs_amax_bias_relu) F(bs_quantize_e4m3fn)                     \
+    F(bs_quantize_e4m3fn_t) F(bs_transpose_u8) F(bs_widen_e4m3fn) F(bs_decompress) F(bs_decompress_packed)       \
+    F(bs_relu_grad) F(bs_relu2_grad) F(bs_relu2_grad_packed) F(bs_grad_sums_workspace_bytes) F(bs_act_grad_sums) \
+    F(bs_col_sum_workspace_bytes) F(bs_col_sum) F(bs_gemm_compressed_b_workspace_bytes) F(bs_gemm_compressed_b)  \
+    F(bs_gemm_compressed_b_packed_workspace_bytes) F(bs_gemm_compressed_b_packed)                                \
+    F(bs_gemm_compressed_b_fp8_workspace_bytes) F(bs_gemm_compressed_b_fp8) F(bs_gemm_compressed_b_fp8_packed)   \
+    F(bs_workspace_amax_slot)
+struct Lib {
+#define F(name) decltype(&::name) name = nullptr;
+    BS_FUNCS(F)
+#undef F
+} L;
+
+void init(const std::string& path)
+{
+    void* h = dlopen(path.c_str(), RTLD_NOW);
+    TORCH_CHECK(h != nullptr, "bitsparse_amd: ", dlerror());
+#define F(name)                                                        \
+    L.name = reinterpret_cast<decltype(&::name)>(dlsym(h, #name));     \
+    TORCH_CHECK(L.name != nullptr, "bitsparse_amd: " #name " missing");
+    BS_FUNCS(F)
+#undef F
+}
+
+void check(int rc, const char* what)
+{
+    if (rc == BS_OK) return;
+    const char* msg = L.bs_last_error();
+    if (rc == BS_ERR_INVALID) TORCH_CHECK_VALUE(false, what, ": ", msg);
+    TORCH_CHECK(false, what, " failed (", rc, "): ", msg);
+}
+
+void* stream_of(const Tensor& t)
+{
+    return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.get_device()).stream();
+}
+
+template <typename T>
+T* ptr(const Tensor& t)
+{
+    return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr;
+}
+void* raw(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+int dtype_code(at::ScalarType t)
+{
+    switch (t) {
+    case at::kBFloat16: return 0;
+    case at::kFloat8_e4m3fn: return 1;
+    case at::kFloat8_e5m2: return 2;
+    default: TORCH_CHECK_TYPE(false, "BitsparseTensor supports bfloat16 and FP8 (e4m3fn/e5m2) values");
+    }
+}
+
+Tensor empty(at::IntArrayRef shape, const Tensor& like, at::ScalarType t)
+{
+    return at::empty(shape, like.options().dtype(t));
+}
+
+// ---------------------------------------------------------------------------
+// per-(device, stream) workspace of the single-pass compress and the amax
+// ---------------------------------------------------------------------------
+constexpr int64_t kEpochLimit = (int64_t(1) << 30) - 1;
+
+// Zero-initialised device scratch with an epoch counter.  Each compress / amax
+// call takes a fresh epoch; status words written under older epochs are
+// ignored by the kernels, so the buffer never needs clearing between calls.
+// When the counter wraps the buffer is zeroed again.  `mu` is held while a
+// sequence that passes an amax through the workspace is enqueued (backward
+// threads run without the interpreter lock).
+struct Workspace {
+    explicit Workspace(c10::Device d) : device(d), buf(at::zeros({0}, at::device(d).dtype(at::kByte))) {}
+    c10::Device device;
+    Tensor buf;
+    int64_t epoch = 0;
+    std::recursive_mutex mu;
+
+    void ensure(int64_t nbytes)
+    {
+        std::lock_guard<std::recursive_mutex> g(mu);
+        if (buf.numel() >= nbytes) return;
+        // grow geometrically; the old contents (amax slot, status words of
+        // earlier epochs) move along and the new tail is zero, so epochs
+        // already handed out stay meaningful
+        const int64_t size = std::max<int64_t>({nbytes, 2 * buf.numel(), 1 << 16});
+        Tensor n = at::zeros({size}, buf.options());
+        if (buf.numel()) n.narrow(0, 0, buf.numel()).copy_(buf);
+        buf = n;
+    }
+    // `reserve`: how many epochs the caller's sequence takes in total (the
+    // amax of a quantizing compress reserves 2), so that the wrap -- which
+    // zeroes the buffer, amax slot included -- never falls inside it
+    int64_t next_epoch(int64_t reserve)
+    {
+        std::lock_guard<std::recursive_mutex> g(mu);
+        if (epoch + reserve > kEpochLimit) {
+            buf.zero_();
+            epoch = 0;
+        }
+        return ++epoch;
+    }
+    int64_t nbytes() const { return buf.numel(); }
+    const uint64_t* slot() const { return L.bs_workspace_amax_slot(buf.data_ptr(), nbytes()); }
+    int64_t fallback_count() const
+    {
+        if (buf.numel() < 12) return 0;
+        return buf.narrow(0, 8, 4).view(at::kInt).item<int>();
+    }
+};
+
+std::shared_ptr<Workspace> workspace(int dev)
+{
+    static std::mutex mu;
+    static auto* all = new std::map<std::pair<int, void*>, std::shared_ptr<Workspace>>();   // (freed by the process)
+    if (dev < 0) dev = c10::hip::current_device();
+    void* st = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev).stream();
+    std::lock_guard<std::mutex> g(mu);
+    auto& w = (*all)[{dev, st}];
+    if (!w) w = std::make_shared<Workspace>(c10::Device(c10::kCUDA, dev));
+    return w;
+}
+Workspace& ws_of(const Tensor& t) { return *workspace(t.get_device()); }
+
+using Lock = std::lock_guard<std::recursive_mutex>;
+
+// amax of a bf16 tensor (of its relu, of relu(x + bias)) under a fresh epoch
+int64_t amax(const Tensor& x, bool relu, const Tensor& bias, Workspace& w, int64_t reserve = 2)
+{
+    w.ensure(256);
+    const int64_t e = w.next_epoch(reserve);
+    void* st = stream_of(x);
+    if (bias.defined())
+        check(L.bs_amax_bias_relu(x.data_ptr(), x.size(0), x.size(1), bias.data_ptr(), w.buf.data_ptr(), w.nbytes(), e,
+                                  st), "bs_amax_bias_relu");
+    else
+        check((relu ? L.bs_amax_relu : L.bs_amax)(x.data_ptr(), x.numel(), w.buf.data_ptr(), w.nbytes(), e, st),
+              "bs_amax");
+    return e;
+}
+
+// ---------------------------------------------------------------------------
+// codec
+// ---------------------------------------------------------------------------
+// The TensorBuffer's cursor for one compress.  No offset: the buffer was just
+// reset, the values start at 0 (no tensor was filled for it) and the kernel
+// writes the start that the BitsparseTensor keeps.  In place: the start is a
+// snapshot and the cursor tensor itself advances.
+struct Cursor {
+    Tensor in, next, start, start_out;
+    Cursor(const std::optional<Tensor>& offset, bool in_place, bool packed, const Tensor& like)
+    {
+        if (offset) in = in_place ? offset->clone() : *offset;
+        next = in_place ? *offset : empty({1}, like, at::kLong);
+        start = in;
+        // (a packed run starts at the cursor rounded up)
+        if (packed || !offset) start = start_out = empty({1}, like, at::kLong);
+    }
+};
+
+int64_t tiles(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 63) / 64); }
+
+// (bitmask, prefix, start of the values, advanced cursor, dense codes, scale):
+// bs_compress / bs_compress_packed of a contiguous dense into a TensorBuffer's
+// storage; quantize: of a bf16 dense's e4m3fn codes, with its amax first
+std::tuple<Tensor, Tensor, Tensor, Tensor, std::optional<Tensor>, std::optional<Tensor>>
+compress(const Tensor& dense, const Tensor& vals, const std::optional<Tensor>& offset, bool in_place,
+         const Tensor& err, bool packed, bool quantize, bool dense_out)
+{
+    const c10::DeviceGuard guard(dense.device());
+    const int64_t M = dense.size(0), N = dense.size(1), T = tiles(M, N);
+    Workspace& w = ws_of(dense);
+    Lock lock(w.mu);
+    Tensor q, scale;
+    int64_t amax_epoch = 0;
+    if (quantize) {
+        amax_epoch = amax(dense, false, Tensor(), w);
+        if (dense_out) q = empty({M, N}, dense, at::kFloat8_e4m3fn);
+        scale = empty({}, dense, at::kFloat);
+    }
+    Tensor bitmask = empty({T * 512}, dense, at::kByte), prefix = empty({T + 1}, dense, at::kUInt32);
+    Cursor c(offset, in_place, packed, dense);
+    w.ensure(L.bs_compress_workspace_bytes(M, N));
+    const int64_t epoch = w.next_epoch(1);
+    const uint64_t* slot = quantize ? w.slot() : nullptr;
+    if (packed) {
+        check(L.bs_compress_packed(dense.data_ptr(), dtype_code(dense.scalar_type()), M, N, quantize, slot, amax_epoch,
+                                   ptr<float>(scale), raw(q), ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix),
+                                   vals.data_ptr(), vals.numel(), ptr<int64_t>(c.in), ptr<int64_t>(c.next),
+                                   ptr<int64_t>(c.start_out), ptr<int32_t>(err), w.buf.data_ptr(), w.nbytes(), epoch, 0,
+                                   nullptr, stream_of(dense)), "bs_compress_packed");
+    } else {
+        check(L.bs_compress(dense.data_ptr(), dtype_code(dense.scalar_type()), M, N, quantize, slot, amax_epoch,
+                            ptr<float>(scale), raw(q), ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix), vals.data_ptr(),
+                            vals.numel(), ptr<int64_t>(c.in), 0, ptr<int64_t>(c.next), ptr<int64_t>(c.start_out), 1,
+                            ptr<int32_t>(err), w.buf.data_ptr(), w.nbytes(), epoch, stream_of(dense)), "bs_compress");
+    }
+    return {bitmask, prefix, c.start, c.next, q.defined() ? std::optional<Tensor>(q) : std::nullopt,
+            scale.defined() ? std::optional<Tensor>(scale) : std::nullopt};
+}
+
+void decompress(const Tensor& vals, at::ScalarType stored, bool packed, const Tensor& bitmask, const Tensor& prefix,
+                const Tensor& offset, const Tensor& out, int64_t first_m_tile, int64_t grid_n, int64_t K,
+                int64_t batch_rows, int64_t num_tiles, bool square, double k, const std::optional<Tensor>& scale)
+{
+    const c10::DeviceGuard guard(out.device());
+    check((packed ? L.bs_decompress_packed : L.bs_decompress)(
+              vals.data_ptr(), dtype_code(stored), vals.numel(), ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix),
+              ptr<int64_t>(offset), out.data_ptr(), first_m_tile, grid_n, K, batch_rows, num_tiles, square, (float)k,
+              scale ? ptr<float>(*scale) : nullptr, stream_of(out)), "bs_decompress");
+}
+
+// ---------------------------------------------------------------------------
+// fp8 operands
+// ---------------------------------------------------------------------------
+struct Fp8 {
+    Tensor codes, scale;
+};
+
+Fp8 quantize_rows(const Tensor& x, int64_t amax_epoch, Workspace& w)
+{
+    Fp8 o{empty(x.sizes(), x, at::kFloat8_e4m3fn), empty({}, x, at::kFloat)};
+    check(L.bs_quantize_e4m3fn(x.data_ptr(), x.numel(), o.codes.data_ptr(), ptr<float>(o.scale), w.buf.data_ptr(),
+                               w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn");
+    return o;
+}
+
+// to_fp8 of a row-major matrix
+Fp8 to_fp8(const Tensor& x, Workspace& w)
+{
+    const Tensor c = x.contiguous();
+    Lock lock(w.mu);
+    return quantize_rows(c, amax(c, false, Tensor(), w), w);
+}
+
+// codes of x.T as a new row-major tensor (and, `rows`, those of x)
+std::pair<Tensor, Fp8> quantize_t(const Tensor& x, int64_t amax_epoch, bool rows, Workspace& w)
+{
+    const int64_t R = x.size(0), C = x.size(1);
+    Tensor q;
+    if (rows) q = empty({R, C}, x, at::kFloat8_e4m3fn);
+    Fp8 t{empty({C, R}, x, at::kFloat8_e4m3fn), empty({}, x, at::kFloat)};
+    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), R, C, raw(q), t.codes.data_ptr(), ptr<float>(t.scale), w.buf.data_ptr(),
+                                 w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn_t");
+    return {q, t};
+}
+
+// an operand multiplied from the right: column-major codes
+Fp8 right_operand(const Tensor& x, Workspace& w)
+{
+    const Tensor c = x.contiguous();
+    Lock lock(w.mu);
+    Fp8 t = quantize_t(c, amax(c, false, Tensor(), w), false, w).second;
+    return {t.codes.t(), t.scale};
+}
+
+Tensor fp8_mm(const Fp8& a, const Fp8& b, at::ScalarType out)
+{
+    return at::_scaled_mm(a.codes, b.codes, a.scale, b.scale, std::nullopt, std::nullopt, out, false);
+}
+
+// a gradient in e4m3fn widened to bf16 (exact)
+Tensor widened(const Tensor& g)
+{
+    if (g.scalar_type() != at::kFloat8_e4m3fn) return g;
+    Tensor o = empty(g.sizes(), g, at::kBFloat16);
+    check(L.bs_widen_e4m3fn(g.data_ptr(), g.numel(), o.data_ptr(), stream_of(g)), "bs_widen_e4m3fn");
+    return o;
+}
+
+// ---------------------------------------------------------------------------
+// the MLP block
+// ---------------------------------------------------------------------------
+// the compressed activation r of a block
+struct Held {
+    Tensor vals, bitmask, prefix, start, scale;
+    int64_t M, N;
+    bool packed, fp8, square;
+    double k;
+};
+
+// C = A @ op(B), B compressed [K, N]: A row-major (a_layout 1) or A.T
+// row-major (0) in `a` with row stride lda; a_scale: A is e4m3fn
+Tensor gemm_compressed(const Tensor& a, int64_t M, int64_t K, int64_t lda, int64_t a_layout,
+                       const std::optional<Tensor>& a_scale, const Tensor& vals, at::ScalarType stored, bool packed,
+                       const Tensor& bitmask, const Tensor& prefix, const Tensor& start, int64_t N, bool square,
+                       double k, const std::optional<Tensor>& scale, const std::optional<Tensor>& b_scale_out)
+{
+    const c10::DeviceGuard guard(a.device());
+    Tensor C = empty({M, N}, a, at::kBFloat16);
+    const int64_t need =
+        a_scale ? L.bs_gemm_compressed_b_fp8_workspace_bytes(M, N, K, a_layout, square || packed)
+                : (packed ? L.bs_gemm_compressed_b_packed_workspace_bytes : L.bs_gemm_compressed_b_workspace_bytes)(
+                      M, N, K, a_layout);
+    const Tensor ws = empty({std::max<int64_t>(need, 0)}, a, at::kByte);
+    float* const bs = scale ? ptr<float>(*scale) : nullptr;
+    if (a_scale)
+        check((packed ? L.bs_gemm_compressed_b_fp8_packed : L.bs_gemm_compressed_b_fp8)(
+                  a.data_ptr(), ptr<float>(*a_scale), M, K, lda, a_layout, vals.data_ptr(), dtype_code(stored),
+                  vals.numel(), ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix), ptr<int64_t>(start), N, square, (float)k,
+                  bs, C.data_ptr(), b_scale_out ? ptr<float>(*b_scale_out) : nullptr, ws.data_ptr(), need,
+                  stream_of(a)), "bs_gemm_compressed_b_fp8");
+    else
+        check((packed ? L.bs_gemm_compressed_b_packed : L.bs_gemm_compressed_b)(
+                  a.data_ptr(), M, K, lda, a_layout, vals.data_ptr(), dtype_code(stored), vals.numel(),
+                  ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix), ptr<int64_t>(start), N, square, (float)k, bs,
+                  C.data_ptr(), ws.data_ptr(), need, stream_of(a)), "bs_gemm_compressed_b");
+    return C;
+}
+
+// dW2 = g^T act(r)
+Tensor down_weight_grad(const Tensor& g, const Tensor& g_scale, const Held& h)
+{
+    Tensor a = g;
+    if (!h.fp8 && (a.stride(1) != 1 || a.stride(0) % 8 != 0 || (reinterpret_cast<uintptr_t>(a.data_ptr()) & 15))) {
+        const int64_t M = g.size(1);
+        a = at::zeros({h.M, (M + 7) / 8 * 8}, g.options());
+        a.narrow(1, 0, M).copy_(g);
+    }
+    return gemm_compressed(a, g.size(1), h.M, a.stride(0), 0, h.fp8 ? std::optional<Tensor>(g_scale) : std::nullopt,
+                           h.vals, h.fp8 ? at::kFloat8_e4m3fn : at::kBFloat16, h.packed, h.bitmask, h.prefix, h.start,
+                           h.N, h.square, h.k, h.fp8 ? std::optional<Tensor>(h.scale) : std::nullopt, std::nullopt);
+}
+
+Tensor col_sum(const Tensor& g)
+{
+    // a graph of this gradient (create_graph), or a layout the kernel does not
+    // take: torch's own sum
+    if (at::GradMode::is_enabled() || !g.is_contiguous() || g.size(1) % 8 != 0 || g.numel() == 0 ||
+        (reinterpret_cast<uintptr_t>(g.data_ptr()) & 15) || g.numel() >= (int64_t(1) << 31))
+        return g.sum(0);
+    const int64_t R = g.size(0), C = g.size(1), need = L.bs_col_sum_workspace_bytes(R, C);
+    Tensor out = empty({C}, g, at::kBFloat16), part = empty({need}, g, at::kByte);
+    check(L.bs_col_sum(g.data_ptr(), R, C, out.data_ptr(), part.data_ptr(), need, stream_of(g)), "bs_col_sum");
+    return out;
+}
+
+// y = act(x @ W1.T + b1) @ W2.T + b2 with act(z) = relu(z) or k relu(z)^2 saved
+// compressed: the products, quantizations and kernels of the separate nodes
+// (matmul, the bias adds, ReluLinear / Relu2Linear), with their roundings.
+// What one node adds is what crosses them: the bias, square and codes of the
+// down-projection's operand ride on the compress pass, the bias gradient and
+// the amax on the activation's gradient, and the fp8 operands of the backward
+// products are quantized into the layout those take.  The caller (layers.py)
+// has checked the operands.
+// -> (y, bitmask, prefix, start of the values, advanced cursor, scale)
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, std::optional<Tensor>>
+block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bias1, const Tensor& W2,
+              const std::optional<Tensor>& bias2, const Tensor& vals, const std::optional<Tensor>& offset,
+              const Tensor& err, bool in_place, bool packed, bool fp8, bool square, double k)
+{
+    const c10::DeviceGuard guard(x.device());
+    const Tensor b1 = bias1.value_or(Tensor()), b2 = bias2.value_or(Tensor());
+    const int64_t M = x.size(0), N = W1.size(0), T = tiles(M, N);
+    Workspace& w = ws_of(x);
+    Tensor z;
+    if (fp8) {
+        const Fp8 a = to_fp8(x, w), b = to_fp8(W1, w);
+        z = fp8_mm(a, {b.codes.t(), b.scale}, at::kBFloat16);
+    } else {
+        z = at::mm(x, W1.t());
+    }
+    Tensor operand, operand_scale, codes, h_out, scale;
+    Tensor bitmask = empty({T * 512}, x, at::kByte), prefix = empty({T + 1}, x, at::kUInt32);
+    const Cursor c(offset, in_place, packed, x);
+    {
+        Lock lock(w.mu);
+        int64_t amax_epoch = 0;
+        if (fp8) {
+            amax_epoch = amax(z, true, b1, w);
+            scale = empty({}, x, at::kFloat);
+            operand_scale = square ? empty({}, x, at::kFloat) : scale;
+            operand = codes = empty({M, N}, x, at::kFloat8_e4m3fn);
+        } else {
+            // over z where that leaves a recount of z (the look-back's fallback) right
+            operand = h_out = b1.defined() || square ? at::empty_like(z) : z;
+        }
+        w.ensure(L.bs_compress_workspace_bytes(M, N));
+        const int64_t epoch = w.next_epoch(1);
+        check(L.bs_compress_act(z.data_ptr(), raw(b1), M, N, square, (float)k, fp8, fp8 ? w.slot() : nullptr,
+                                amax_epoch, ptr<float>(scale), raw(codes),
+                                square && fp8 ? ptr<float>(operand_scale) : nullptr, raw(h_out), ptr<uint8_t>(bitmask),
+                                ptr<uint32_t>(prefix), vals.data_ptr(), vals.numel(), packed, ptr<int64_t>(c.in),
+                                ptr<int64_t>(c.next), ptr<int64_t>(c.start_out), ptr<int32_t>(err), w.buf.data_ptr(),
+                                w.nbytes(), epoch, stream_of(x)), "bs_compress_act");
+    }
+    Tensor y;
+    if (fp8) {
+        const Fp8 b = to_fp8(W2, w);
+        y = fp8_mm({operand, operand_scale}, {b.codes.t(), b.scale}, at::kBFloat16);
+    } else {
+        y = at::mm(operand, W2.t());
+    }
+    if (b2.defined()) y.add_(b2);
+    return {y, bitmask, prefix, c.start, c.next, scale.defined() ? std::optional<Tensor>(scale) : std::nullopt};
+}
+
+// (dx, dW1, db1, dW2, db2), each where `need` asks for it
+std::vector<std::optional<Tensor>>
+block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const Tensor& vals,
+               const Tensor& bitmask, const Tensor& prefix, const Tensor& start, const std::optional<Tensor>& scale,
+               bool packed, bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
+               const std::vector<bool>& need)
+{
+    const c10::DeviceGuard guard(x.device());
+    const Held h{vals, bitmask, prefix, start, scale.value_or(Tensor()), x.size(0), W1.size(0), packed, fp8, square, k};
+    const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3], need_b2 = need[4];
+    std::vector<std::optional<Tensor>> out(5);
+    Workspace& w = ws_of(x);
+    if (need_b2) out[4] = col_sum(g);
+    Fp8 g8;
+    if (fp8) g8 = to_fp8(g, w);
+    if (need_W2) out[3] = down_weight_grad(fp8 ? g8.codes : g, g8.scale, h);
+    if (!(need_x || need_W1 || need_b1)) return out;
+    Tensor dz = fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
+    const bool want8 = fp8 && (need_x || need_W1);
+    const bool sums = need_b1 && !at::GradMode::is_enabled();
+    Fp8 z8, zt8;
+    if (sums || want8) {
+        Lock lock(w.mu);
+        int64_t epoch = 0;
+        if (want8) {
+            w.ensure(256);
+            epoch = w.next_epoch(2);
+        }
+        Tensor db1;
+        if (sums) out[2] = db1 = empty({h.N}, x, at::kBFloat16);
+        const int64_t bytes = L.bs_grad_sums_workspace_bytes(h.M, h.N);
+        const Tensor part = empty({bytes}, x, at::kByte);
+        check(L.bs_act_grad_sums(dz.data_ptr(), h.M, h.N, square, vals.data_ptr(), fp8 ? 1 : 0, vals.numel(), packed,
+                                 ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix), ptr<int64_t>(start), (float)k,
+                                 ptr<float>(h.scale), raw(db1), want8 ? w.buf.data_ptr() : nullptr, epoch,
+                                 part.data_ptr(), bytes, stream_of(x)), "bs_act_grad_sums");
+        if (want8 && need_W1) {
+            const auto [q, t] = quantize_t(dz, epoch, need_x, w);
+            z8 = {q, t.scale};
+            zt8 = t;
+        } else if (want8) {
+            z8 = quantize_rows(dz, epoch, w);
+        }
+    } else if (square) {
+        check((packed ? L.bs_relu2_grad_packed : L.bs_relu2_grad)(
+                  dz.data_ptr(), h.M, h.N, vals.data_ptr(), fp8 ? 1 : 0, vals.numel(), ptr<uint8_t>(bitmask),
+                  ptr<uint32_t>(prefix), ptr<int64_t>(start), (float)k, ptr<float>(h.scale), stream_of(x)),
+              "bs_relu2_grad");
+    } else {
+        check(L.bs_relu_grad(dz.data_ptr(), h.M, h.N, ptr<uint8_t>(bitmask), stream_of(x)), "bs_relu_grad");
+    }
+    if (need_b1 && !sums) out[2] = col_sum(dz);
+    if (fp8) {
+        const at::ScalarType gd = grad_dtype.value_or(at::kFloat8_e4m3fn);
+        if (need_x) out[0] = widened(fp8_mm(z8, right_operand(W1, w), gd));
+        if (need_W1) out[1] = widened(fp8_mm(zt8, right_operand(x, w), gd));
+    } else {
+        if (need_x) out[0] = at::mm(dz, W1);
+        if (need_W1) out[1] = at::mm(dz.t(), x);      // W1's own layout, as autograd forms it
+    }
+    return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
+{
+    m.def("init", &init);
+    py::class_<Workspace, std::shared_ptr<Workspace>>(m, "Workspace")
+        .def_readonly("buf", &Workspace::buf)
+        .def_readwrite("epoch", &Workspace::epoch)
+        .def_property_readonly("nbytes", &Workspace::nbytes)
+        .def("ensure", &Workspace::ensure)
+        .def("next_epoch", &Workspace::next_epoch, py::arg("reserve") = 1)
+        .def("amax_slot_ptr", [](const Workspace& w) { return reinterpret_cast<uintptr_t>(w.slot()); })
+        .def("fallback_count", &Workspace::fallback_count);
+    m.def("workspace", &workspace);
+    m.def("compress", &compress);
+    m.def("decompress", &decompress);
+    m.def("gemm_compressed", &gemm_compressed);
+    m.def("block_forward", &block_forward);
+    m.def("block_backward", &block_backward);
+}

@@ -69,17 +69,6 @@ def as_fp8_operand(x: Tensor, scale: Tensor | None) -> Fp8Operand:
     return Fp8Operand(x, scale)
 
 
-def as_right_operand(x: Tensor) -> Fp8Operand:
-    """``to_fp8`` of a bf16 matrix that ``fp8_gemm`` multiplies from the right:
-    its codes are laid out column-major by the quantizer itself where it can
-    (``fp8_gemm`` would transpose them)."""
-    from .src import hip_operators as ops
-    if not ops.quantize_t_supported(x):
-        return as_fp8_operand(x, None)
-    _, qt, scale = ops.quantize_e4m3fn_t(x, ops.amax_into_workspace(x), False)
-    return Fp8Operand(qt.t(), scale)
-
-
 def fp8_gemm(a: Fp8Operand, b: Fp8Operand, out_dtype: torch.dtype) -> Tensor:
     """(a.codes * a.scale) @ (b.codes * b.scale) on hipBLASLt, fp32
     accumulation, rounded once to ``out_dtype`` (bf16, fp32 or an fp8 dtype,
@@ -150,22 +139,6 @@ class MatmulFp8(Function):
             else:
                 grad_b = _as_input_dtype(fp8_gemm(opa.T, g, _grad_dtype(ctx.grad_dtypes[1])), ctx.in_dtypes[1])
         return grad_a, grad_b, None, None
-
-
-def linear_fp8_backward(x: Tensor, W: Tensor, g: Fp8Operand | None, gt: Fp8Operand | None, need_x: bool,
-                        need_W: bool) -> tuple[Tensor | None, Tensor | None]:
-    """(grad of x, grad of W) of z = matmul(x, W.T, True) for bf16 x and W
-    and z's gradient in fp8, g row-major and gt its transpose:
-    ``MatmulFp8``'s backward with its operands quantized again, W's gradient
-    in W's own layout."""
-    grad_x = grad_W = None
-    if need_x:
-        w = as_right_operand(W)
-        grad_x = _as_input_dtype(fp8_gemm(g, w, _grad_dtype(w.codes.dtype)), x.dtype)
-    if need_W:
-        a = as_right_operand(x)
-        grad_W = _as_input_dtype(fp8_gemm(gt, a, _grad_dtype(a.codes.dtype)), W.dtype)
-    return grad_x, grad_W
 
 
 def _as_input_dtype(grad: Tensor, in_dtype: torch.dtype) -> Tensor:

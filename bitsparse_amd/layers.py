@@ -10,21 +10,22 @@ bitmask (HIP mask / ReLU^2-gradient kernels).
 """
 from __future__ import annotations
 
+import math
+
 import torch
 from torch import Tensor
 from torch.autograd import Function, forward_ad
 
 from . import config
 from .bitsparse import BitsparseTensor, TensorBuffer
-from .config import RELU2_SCALE
-from .fp8 import (Fp8Operand, as_fp8_operand, as_right_operand, fp8_gemm, is_fp8, linear_fp8_backward, matmul,
-                  to_fp8)
-from .src.functions import (activate_and_compress, activate_ok, fused_linear_relu_ok, linear_relu_and_compress,
-                            relu2_and_compress, relu2_fused_ok, relu2_quantize_and_compress, relu_and_compress,
+from .config import BLOCK_M, BLOCK_N, RELU2_SCALE
+from .fp8 import is_fp8, matmul, to_fp8
+from ._lib import native
+from .src import sparse_matmul
+from .src.functions import (fused_linear_relu_ok, linear_relu_and_compress, relu2_and_compress,
+                            relu2_fused_ok, relu2_quantize_and_compress, relu_and_compress,
                             relu_quantize_and_compress)
-from .src.hip_operators import (act_grad_sums_, act_grad_sums_supported, col_sum, col_sum_supported,
-                                mask_with_bitmask_, quantize_e4m3fn, quantize_e4m3fn_t, quantize_t_supported,
-                                relu2_grad_sparse_, relu2_square_amax_)
+from .src.hip_operators import mask_with_bitmask_, quantize_e4m3fn, relu2_grad_sparse_, relu2_square_amax_
 from .src.sparse_matmul import AspB, AspRelu2B
 
 # FFNRelu / FFNRelu2 with bf16 storage into a TensorBuffer run the up-projection
@@ -95,8 +96,8 @@ class FFNRelu:
         bs_dims = x.shape[:-1]
         x = x.reshape(-1, x.shape[-1])
 
-        if _block_ok(x, W1, W2, b1, b2):
-            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, pack_sbit, dtype, False)
+        if _block_ok(x, W1, W2, b1, b2, sparse_data, pack_sbit, dtype):
+            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, is_fp8(dtype), False)
             return y.reshape(*bs_dims, y.shape[-1])
         if not is_fp8(dtype) and not pack_sbit and USE_FUSED_UP and fused_linear_relu_ok(x, W1, b1, sparse_data):
             y = _UpReluLinear.apply(x, W1, b1, W2, sparse_data, False)
@@ -190,8 +191,8 @@ class FFNRelu2:
               storage_dtype: torch.dtype = torch.bfloat16):
         bs_dims = x.shape[:-1]
         x = x.reshape(-1, x.shape[-1])
-        if _block_ok(x, W1, W2, b1, b2):
-            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, pack_sbit, storage_dtype, True)
+        if _block_ok(x, W1, W2, b1, b2, sparse_data, pack_sbit, storage_dtype):
+            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, is_fp8(storage_dtype), True)
             return y.reshape(*bs_dims, y.shape[-1])
         if (not is_fp8(storage_dtype) and not pack_sbit and USE_FUSED_UP
                 and fused_linear_relu_ok(x, W1, b1, sparse_data)):
@@ -208,59 +209,64 @@ class FFNRelu2:
 
 
 # ------------------------------------------------------------
-# the whole block as one autograd node
+# the whole block as one autograd node (its body: csrc/native.cpp)
 # ------------------------------------------------------------
 def _plain(t: Tensor) -> bool:
     return type(t) in (Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.bfloat16
 
 
-def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor | None) -> bool:
-    """The MLP block runs as one node (``_FFNBlock``): plain bf16 matrices on
-    the GPU and bias rows, outside autocast, tracing, forward-mode AD and the
-    options that choose another path.  Everything else takes the layers'
-    separate nodes, with their errors."""
-    if not (_plain(x) and _plain(W1) and _plain(W2)) or USE_FUSED_UP or config.CACHE_FP8_MATMUl:
+def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor | None,
+              sparse_data: TensorBuffer | None, pack_sbit: bool, dtype: torch.dtype) -> bool:
+    """The MLP block runs as one node (``_FFNBlock``): plain bf16 matrices and bias
+    rows on one GPU in the shapes and alignments its kernels take, a
+    TensorBuffer of the stored type, outside autocast, tracing, forward-mode
+    AD and the options that choose another path.  Everything else takes the
+    layers' separate nodes, with their errors."""
+    if sparse_data is None or not (_plain(x) and _plain(W1) and _plain(W2)):
         return False
-    if x.dim() != 2 or W1.dim() != 2 or W2.dim() != 2 or 0 in x.shape or 0 in W1.shape or 0 in W2.shape:
+    if USE_FUSED_UP or config.CACHE_FP8_MATMUl or not sparse_matmul.USE_LDS_GEMM or not math.isfinite(RELU2_SCALE):
         return False
-    if x.shape[1] != W1.shape[1] or W1.shape[0] != W2.shape[1]:
+    if x.dim() != 2 or W1.dim() != 2 or W2.dim() != 2 or not (W1.is_contiguous() and W2.is_contiguous()):
         return False
-    if not (W1.is_contiguous() and W2.is_contiguous() and x.device == W1.device == W2.device):
+    T, D = x.shape
+    H, O = W1.shape[0], W2.shape[0]
+    if W1.shape[1] != D or W2.shape[1] != H or 0 in (T, D, H, O) or H % 8 or T * H >= 2 ** 31:
         return False
-    for b, n in ((b1, W1.shape[0]), (b2, W2.shape[0])):
-        if b is not None and not (_plain(b) and b.shape == (n,) and b.is_contiguous() and b.device == x.device):
+    fp8 = is_fp8(dtype)
+    if fp8 and (T % 16 or D % 16 or H % 16 or O % 16 or T * D >= 2 ** 31 or D * H >= 2 ** 31 or H * O >= 2 ** 31
+                or any(t.data_ptr() % 16 for t in (x, W1, W2))):
+        return False
+    for b, n in ((b1, H), (b2, O)):
+        if b is not None and not (_plain(b) and b.shape == (n,) and b.is_contiguous() and b.data_ptr() % 16 == 0):
             return False
+    buf = sparse_data.vals
+    stored = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    if (bool(sparse_data.pack_sbit) != bool(pack_sbit) or sparse_data.dtype != stored
+            or (not pack_sbit and buf.dtype != stored) or buf.data_ptr() % (4 if pack_sbit else 16)):
+        return False
+    if not (x.device == W1.device == W2.device == buf.device) or any(
+            b is not None and b.device != x.device for b in (b1, b2)):
+        return False
     return (not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
             and not torch.compiler.is_compiling())
 
 
 class _FFNBlock(Function):
     """y = act(x @ W1.T + b1) @ W2.T + b2 with act(z) = relu(z) or
-    k * relu(z)^2 saved compressed: the products, quantizations and kernels of
-    the nodes it stands for (``matmul``, the bias adds, ``ReluLinear`` /
-    ``Relu2Linear``), in their order and with their roundings.  What the one
-    node adds is what crosses them: bias gradients are column sums of the
-    gradients at hand."""
+    k * relu(z)^2 saved compressed, for operands ``_block_ok`` accepts."""
 
     @staticmethod
-    def forward(ctx, x, W1, b1, W2, b2, sparse_data, pack_sbit, dtype, square):
-        fp8 = is_fp8(dtype)
-        ctx.save_for_backward(x, W1, W2)
+    def forward(ctx, x, W1, b1, W2, b2, buf, fp8, square):
+        y, bitmask, prefix, start, buf._offset, scale = native().block_forward(
+            x, W1, b1, W2, b2, buf.vals, buf._offset, buf.err_flags, buf.inplace_offset, buf.pack_sbit, fp8, square,
+            float(RELU2_SCALE))
+        M, N = x.shape[0], W1.shape[0]
+        ctx.h_sparse = BitsparseTensor(buf.vals, bitmask, prefix, (M, N), torch.float8_e4m3fn if fp8 else torch.bfloat16,
+                                       (M + BLOCK_M - 1) // BLOCK_M, (N + BLOCK_N - 1) // BLOCK_N, BLOCK_M, BLOCK_N,
+                                       scale=scale, vals_offset=start, pack_sbit=buf.pack_sbit)
         ctx.fp8, ctx.square = fp8, square
-        if fp8:
-            z = fp8_gemm(as_fp8_operand(x, None), as_fp8_operand(W1.T, None), torch.bfloat16)
-        else:
-            z = x @ W1.T
-        if activate_ok(z, b1, sparse_data, RELU2_SCALE):
-            h, scale, ctx.h_sparse = activate_and_compress(z, b1, sparse_data, pack_sbit, fp8, square)
-            y = (fp8_gemm(Fp8Operand(h, scale), as_fp8_operand(W2.T, None), torch.bfloat16) if fp8
-                 else h @ W2.T)
-        else:
-            if b1 is not None:
-                z = z + b1
-            down = Relu2Linear if square else ReluLinear
-            y, ctx.h_sparse = down.activate_and_project(z, W2, sparse_data, pack_sbit, dtype)
-        return y if b2 is None else y + b2
+        ctx.save_for_backward(x, W1, W2)
+        return y
 
     @staticmethod
     @torch.compiler.disable
@@ -268,55 +274,10 @@ class _FFNBlock(Function):
         x, W1, W2 = ctx.saved_tensors
         h: BitsparseTensor = ctx.h_sparse
         ctx.h_sparse = None
-        need_x, need_W1, need_b1, need_W2, need_b2 = ctx.needs_input_grad[:5]
-        grad_x = grad_W1 = grad_b1 = grad_W2 = grad_b2 = None
-        if need_b2:
-            grad_b2 = _col_sum(grad_output)
-        scale = None
-        if ctx.fp8:
-            grad_output, scale = to_fp8(grad_output)
-        if need_W2:
-            product = AspRelu2B if ctx.square else AspB
-            grad_W2 = product(grad_output.T, h, A_scale=scale)
-        if need_x or need_W1 or need_b1:
-            if ctx.fp8:
-                grad_h = fp8_gemm(Fp8Operand(grad_output, scale), as_right_operand(W2), torch.bfloat16)
-            else:
-                grad_h = grad_output @ W2
-            need_g = ctx.fp8 and (need_x or need_W1)
-            g8 = gt8 = None
-            if (need_b1 or need_g) and not torch.is_grad_enabled() and act_grad_sums_supported(grad_h, h, ctx.square):
-                grad_z = grad_h
-                grad_b1, epoch = act_grad_sums_(grad_z, h, ctx.square, need_b1, need_g)
-                if need_g:
-                    g8, gt8 = _quantized_both_ways(grad_z, epoch, need_x, need_W1)
-            else:
-                grad_z = relu2_grad_sparse_(grad_h, h) if ctx.square else mask_with_bitmask_(grad_h, h)
-                if need_b1:
-                    grad_b1 = _col_sum(grad_z)
-                if need_g:
-                    g8 = as_fp8_operand(grad_z, None)
-                    gt8 = g8.T
-            if ctx.fp8:
-                grad_x, grad_W1 = linear_fp8_backward(x, W1, g8, gt8, need_x, need_W1)
-            else:
-                grad_x = grad_z.mm(W1) if need_x else None
-                grad_W1 = grad_z.t().mm(x) if need_W1 else None   # W1's own layout, as autograd forms it
-        return grad_x, grad_W1, grad_b1, grad_W2, grad_b2, None, None, None, None
-
-
-def _quantized_both_ways(g: Tensor, epoch: int, rows: bool, cols: bool) -> tuple[Fp8Operand | None, Fp8Operand | None]:
-    """(g in fp8, its transpose in fp8), each row-major, from the amax of ``epoch``."""
-    if cols and quantize_t_supported(g):
-        q, qt, scale = quantize_e4m3fn_t(g, epoch, rows)
-        return (Fp8Operand(q, scale) if rows else None), Fp8Operand(qt, scale)
-    g8 = Fp8Operand(*quantize_e4m3fn(g, epoch))
-    return g8, g8.T
-
-
-def _col_sum(g: Tensor) -> Tensor:
-    # a graph of this gradient (create_graph) needs torch's own sum
-    return col_sum(g) if col_sum_supported(g) and not torch.is_grad_enabled() else g.sum(0)
+        grads = native().block_backward(
+            grad_output, x, W1, W2, h.vals, h.bitmask, h.prefix, h.vals_offset, h.scale, h.pack_sbit, ctx.fp8,
+            ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE, ctx.needs_input_grad[:5])
+        return *grads, None, None, None
 
 
 # ------------------------------------------------------------

@@ -14,7 +14,6 @@ import torch
 from torch import Tensor
 
 from .. import _lib
-from .._lib import check, ptr, stream_handle
 from ..config import RELU2_SCALE
 
 
@@ -60,7 +59,6 @@ def gemm_compressed_b_fp8(A: Tensor, A_scale: Tensor, B_sparse, square: bool,
     square=True the to_fp8 re-quantization of the bf16 k*v^2 (times
     bf16(scale^2)) that AspRelu2B unpacks, formed from the codes in the
     kernel.  ``b_scale_out`` (fp32 0-d) receives sB."""
-    from .hip_operators import dtype_code
     if not supports_fp8(A, B_sparse):
         raise ValueError("gemm_compressed_b_fp8: unsupported operand combination")
     if A_scale is None or not A_scale.is_cuda or A_scale.dtype != torch.float32:
@@ -76,24 +74,12 @@ def gemm_compressed_b_fp8(A: Tensor, A_scale: Tensor, B_sparse, square: bool,
     stored_scale = B_sparse.scale
     if not square and stored_scale is None:
         raise ValueError("gemm_compressed_b_fp8: fp8 values without their scale")
-    L = _lib.load()
-    C = torch.empty((M, N), device=A.device, dtype=torch.bfloat16)
-    packed = B_sparse.pack_sbit
-    # a packed stream is unpacked into the room square=1 maps its codes into
-    need = L.bs_gemm_compressed_b_fp8_workspace_bytes(M, N, K, a_layout, int(square or packed))
-    ws = torch.empty(need, device=A.device, dtype=torch.uint8)
-    fn = L.bs_gemm_compressed_b_fp8_packed if packed else L.bs_gemm_compressed_b_fp8
-    check(fn(
-        a_src.data_ptr(), A_scale.data_ptr(), M, K, lda, a_layout, B_sparse.vals.data_ptr(),
-        dtype_code(_stored(B_sparse)), B_sparse.vals.numel(), B_sparse.bitmask.data_ptr(),
-        B_sparse.prefix.data_ptr(), B_sparse.vals_offset.data_ptr(), N, int(square), float(RELU2_SCALE),
-        ptr(stored_scale), C.data_ptr(), ptr(b_scale_out), ws.data_ptr(), need, stream_handle(A.device)),
-        "bs_gemm_compressed_b_fp8")
-    return C
+    return _lib.native().gemm_compressed(
+        a_src, M, K, lda, a_layout, A_scale, B_sparse.vals, _stored(B_sparse), B_sparse.pack_sbit, B_sparse.bitmask,
+        B_sparse.prefix, B_sparse.vals_offset, N, square, float(RELU2_SCALE), stored_scale, b_scale_out)
 
 
 def gemm_compressed_b(A: Tensor, B_sparse, square: bool) -> Tensor:
-    from .hip_operators import dtype_code
     if not supports(A, B_sparse, square):
         raise ValueError("gemm_compressed_b: unsupported operand combination")
     K, N = B_sparse.shape
@@ -110,17 +96,6 @@ def gemm_compressed_b(A: Tensor, B_sparse, square: bool) -> Tensor:
             pad[:, :M] = At
             At = pad
         a_layout, a_src, lda = 0, At, At.stride(0)
-    L = _lib.load()
-    C = torch.empty((M, N), device=A.device, dtype=torch.bfloat16)
-    wsfn = (L.bs_gemm_compressed_b_packed_workspace_bytes if B_sparse.pack_sbit
-            else L.bs_gemm_compressed_b_workspace_bytes)
-    need = wsfn(M, N, K, a_layout)
-    ws = torch.empty(max(need, 0), device=A.device, dtype=torch.uint8) if need > 0 else None
-    scale = B_sparse.scale if (square and B_sparse.scale is not None) else None
-    fn = L.bs_gemm_compressed_b_packed if B_sparse.pack_sbit else L.bs_gemm_compressed_b
-    check(fn(
-        a_src.data_ptr(), M, K, lda, a_layout, B_sparse.vals.data_ptr(), dtype_code(_stored(B_sparse)),
-        B_sparse.vals.numel(), B_sparse.bitmask.data_ptr(), B_sparse.prefix.data_ptr(),
-        B_sparse.vals_offset.data_ptr(), N, int(square), float(RELU2_SCALE), ptr(scale),
-        C.data_ptr(), ptr(ws), need, stream_handle(A.device)), "bs_gemm_compressed_b")
-    return C
+    return _lib.native().gemm_compressed(
+        a_src, M, K, lda, a_layout, None, B_sparse.vals, _stored(B_sparse), B_sparse.pack_sbit, B_sparse.bitmask,
+        B_sparse.prefix, B_sparse.vals_offset, N, square, float(RELU2_SCALE), B_sparse.scale if square else None, None)

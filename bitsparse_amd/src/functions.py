@@ -27,6 +27,7 @@ from torch import Tensor
 
 from . import hip_operators as ops
 from .bitpacking import pack_bits
+from .._lib import native
 from ..bitsparse import BitsparseTensor, TensorBuffer, tile_grid
 from ..config import BLOCK_M, BLOCK_N
 from ..fp8 import is_fp8
@@ -219,6 +220,8 @@ def _to_tilesparse(dense: Tensor, scale: Tensor | None, sparse_data: TensorBuffe
                                vals_offset=vals_offset, pack_sbit=pack_sbit)
 
     _check_buffer(sparse_data, dense.dtype, pack_sbit)
+    if not relu and dense.numel() > 0 and (pack_sbit or sparse_data.vals.dtype == dense.dtype):
+        return _compress_into_buffer(dense, sparse_data, pack_sbit, scale)
     fused = dict(relu=True, relu_out=dense) if relu else {}
     if pack_sbit:
         return _compress_packed_into_buffer(dense, scale, sparse_data, **fused)
@@ -233,6 +236,15 @@ def _to_tilesparse(dense: Tensor, scale: Tensor | None, sparse_data: TensorBuffe
     return BitsparseTensor(sparse_data.vals, bitmask, prefix, dense.shape, dense.dtype,
                            grid_m, grid_n, BLOCK_M, BLOCK_N, scale=scale,
                            vals_offset=vals_offset, pack_sbit=pack_sbit)
+
+
+def _compress_into_buffer(dense: Tensor, buf: TensorBuffer, pack_sbit: bool, scale: Tensor | None) -> BitsparseTensor:
+    """bs_compress / bs_compress_packed of a non-empty contiguous ``dense``, by the native host path."""
+    bitmask, prefix, start, buf._offset, _, _ = native().compress(
+        dense, buf.vals, buf._offset, buf.inplace_offset, buf.err_flags, pack_sbit, False, False)
+    grid_m, grid_n, *_ = tile_grid(*dense.shape, BLOCK_M, BLOCK_N)
+    return BitsparseTensor(buf.vals, bitmask, prefix, dense.shape, dense.dtype, grid_m, grid_n, BLOCK_M, BLOCK_N,
+                           scale=scale, vals_offset=start, pack_sbit=pack_sbit)
 
 
 def _check_buffer(buf: TensorBuffer, dtype: torch.dtype, pack_sbit: bool) -> None:
@@ -432,6 +444,16 @@ def quantize_and_compress(
     dense = dense.contiguous()
     M, N = dense.shape
     grid_m, grid_n, num_tiles, TILE_NUMEL, TILE_BYTES = tile_grid(M, N, BLOCK_M, BLOCK_N)
+    if sparse_data is not None and not _relu and M * N > 0:
+        _check_buffer(sparse_data, torch.float8_e4m3fn, pack_sbit)
+        if not pack_sbit and sparse_data.vals.dtype != torch.float8_e4m3fn:
+            raise TypeError(f"TensorBuffer stores {sparse_data.vals.dtype}, need float8_e4m3fn")
+        bitmask, prefix, start, sparse_data._offset, q, scale = native().compress(
+            dense, sparse_data.vals, sparse_data._offset, sparse_data.inplace_offset, sparse_data.err_flags,
+            pack_sbit, True, dense_out)
+        sp = BitsparseTensor(sparse_data.vals, bitmask, prefix, (M, N), torch.float8_e4m3fn, grid_m, grid_n,
+                             BLOCK_M, BLOCK_N, scale=scale, vals_offset=start, pack_sbit=pack_sbit)
+        return q, scale, sp
     amax_epoch = ops.amax_into_workspace(dense, relu=_relu)
     fused = dict(relu=True, relu_out=dense) if _relu else {}
     # the standalone path compacts from the quantized dense copy

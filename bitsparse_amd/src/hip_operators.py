@@ -465,13 +465,9 @@ def _unpack(sparse: BitsparseTensor, output: Tensor, first_m_tile: int, grid_n: 
         raise ValueError("unpack: output smaller than batch_rows x K")
     if first_m_tile + (num_tiles_in_batch + grid_n - 1) // grid_n > sparse.grid_m:
         raise ValueError("unpack: tile batch runs past the tile grid")
-    L = _lib.load()
-    fn = L.bs_decompress_packed if sparse.pack_sbit else L.bs_decompress
-    check(fn(sparse.vals.data_ptr(), dtype_code(stored), sparse.vals.numel(),
-             sparse.bitmask.data_ptr(), sparse.prefix.data_ptr(),
-             sparse.vals_offset.data_ptr(), output.data_ptr(), first_m_tile, grid_n, K,
-             batch_rows, num_tiles_in_batch, int(square), float(RELU2_SCALE),
-             ptr(scale), stream_handle(output.device)), "bs_decompress")
+    _lib.native().decompress(sparse.vals, stored, sparse.pack_sbit, sparse.bitmask, sparse.prefix, sparse.vals_offset,
+                             output, first_m_tile, grid_n, K, batch_rows, num_tiles_in_batch, square,
+                             float(RELU2_SCALE), scale)
     return output
 
 
