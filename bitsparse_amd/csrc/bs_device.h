@@ -84,6 +84,38 @@ __device__ __forceinline__ void st_chunk(void* p, const T& v)
     else st8<NT>(p, v);
 }
 
+// a chunk at any address its elements can have (2-byte aligned bf16, any byte
+// for fp8): gfx950's global accesses need no more, so rows whose length is no
+// multiple of 8 still move as one instruction per chunk
+template <typename T>
+__device__ __forceinline__ T ld_chunk_unaligned(const void* p)
+{
+    T v;
+    __builtin_memcpy(&v, p, sizeof(T));
+    return v;
+}
+template <typename T>
+__device__ __forceinline__ void st_chunk_unaligned(void* p, const T& v)
+{
+    __builtin_memcpy(p, &v, sizeof(T));
+}
+// the chunk without its first `s` elements of B bytes, zeros behind (s >= 8: none left)
+template <int B, typename T>
+__device__ __forceinline__ T chunk_drop_front(const T& v, int s)
+{
+    if constexpr (B == 2) {
+        const uint64_t lo = ((uint64_t)v.y << 32) | v.x, hi = ((uint64_t)v.w << 32) | v.z;
+        const int b = 16 * (s & 3);
+        const uint64_t l0 = s >= 8 ? 0 : s >= 4 ? hi : lo, h0 = s >= 4 ? 0 : hi;
+        const uint64_t l = b ? (l0 >> b) | (h0 << (64 - b)) : l0, h = h0 >> b;
+        return T{(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
+    } else {
+        const uint64_t w = ((uint64_t)v.y << 32) | v.x;
+        const uint64_t l = s >= 8 ? 0 : w >> (8 * s);
+        return T{(uint32_t)l, (uint32_t)(l >> 32)};
+    }
+}
+
 // ---------------------------------------------------------------------------
 // positive tests on raw bits: x > 0 <=> bits in (0, +Inf]
 // ---------------------------------------------------------------------------

@@ -82,9 +82,10 @@ def compact_vals(
         return _compact_vals_packed(dense, tile_bitmasks, tile_prefix, vals, vals_offset, M, N,
                                     num_tiles)
     if vals is None:
+        # (filled ahead of the read-back that the host waits for)
+        vals_offset = torch.zeros((), device=dense.device, dtype=torch.int64)
         nnz = int(tile_prefix[-1].item())
         vals = torch.empty(nnz, device=dense.device, dtype=dense.dtype)
-        vals_offset = torch.zeros((), device=dense.device, dtype=torch.int64)
     elif vals.dtype != dense.dtype:
         raise TypeError(f"compact_vals: storage dtype {vals.dtype} differs from input {dense.dtype}")
     L = _lib.load()
