@@ -174,3 +174,26 @@ def test_block_equals_the_separate_nodes(dev, square, store, use_buffer, monkeyp
     for a, b, name in zip(outs[0][4:], outs[1][4:], ("db1", "db2")):
         # two bf16 roundings of fp32 sums
         assert ((a - b).double().abs() <= 2.0 ** -7 * b.double().abs() + 1e-2).all(), name
+
+
+def test_block_under_saved_tensor_hooks(dev):
+    """Hooks that hand the backward other values than the forward saw: the
+    operands' scales are taken from those values (no code past the format)."""
+    from bitsparse_amd.bitsparse import TensorBuffer
+    from bitsparse_amd.layers import FFNRelu2
+    g = torch.Generator().manual_seed(21)
+    x, W1, W2, dY = (torch.randn(s, generator=g).to(torch.bfloat16).to(dev) * 0.1
+                     for s in ((64, 64), (128, 64), (64, 128), (64, 64)))
+    grads = []
+    for scaled in (False, True):
+        p = [t.clone().requires_grad_() for t in (x, W1, W2)]
+        buf = TensorBuffer(64 * 128, device=dev, dtype=E4M3)
+        unpack = (lambda t: t * 4) if scaled else (lambda t: t)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            y = FFNRelu2.apply(*p, sparse_data=buf, storage_dtype=E4M3)
+        y.backward(dY)
+        assert all(bool(t.grad.isfinite().all()) for t in p)
+        grads.append(p[0].grad)
+    # dx = (dY W2 ...) W1 with both weights times 4
+    ratio = grads[1].double().norm() / grads[0].double().norm()
+    assert 12 < float(ratio) < 20
