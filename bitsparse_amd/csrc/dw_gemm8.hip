@@ -537,22 +537,21 @@ __global__ __launch_bounds__(CFG::THREADS, CFG::MINB) void gemm_cb8_kernel(Gemm8
 // each of a wave's two 16-byte loads reads 1 KiB of whole cache lines; zero
 // past M and K.  k-block major: the A rows a workgroup reads in one step
 // are one contiguous range (spread over all L2 channels).
-__device__ __forceinline__ int64_t apk8_index(int64_t m, int64_t k, uint32_t nrb)
-{
-    const int64_t rb = m >> 5, kb = k >> 6;
-    const int l = (int)(m & 31) + 32 * (int)((k >> 5) & 1);
-    return (kb * nrb + rb) * 2048 + ((k >> 4) & 1) * 1024 + l * 16 + (k & 15);
-}
 
-// from At [K, M] (row stride ldat, m contiguous): 64 x 64 blocks through LDS
-__global__ __launch_bounds__(256) void pack_a8_t_kernel(const uint8_t* At, int64_t K, int64_t M, int64_t ldat,
-                                                        uint8_t* Apk, uint32_t nrb)
+// from At [K, M] (row stride ldat, m contiguous): 64 k x 128 m blocks through
+// LDS, read back k-contiguous with the transposing reads of the GEMM's B
+// fragments (four per lane for its 32 bytes; one byte at a time, a 4096 x 4096
+// A took 9.4 us)
+__device__ __forceinline__ void pack_a8_block(const uint8_t* At, int64_t K, int64_t M, int64_t ldat, uint8_t* Apk,
+                                              uint32_t nrb, int64_t kb, int64_t mb)
 {
-    __shared__ __align__(16) uint8_t t[64][64 + 16];
+    constexpr int P = 128 + 16;
+    __shared__ __align__(16) uint8_t t[64 * P];
     const int tid = threadIdx.x;
-    const int64_t k0 = (int64_t)blockIdx.x * 64, m0 = (int64_t)blockIdx.y * 64;
-    {
-        const int row = tid >> 2, c16 = (tid & 3) * 16;          // k row, 16 m
+    const int64_t k0 = kb * 64, m0 = mb * 128;
+#pragma unroll
+    for (int it = 0; it < 2; it++) {
+        const int row = it * 32 + (tid >> 3), c16 = (tid & 7) * 16;   // k row, 16 m
         const int64_t k = k0 + row, m = m0 + c16;
         uint4 v = {0u, 0u, 0u, 0u};
         if (k < K && m < M) {
@@ -565,18 +564,22 @@ __global__ __launch_bounds__(256) void pack_a8_t_kernel(const uint8_t* At, int64
                 v = uint4{w[0], w[1], w[2], w[3]};
             }
         }
-        *reinterpret_cast<uint4*>(&t[row][c16]) = v;
+        *reinterpret_cast<uint4*>(&t[row * P + c16]) = v;
     }
     __syncthreads();
-    const int64_t mrows = (M + 31) / 32 * 32;           // Apk rows (whole 32-row blocks)
-    {
-        const int mm = tid >> 2, kc = (tid & 3) * 16;           // m row, 16 k
-        if (m0 + mm < mrows) {
-            uint32_t w[4] = {0u, 0u, 0u, 0u};
+    // wave w: row block w; lane l: row l % 32 of it, k = 32 (l/32) .. +31
+    const int wave = tid >> 6, lane = tid & 63, j = lane & 15;
+    if (m0 + 32 * wave < M) {
+        typedef __attribute__((address_space(3))) i32x2_t lds_i32x2;
+        i32x2_t v[4];
 #pragma unroll
-            for (int e = 0; e < 16; e++) w[e >> 2] |= (uint32_t)t[kc + e][mm] << (8 * (e & 3));
-            *reinterpret_cast<uint4*>(Apk + apk8_index(m0 + mm, k0 + kc, nrb)) = uint4{w[0], w[1], w[2], w[3]};
-        }
+        for (int c = 0; c < 4; c++)
+            v[c] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(t + (32 * (lane >> 5) + 8 * c + (j >> 1)) * P +
+                                                                       32 * wave + 16 * ((lane >> 4) & 1) + 8 * (j & 1)));
+        uint8_t* dst = Apk + (kb * nrb + (m0 >> 5) + wave) * 2048 + lane * 16;
+        *reinterpret_cast<uint4*>(dst) = uint4{(uint32_t)v[0][0], (uint32_t)v[0][1], (uint32_t)v[1][0], (uint32_t)v[1][1]};
+        *reinterpret_cast<uint4*>(dst + 1024) =
+            uint4{(uint32_t)v[2][0], (uint32_t)v[2][1], (uint32_t)v[3][0], (uint32_t)v[3][1]};
     }
 }
 
@@ -629,7 +632,7 @@ constexpr int kCodeMaxBlocks = 256;
 // Block b writes the largest magnitude of its 16-byte units of the run
 // [vo + prefix[0], vo + prefix[T]) to cmax[b] (every block writes, so the
 // slots need no clearing).
-__global__ __launch_bounds__(256) void code_max_kernel(Lut8Args a)
+__device__ __forceinline__ void code_max_block(const Lut8Args& a, uint32_t block, uint32_t blocks)
 {
     const int64_t vo = a.vals_offset ? *a.vals_offset : 0;
     int64_t b0 = vo + (int64_t)a.prefix[0];
@@ -640,8 +643,8 @@ __global__ __launch_bounds__(256) void code_max_kernel(Lut8Args a)
     if (b1 > b0) {
         const int64_t u0 = b0 >> 4, u1 = (b1 + 15) >> 4;
         const bs_rsrc rs = make_rsrc(a.vals + u0 * 16, (uint32_t)std::min<int64_t>(a.vals_numel - u0 * 16, 0xffffffffll));
-        const int64_t stride = (int64_t)gridDim.x * 256;
-        for (int64_t u = u0 + (int64_t)blockIdx.x * 256 + threadIdx.x; u < u1; u += stride) {
+        const int64_t stride = (int64_t)blocks * 256;
+        for (int64_t u = u0 + (int64_t)block * 256 + threadIdx.x; u < u1; u += stride) {
             const int64_t e0 = u * 16;
             uint32_t w[4];
             if (e0 + 16 <= a.vals_numel) {
@@ -666,8 +669,27 @@ __global__ __launch_bounds__(256) void code_max_kernel(Lut8Args a)
     __shared__ uint32_t s_w[4];
     if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) a.cmax[blockIdx.x] = max(max(s_w[0], s_w[1]), max(s_w[2], s_w[3]));
+    if (threadIdx.x == 0) a.cmax[block] = max(max(s_w[0], s_w[1]), max(s_w[2], s_w[3]));
 }
+
+// A's packing (a_layout 0) and the code maximum, which do not depend on each
+// other, as one launch: workgroups below max_blocks scan the codes (first, as
+// the table pass waits for them), the rest pack 64 k x 128 m blocks of A, k
+// fastest.  Each alone left most of the chip idle (8 + 9 us at the 4096 x
+// 4096 x 16384 weight gradient).
+__global__ __launch_bounds__(256) void pack_a8_t_kernel(const uint8_t* At, int64_t K, int64_t M, int64_t ldat,
+                                                        uint8_t* Apk, uint32_t nrb, uint32_t nkb, uint32_t max_blocks,
+                                                        Lut8Args la)
+{
+    if (blockIdx.x < max_blocks) {
+        code_max_block(la, blockIdx.x, max_blocks);
+        return;
+    }
+    const uint32_t id = blockIdx.x - max_blocks;
+    pack_a8_block(At, K, M, ldat, Apk, nrb, id % nkb, id / nkb);
+}
+
+__global__ __launch_bounds__(256) void code_max_kernel(Lut8Args a) { code_max_block(a, blockIdx.x, gridDim.x); }
 
 // D(c) of code c as bf16 bits: the ReLU^2 unpack of fp8 storage
 // (bf16((k v) v), then bf16(. * bf16(s^2)) with a scale)
@@ -1077,27 +1099,31 @@ static int gemm8_impl(const void* A, const float* a_scale, int64_t M, int64_t K,
             hipLaunchKernelGGL((map_packed_kernel<DT_E4M3FN, true>), dim3(mblk), dim3(256), 0, st, la, map_out,
                                map_cap, map_vo);
         }
-    } else if (square) {
-        hipLaunchKernelGGL(code_max_kernel, dim3(kCodeMaxBlocks), dim3(256), 0, st, la);
-        if (vals_dtype == DT_E4M3FN)
-            hipLaunchKernelGGL(map_codes_kernel<DT_E4M3FN>, dim3(mblk), dim3(256), 0, st, la, map_out, map_cap, map_vo);
-        else
-            hipLaunchKernelGGL(map_codes_kernel<DT_E5M2>, dim3(mblk), dim3(256), 0, st, la, map_out, map_cap, map_vo);
-    } else {
-        hipLaunchKernelGGL(copy_scale_kernel, dim3(1), dim3(64), 0, st, b_scale, sB, b_scale_out);
     }
-
     // A into MFMA-fragment order (workspace after the partial sums)
     uint8_t* apk = (uint8_t*)workspace + part_bytes;
+    const bool max_here = square && !packed && a_layout == 0;      // with A's packing
     if (a_layout == 0) {
-        hipLaunchKernelGGL(pack_a8_t_kernel, dim3((uint32_t)nkb, (uint32_t)((M + 63) / 64)), dim3(256), 0, st,
-                           (const uint8_t*)A, K, M, lda, apk, (uint32_t)nrb);
+        const uint32_t mb = max_here ? (uint32_t)kCodeMaxBlocks : 0u;
+        const uint64_t pb = (uint64_t)nkb * (uint64_t)((M + 127) / 128);
+        if (pb + mb >= (1ull << 31)) return set_error(BS_ERR_INVALID, "%s: grid too large", fn);
+        hipLaunchKernelGGL(pack_a8_t_kernel, dim3(mb + (uint32_t)pb), dim3(256), 0, st, (const uint8_t*)A, K, M, lda, apk,
+                           (uint32_t)nrb, (uint32_t)nkb, mb, la);
     } else {
         const int64_t pieces = nrb * nkb * 128;
         int64_t nblk = (pieces + 255) / 256;
         if (nblk > 4096) nblk = 4096;
         hipLaunchKernelGGL(pack_a8_n_kernel, dim3((uint32_t)nblk), dim3(256), 0, st, (const uint8_t*)A, K, M, lda,
                            apk, (uint32_t)nrb, pieces);
+    }
+    if (square && !packed) {
+        if (!max_here) hipLaunchKernelGGL(code_max_kernel, dim3(kCodeMaxBlocks), dim3(256), 0, st, la);
+        if (vals_dtype == DT_E4M3FN)
+            hipLaunchKernelGGL(map_codes_kernel<DT_E4M3FN>, dim3(mblk), dim3(256), 0, st, la, map_out, map_cap, map_vo);
+        else
+            hipLaunchKernelGGL(map_codes_kernel<DT_E5M2>, dim3(mblk), dim3(256), 0, st, la, map_out, map_cap, map_vo);
+    } else if (!square && !packed) {
+        hipLaunchKernelGGL(copy_scale_kernel, dim3(1), dim3(64), 0, st, b_scale, sB, b_scale_out);
     }
     Gemm8Args g{};
     g.Apk = apk;
