@@ -318,11 +318,14 @@ template <int DT>
 __device__ __forceinline__ typename Raw<DT == DT_BF16 ? 2 : 1>::T relu_chunk(typename Raw<DT == DT_BF16 ? 2 : 1>::T v)
 {
     if constexpr (DT == DT_BF16) {
+        // as signed halves these are the values <= -128: those that adding 127,
+        // saturating, leaves negative (3 instructions for two elements)
+        typedef short i16x2 __attribute__((ext_vector_type(2)));
         uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const uint32_t lo = w[i] & 0xffffu, hi = w[i] >> 16;
-            w[i] = ((lo - 0x8000u) < 0x7f81u ? 0u : lo) | (((hi - 0x8000u) < 0x7f81u ? 0u : hi) << 16);
+            const i16x2 t = __builtin_elementwise_add_sat(__builtin_bit_cast(i16x2, w[i]), (i16x2)(short)127);
+            w[i] &= ~__builtin_bit_cast(uint32_t, t >> (i16x2)(short)15);
         }
         return uint4{w[0], w[1], w[2], w[3]};
     } else {
@@ -498,7 +501,7 @@ __device__ uint32_t wave_lookback_grouped(const CompressArgs& a, uint32_t u, uin
 #ifndef BS_STREAM_ROUNDS
 #define BS_STREAM_ROUNDS 2
 #endif
-constexpr int kRoundsPerPass = BS_STREAM_ROUNDS;   // rounds written before each store pass
+constexpr int kRoundsPerPass = BS_STREAM_ROUNDS;   // rounds written before each store pass (even: ranked in pairs)
 // >= 15 (pending) + 512 per round + 8 (overrun), a multiple of 16
 constexpr int kRingElems = 512 * kRoundsPerPass + 32;
 
@@ -547,8 +550,20 @@ __device__ __forceinline__ uint32_t bit_range_mask(uint32_t lb, uint32_t hb)
     return hi & ~lo;
 }
 
+// Ranks of the lane's chunks inside rounds k and k + 1 (k even), and the
+// rounds' totals, in the two halves of a register: one scan for both (a round
+// has at most 512 values).
+__device__ __forceinline__ void round_ranks(const uint32_t* mp, int k, uint32_t& ranks, uint32_t& total)
+{
+    const uint32_t w = mp[k >> 2] >> (8 * (k & 3));
+    const uint32_t c = (uint32_t)__popc(w & 0xffu) | ((uint32_t)__popc(w & 0xff00u) << 16);
+    const uint32_t in = wave_incl_scan(c);
+    ranks = in - c;
+    total = (uint32_t)__builtin_amdgcn_readlane((int)in, 63);
+}
+
 // Packed stream phase of one wave's run: values [0, cnt) of the tile's run
-// (compacted chunks o[k] of round k at run position P[k] + in-round rank) go
+// (compacted chunks o[k] of round k at the round's run position + in-round rank) go
 // to stream bits [g*PB, (g+cnt)*PB) of a.vals (a.vals_capacity dwords).
 // ring[i] holds run value base + i.
 // The run's partial dwords (shared with the neighbouring runs) are OR-ed into
@@ -556,8 +571,7 @@ __device__ __forceinline__ uint32_t bit_range_mask(uint32_t lb, uint32_t hb)
 // writes those dwords afterwards (packed_unit_edges).  s_toff[b] is the run
 // offset of boundary b inside the unit, whose run starts at value gu.
 template <int OUTB, int PB, int U>
-__device__ __forceinline__ void stream_packed(const CompressArgs& a, int64_t g, int cnt, const uint32_t* P,
-                                              const uint32_t* mp, const typename Raw<OUTB>::T* o,
+__device__ __forceinline__ void stream_packed(const CompressArgs& a, int64_t g, int cnt, const uint32_t* mp, const typename Raw<OUTB>::T* o,
                                               uint8_t* ring, int lane, int64_t gu, const uint32_t* s_toff,
                                               uint32_t* s_edge)
 {
@@ -579,20 +593,23 @@ __device__ __forceinline__ void stream_packed(const CompressArgs& a, int64_t g, 
     const int dcap = capw <= 0 ? 0 : (int)min<int64_t>(capw, (int64_t)dend);   // far cursor must not wrap)
     int dn = 0;                                  // next dword to produce
     int base = 0;
+    int at = 0;                                  // run position of the next round
+    uint32_t ranks = 0, total = 0;
     // rounds are written into the ring until the next one might not fit
     // (a round adds <= 512 values and 8 of overrun); each flush then builds
     // the dwords its values complete
 #pragma unroll
     for (int k = 0; k < 8; k++) {
         {
+            if ((k & 1) == 0) round_ranks(mp, k, ranks, total);
             const uint32_t m = (mp[k >> 2] >> (8 * (k & 3))) & 0xffu;
-            const uint32_t c = (uint32_t)__popc(m);
-            const uint32_t ex = wave_incl_scan(c) - c;
-            if (c != 0u) write_compacted<OUTB>(ring + ((int)P[k] - base + (int)ex) * OUTB, o[k]);
+            const uint32_t ex = (k & 1) ? ranks >> 16 : ranks & 0xffffu;
+            if (m != 0u) write_compacted<OUTB>(ring + (at - base + (int)ex) * OUTB, o[k]);
+            at += (int)((k & 1) ? total >> 16 : total & 0xffffu);
         }
-        if (k < 7 && (int)P[k + 1] - base + 520 <= kRingElems) continue;
+        if (k < 7 && at - base + 520 <= kRingElems) continue;
         wave_sync_lds();
-        const int done = (int)P[k + 1];
+        const int done = at;
         const int dl = done == cnt ? dend : ((sb + done * PB) >> 5);
         const int dlw = min(dl, dcap);
         for (int d = dn + lane; d < dlw; d += 64) {
@@ -701,6 +718,17 @@ void compress_stream_kernel(CompressArgs a)
     constexpr int NSEL = OUTB == 2 ? 8 : 2; // selector dwords per mask byte
     using RawIn = typename Raw<INB>::T;
     using RawOut = typename Raw<OUTB>::T;
+    // The tile's value count: one wave reduction of the sixty-four popcounts
+    // after the last chunk, or (raw bf16 values streamed past the caches) four
+    // ballots per chunk.  Up to the streaming size the kernel is short of VALU
+    // issue slots as much as of bandwidth, and the ballots and the eight
+    // per-round totals they used to leave in scalar registers (most of them
+    // spilled) cost 7 + 6 instructions a chunk; above it the reads and writes
+    // are the bound and the count at the end lets all eight loads drain before
+    // any mask work.  compress + decompress, ballots -> one reduction:
+    // 8192 x 3072 36.5 -> 35.8 us, 5053 x 6152 packed 50.1 -> 49.0, 16384 x
+    // 16384 packed 374 -> 366, but 16384 x 16384 raw 319 -> 324 (322 -> 330).
+    constexpr bool BALLOT_SUM = NT && !PACKED && OUTB == 2;
     static_assert(U >= 1 && U <= 16, "one wave per tile, at most 16 waves");
 
     __shared__ uint32_t s_cnt[U];
@@ -828,8 +856,7 @@ void compress_stream_kernel(CompressArgs a)
         // ---- masks, bitmask bytes, round totals
         RawOut o[8];
         uint32_t mp[2] = {0u, 0u};              // the eight mask bytes, four per register
-        uint32_t P[9];                          // wave-uniform run offset of each round
-        P[0] = 0;
+        int cnt = 0;                            // the tile's values (wave-uniform)
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             uint32_t m;
@@ -885,10 +912,11 @@ void compress_stream_kernel(CompressArgs a)
                 }
             }
             mp[k >> 2] |= m << (8 * (k & 3));
-            P[k + 1] = P[k] + wave_sum_count(__popc(m));
+            if constexpr (BALLOT_SUM) cnt += (int)wave_sum_count(__popc(m));
         }
+        if constexpr (!BALLOT_SUM) cnt = (int)wave_total(__popc(mp[0]) + __popc(mp[1]));
         if constexpr (MODE != MODE_VALS) {
-            if (lane == 0) s_cnt[wave] = P[8];
+            if (lane == 0) s_cnt[wave] = (uint32_t)cnt;
         }
         __syncthreads();                        // s_cnt; the selector table
 
@@ -990,9 +1018,8 @@ void compress_stream_kernel(CompressArgs a)
                     g = start + (int64_t)(a.prefix[t] - a.prefix[a.tile0]);
                 else
                     g = start + (int64_t)uniform_u32(s_excl[0]) + (int64_t)uniform_u32(s_toff[wave]);
-                const int cnt = (int)P[8];
                 if constexpr (PACKED) {
-                    stream_packed<OUTB, TR::PB, U>(a, g, cnt, P, mp, o, s_ring + wave * (kRingElems * OUTB), lane,
+                    stream_packed<OUTB, TR::PB, U>(a, g, cnt, mp, o, s_ring + wave * (kRingElems * OUTB), lane,
                                                    start + (int64_t)uniform_u32(s_excl[0]),
                                                    s_toff, s_edge);
                 } else {
@@ -1009,24 +1036,29 @@ void compress_stream_kernel(CompressArgs a)
                 bool front_done = front_n == 0;
                 bool back_done = back_s >= endr;
                 int pend = 0;                   // output slot held in ring slot 0
+                int at = 0;                     // run offset of the next round
 #pragma unroll
                 for (int k0 = 0; k0 < 8; k0 += kRoundsPerPass) {
                     if (front_done && back_done && max(pend, j_lo) >= j_hi) break;
                     // one pass at a time: nothing of a later pass is computed early
                     asm volatile("" : "+v"(mp[0]), "+v"(mp[1]) : : "memory");
 #pragma unroll
-                    for (int kk = 0; kk < kRoundsPerPass; kk++) {
-                        const int k = k0 + kk;
-                        const uint32_t m = (mp[k >> 2] >> (8 * (k & 3))) & 0xffu;
-                        const uint32_t c = (uint32_t)__popc(m);
-                        const uint32_t ex = wave_incl_scan(c) - c;
-                        const int rb = a0 + (int)P[k] - pend * EPS;       // ring index of the round's first element
-                        if (c != 0u) write_compacted<OUTB>(ring + (rb + (int)ex) * OUTB, o[k]);
+                    for (int k = k0; k < k0 + kRoundsPerPass; k += 2) {
+                        uint32_t ranks, total;
+                        round_ranks(mp, k, ranks, total);
+                        const uint32_t w = mp[k >> 2] >> (8 * (k & 3));
+                        const int rb = a0 + at - pend * EPS;              // ring index of the round's first element
+                        if ((w & 0xffu) != 0u)
+                            write_compacted<OUTB>(ring + (rb + (int)(ranks & 0xffffu)) * OUTB, o[k]);
+                        if ((w & 0xff00u) != 0u)
+                            write_compacted<OUTB>(ring + (rb + (int)(total & 0xffffu) + (int)(ranks >> 16)) * OUTB,
+                                                  o[k + 1]);
+                        at += (int)(total & 0xffffu) + (int)(total >> 16);
                     }
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    const int done = (int)P[k0 + kRoundsPerPass];
+                    const int done = at;
                     const int npend = (a0 + done) / EPS;
                     if (!front_done && done >= front_n) {
                         front_done = true;          // pend is still 0 here
