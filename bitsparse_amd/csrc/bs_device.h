@@ -424,6 +424,32 @@ __device__ __forceinline__ uint2 quant_chunk_tab(const uint4 v, const uint8_t* q
     return uint2{p[0] | (p[1] << 16), p[2] | (p[3] << 16)};
 }
 
+// The code table of `scale` (layout above) built in LDS by a workgroup of THREADS
+// threads: the positive half from div2_to_e4m3 on pairs of magnitudes
+// (exact: f32_to_e4m3 of the correctly rounded quotient), the negative half
+// with the sign bit set; a NaN scale gives the scale's NaN for every non-NaN
+// magnitude and x's own NaN otherwise, as the division does.
+template <int THREADS>
+__device__ __forceinline__ void qtab_build_lds(uint8_t* tab, float scale, float rcp, int tid)
+{
+    const int qoff = qtab_offset(scale);
+    const bool nan_s = scale != scale;
+    static_assert(kQtabEntries % 2 == 0, "entries come in pairs");
+    for (int p = tid; p < kQtabEntries / 2; p += THREADS) {
+        const int m0 = min(max(qoff + 2 * p, 0), 0x7fff), m1 = min(max(qoff + 2 * p + 1, 0), 0x7fff);
+        uint32_t pos, neg;
+        if (nan_s) {
+            pos = 0x7f7fu;
+            neg = (m0 > 0x7f80 ? 0xffu : 0x7fu) | ((m1 > 0x7f80 ? 0xffu : 0x7fu) << 8);
+        } else {
+            pos = div2_to_e4m3(bf16_to_f32((uint32_t)m0), bf16_to_f32((uint32_t)m1), scale, rcp);
+            neg = pos | 0x8080u;
+        }
+        *reinterpret_cast<uint16_t*>(tab + 2 * p) = (uint16_t)pos;
+        *reinterpret_cast<uint16_t*>(tab + kQtabEntries + 2 * p) = (uint16_t)neg;
+    }
+}
+
 // The activation step's pair table: entry i (as above, positive magnitudes
 // only) holds the code of r in its low byte and that of h(r) in its high one.
 // It serves a tensor whose scale of h is finite: its r (>= 0) are then finite

@@ -148,25 +148,10 @@ __device__ __forceinline__ uint32_t qtab_entry(int m, float scale)
     const uint32_t c = f32_to_e4m3(bf16_to_f32((uint32_t)m) / scale);
     return scale != scale ? 0x7fu : c;
 }
-__global__ __launch_bounds__(256) void qtab_build_kernel(const uint64_t* slot, uint32_t epoch, uint8_t* qtab)
-{
-    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (i >= kQtabEntries) return;
-    const float scale = scale_from_slot(slot, epoch);
-    const int m = min(max(qtab_offset(scale) + i, 0), 0x7fff);
-    const uint32_t c = qtab_entry(m, scale);
-    qtab[i] = (uint8_t)c;
-    // (a NaN scale gives x's own NaN for a NaN x, else the scale's)
-    qtab[kQtabEntries + i] = (uint8_t)(scale != scale && m <= 0x7f80 ? 0x7fu : c | 0x80u);
-}
 
 // The pair table (pair_codes_tab): the code of r and that of h = k r^2
-__global__ __launch_bounds__(256) void pair_tab_build_kernel(const uint64_t* slot, uint32_t epoch, uint16_t* tab,
-                                                             float k)
+__device__ __forceinline__ void pair_tab_put(uint16_t* tab, int i, float scale, float h_scale, float k)
 {
-    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (i >= kQtabEntries) return;
-    const float scale = scale_from_slot(slot, epoch), h_scale = relu2_scale_from_slot(slot, epoch, k);
     const int m = min(max(qtab_offset(scale) + i, 0), 0x7fff);
     const uint32_t hc = f32_to_e4m3(bf16_to_f32(relu2_sq_bits((uint32_t)m, k)) / h_scale);
     tab[i] = (uint16_t)(qtab_entry(m, scale) | (hc << 8));
@@ -234,7 +219,6 @@ struct CompressArgs {
     int32_t* err;
     uint32_t* fallbacks;
     uint64_t patience;          // look-back wait (s_memrealtime ticks) before counting a unit itself
-    const uint8_t* qtab;        // quantize: the code table (kQtabBytes), copied into LDS
     float relu_k;               // WB_SQUARE / WB_ACT_SQUARE: h = bf16(bf16(r * r) * relu_k), r = relu(dense)
     const uint16_t* bias;       // WB_ACT*: nullable, dense + bias is the pre-activation
     float* h_scale_out;         // WB_ACT_SQUARE, quantizing: scale of h's codes
@@ -827,9 +811,19 @@ void compress_stream_kernel(CompressArgs a)
             }
         }
         if constexpr (QUANT) {
-            // the code table into LDS, behind the dense loads (16-byte copies)
-            for (int i = tid; i < kQtabBytes / 16; i += 64 * U)
-                reinterpret_cast<uint4*>(s_qtab)[i] = reinterpret_cast<const uint4*>(a.qtab)[i];
+            // the code table, while the dense loads are in flight: its few
+            // divisions a thread cost less than a launch of their own and
+            // a copy per workgroup (amax + compress + decompress, table kernel
+            // -> here: 256 x 512 21.6 -> 20.9 us, 8192 x 3072 48.8 -> 47.5,
+            // 4096 x 16384 108.5 -> 106.9, 8192 x 16384 196.4 -> 194.0; with
+            // the pair table, two divisions an entry, the block step is the same)
+            if constexpr (HCODES) {
+#pragma unroll 1
+                for (int i = tid; i < kQtabEntries; i += 64 * U)
+                    pair_tab_put(reinterpret_cast<uint16_t*>(s_qtab), i, scale, h_scale, a.relu_k);
+            } else {
+                qtab_build_lds<64 * U>(s_qtab, scale, rcp, tid);
+            }
             __syncthreads();
         }
         if constexpr (!VEC) {
@@ -2075,17 +2069,15 @@ static hipError_t launch_compress(const CompressArgs& a, int in_dtype, bool quan
 
 using namespace bs;
 
-// The quantizer's code table sits after the status words (256-byte aligned).
-static int64_t ws_qtab_offset(int64_t T) { return (kWsHeaderBytes + 8 * (T + 2) + 255) / 256 * 256; }
-
 extern "C" int64_t bs_compress_workspace_bytes(int64_t M, int64_t N)
 {
     if (M < 0 || N < 0) return -1;
     int64_t T = ((M + 63) / 64) * ((N + 63) / 64);
     // status words: one per tile covers the units and the unit groups of the
-    // streaming kernel (T/8 + T/512 words) and the units of the others; then
-    // the quantizer's code table
-    return ws_qtab_offset(T) + kQtabBytes;
+    // streaming kernel (T/8 + T/512 words) and the units of the others.  The
+    // size callers know is that of an earlier form, which kept the quantizer's
+    // code table behind the words (256-byte aligned); it is still what they ask for
+    return (kWsHeaderBytes + 8 * (T + 2) + 255) / 256 * 256 + kQtabBytes;
 }
 
 extern "C" const uint64_t* bs_workspace_amax_slot(const void* ws, int64_t)
@@ -2225,17 +2217,6 @@ static int compress_impl(const void* dense, int in_dtype, int64_t M, int64_t N, 
     }
     if (wb == WB_SQUARE && relu_out == dense) a.patience = kInPlaceSquareTicks;
     a.gstat = a.status + (T + kStreamU - 1) / kStreamU;
-    if (quantize) {
-        // the code table of this call's scale, built after the amax it reads
-        uint8_t* qtab = (uint8_t*)workspace + ws_qtab_offset(T);
-        if (wb == WB_ACT_SQUARE)
-            hipLaunchKernelGGL(pair_tab_build_kernel, dim3((kQtabEntries + 255) / 256), dim3(256), 0, st, amax_slot,
-                               amax_epoch, (uint16_t*)qtab, relu_k);
-        else
-            hipLaunchKernelGGL(qtab_build_kernel, dim3((kQtabEntries + 255) / 256), dim3(256), 0, st, amax_slot,
-                               amax_epoch, qtab);
-        a.qtab = qtab;
-    }
     const int inb = in_dtype == DT_BF16 ? 2 : 1;
     bool vec = (N % 8 == 0) && (((uintptr_t)dense) % (8 * inb) == 0) && vec_rows_fit(N, inb) &&
                (dense_q_out == nullptr || aligned8(dense_q_out)) &&

@@ -139,31 +139,6 @@ __device__ __forceinline__ float fp8_scale_from_slot(const uint64_t* slot, uint3
     return (sc < 1e-9f) ? 1e-9f : sc;
 }
 
-// The code table of `scale` (qtab_build_kernel's layout) built in LDS by the
-// workgroup: the positive half from div2_to_e4m3 on pairs of magnitudes
-// (exact: f32_to_e4m3 of the correctly rounded quotient), the negative half
-// with the sign bit set; a NaN scale gives the scale's NaN for every non-NaN
-// magnitude and x's own NaN otherwise, as the division does.
-__device__ __forceinline__ void qtab_build_lds(uint8_t* tab, float scale, float rcp, int tid)
-{
-    const int qoff = qtab_offset(scale);
-    const bool nan_s = scale != scale;
-    static_assert(kQtabEntries % 2 == 0, "entries come in pairs");
-    for (int p = tid; p < kQtabEntries / 2; p += kFp8Threads) {
-        const int m0 = min(max(qoff + 2 * p, 0), 0x7fff), m1 = min(max(qoff + 2 * p + 1, 0), 0x7fff);
-        uint32_t pos, neg;
-        if (nan_s) {
-            pos = 0x7f7fu;
-            neg = (m0 > 0x7f80 ? 0xffu : 0x7fu) | ((m1 > 0x7f80 ? 0xffu : 0x7fu) << 8);
-        } else {
-            pos = div2_to_e4m3(bf16_to_f32((uint32_t)m0), bf16_to_f32((uint32_t)m1), scale, rcp);
-            neg = pos | 0x8080u;
-        }
-        *reinterpret_cast<uint16_t*>(tab + 2 * p) = (uint16_t)pos;
-        *reinterpret_cast<uint16_t*>(tab + kQtabEntries + 2 * p) = (uint16_t)neg;
-    }
-}
-
 // NT: nontemporal loads of x and stores of q.  Each thread's first chunk is
 // loaded before the table is built.
 template <bool NT>
@@ -182,7 +157,7 @@ __global__ __launch_bounds__(kFp8Threads) void quantize_e4m3_kernel(const uint16
     const int64_t stride = (int64_t)gridDim.x * kFp8Threads;
     int64_t i = (int64_t)blockIdx.x * kFp8Threads + tid;
     uint4 v = i < nvec ? ld16<NT>(reinterpret_cast<const uint4*>(x) + i) : uint4{0u, 0u, 0u, 0u};
-    qtab_build_lds(s_tab, scale, rcp, tid);
+    qtab_build_lds<kFp8Threads>(s_tab, scale, rcp, tid);
     __syncthreads();
     const int qoff = qtab_offset(scale);
     for (; i < nvec; i += stride) {
@@ -318,7 +293,7 @@ __global__ __launch_bounds__(kFp8Threads) void quantize_t_kernel(const uint16_t*
             v[i] = ld16<NT>(x + r * C + min(c, C - 8));
         }
         if (!built) {
-            qtab_build_lds(s_tab, scale, 1.0f / scale, t);
+            qtab_build_lds<kFp8Threads>(s_tab, scale, 1.0f / scale, t);
             built = true;
         }
         __syncthreads();                               // the table; the last tile's reads of s
