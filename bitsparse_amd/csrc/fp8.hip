@@ -269,15 +269,14 @@ __global__ __launch_bounds__(256) void transpose_u8_kernel(const uint8_t* in, in
 // Needs C % 8 == 0, R % 4 == 0, 16-byte aligned x, 8-byte aligned q.
 template <bool BOTH, bool NT>
 __global__ __launch_bounds__(kFp8Threads) void quantize_t_kernel(const uint16_t* x, int64_t R, int64_t C, uint8_t* q,
-                                                                 uint8_t* qt, float* scale_out, const float* scale_in,
-                                                                 const uint64_t* slot, uint32_t epoch,
-                                                                 uint32_t tiles_c, uint32_t ntiles)
+                                                                 uint8_t* qt, float* scale_out, const uint64_t* slot,
+                                                                 uint32_t epoch, uint32_t tiles_c, uint32_t ntiles)
 {
     __shared__ __align__(16) uint8_t s_tab[kQtabBytes];
     __shared__ __align__(16) uint32_t s[kTrTile * 32];
-    const float scale = scale_in ? *scale_in : fp8_scale_from_slot(slot, epoch);
+    const float scale = fp8_scale_from_slot(slot, epoch);
     const int t = threadIdx.x;
-    if (blockIdx.x == 0 && t == 0 && scale_out) *scale_out = scale;
+    if (blockIdx.x == 0 && t == 0) *scale_out = scale;
     const int qoff = qtab_offset(scale);
     const int cc = 8 * (t % 16), d0 = cc / 4;          // the thread's columns in the tile, as dword columns
     const int rb = t % 32;                             // transposed side: input rows 4 rb .. 4 rb + 3 (swizzle rb)
@@ -548,21 +547,19 @@ extern "C" int bs_quantize_e4m3fn(const void* x, int64_t n, void* q_out, float* 
 }
 
 extern "C" int bs_quantize_e4m3fn_t(const void* x, int64_t R, int64_t C, void* q_out, void* qt_out, float* scale_out,
-                                    const float* scale_in, const void* workspace, int64_t workspace_bytes,
-                                    uint32_t epoch, void* stream)
+                                    const void* workspace, int64_t workspace_bytes, uint32_t epoch, void* stream)
 {
     clear_error();
     if (R <= 0 || C <= 0) return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: empty input");
-    if (scale_in == nullptr && (workspace == nullptr || workspace_bytes < kWsHeaderBytes))
+    if (workspace == nullptr || workspace_bytes < kWsHeaderBytes)
         return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: workspace too small");
-    if (x == nullptr || qt_out == nullptr || (scale_out == nullptr && scale_in == nullptr))
+    if (x == nullptr || qt_out == nullptr || scale_out == nullptr)
         return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: null pointer");
     if (C % 8 != 0 || R % 4 != 0 || (((uintptr_t)x) & 15u) || (((uintptr_t)q_out) & 7u) || (((uintptr_t)qt_out) & 3u))
         return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: needs C %% 8 == 0, R %% 4 == 0 and aligned operands");
     if ((uint64_t)R * (uint64_t)C >= kMaxElemsUntested)
         return set_error(BS_ERR_INVALID, "bs_quantize_e4m3fn_t: R*C must be < 2^31");
-    const uint64_t* slot = scale_in ? nullptr
-                                    : reinterpret_cast<const uint64_t*>((const uint8_t*)workspace + kWsAmaxOffset);
+    const uint64_t* slot = reinterpret_cast<const uint64_t*>((const uint8_t*)workspace + kWsAmaxOffset);
     const uint32_t tiles_c = (uint32_t)((C + kTrTile - 1) / kTrTile);
     const uint32_t ntiles = (uint32_t)((R + kTrTile - 1) / kTrTile) * tiles_c;
     // six workgroups' tiles and tables fit a CU's LDS at once
@@ -571,7 +568,7 @@ extern "C" int bs_quantize_e4m3fn_t(const void* x, int64_t R, int64_t C, void* q
     auto kernel = q_out ? (nt ? quantize_t_kernel<true, true> : quantize_t_kernel<true, false>)
                         : (nt ? quantize_t_kernel<false, true> : quantize_t_kernel<false, false>);
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFp8Threads), 0, (hipStream_t)stream, (const uint16_t*)x, R, C,
-                       (uint8_t*)q_out, (uint8_t*)qt_out, scale_out, scale_in, slot, epoch, tiles_c, ntiles);
+                       (uint8_t*)q_out, (uint8_t*)qt_out, scale_out, slot, epoch, tiles_c, ntiles);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(BS_ERR_HIP, "bs_quantize_e4m3fn_t launch: %s", hipGetErrorString(e));
     return BS_OK;

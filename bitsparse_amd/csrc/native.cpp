@@ -7,7 +7,6 @@
 #include <dlfcn.h>
 #include <torch/extension.h>
 
-#include <ATen/SavedTensorHooks.h>
 #include <ATen/core/grad_mode.h>
 #include <ATen/hip/HIPContext.h>
 #include <c10/core/DeviceGuard.h>
@@ -269,22 +268,15 @@ std::pair<Tensor, Fp8> quantize_t(const Tensor& x, int64_t amax_epoch, bool rows
     Tensor q;
     if (rows) q = empty({R, C}, x, at::kFloat8_e4m3fn);
     Fp8 t{empty({C, R}, x, at::kFloat8_e4m3fn), empty({}, x, at::kFloat)};
-    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), R, C, raw(q), t.codes.data_ptr(), ptr<float>(t.scale), nullptr,
-                                 w.buf.data_ptr(), w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn_t");
+    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), R, C, raw(q), t.codes.data_ptr(), ptr<float>(t.scale), w.buf.data_ptr(),
+                                 w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn_t");
     return {q, t};
 }
 
-// an operand multiplied from the right: column-major codes; `scale`: x's own,
-// from an earlier quantization of the same x
-Fp8 right_operand(const Tensor& x, const std::optional<Tensor>& scale, Workspace& w)
+// an operand multiplied from the right: column-major codes
+Fp8 right_operand(const Tensor& x, Workspace& w)
 {
     const Tensor c = x.contiguous();
-    if (scale) {
-        const Tensor qt = empty({c.size(1), c.size(0)}, c, at::kFloat8_e4m3fn);
-        check(L.bs_quantize_e4m3fn_t(c.data_ptr(), c.size(0), c.size(1), nullptr, qt.data_ptr(), nullptr,
-                                     ptr<float>(*scale), nullptr, 0, 0, stream_of(c)), "bs_quantize_e4m3fn_t");
-        return {qt.t(), *scale};
-    }
     Lock lock(w.mu);
     Fp8 t = quantize_t(c, amax(c, false, Tensor(), w), false, w).second;
     return {t.codes.t(), t.scale};
@@ -379,12 +371,8 @@ Tensor col_sum(const Tensor& g)
 // the amax on the activation's gradient, and the fp8 operands of the backward
 // products are quantized into the layout those take.  The caller (layers.py)
 // has checked the operands.
-// -> (y, bitmask, prefix, start of the values, advanced cursor, scale, the fp8
-// scales of x, W1 and W2).  The backward quantizes these three again; where
-// autograd hands it the very tensors back (it checks their versions; not
-// under saved-tensor hooks, which may change values) their scales still hold
-// and spare it three passes over them (75 us of the 4096 x 4096 -> 16384 step).
-std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, std::optional<Tensor>, std::vector<Tensor>>
+// -> (y, bitmask, prefix, start of the values, advanced cursor, scale)
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, std::optional<Tensor>>
 block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bias1, const Tensor& W2,
               const std::optional<Tensor>& bias2, const Tensor& vals, const std::optional<Tensor>& offset,
               const Tensor& err, bool in_place, bool packed, bool fp8, bool square, double k)
@@ -394,10 +382,8 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bi
     const int64_t M = x.size(0), N = W1.size(0), T = tiles(M, N);
     Workspace& w = ws_of(x);
     Tensor z;
-    std::vector<Tensor> scales;
     if (fp8) {
         const Fp8 a = to_fp8(x, w), b = to_fp8(W1, w);
-        scales = {a.scale, b.scale};
         z = fp8_mm(a, {b.codes.t(), b.scale}, at::kBFloat16);
     } else {
         z = at::mm(x, W1.t());
@@ -429,14 +415,12 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bi
     Tensor y;
     if (fp8) {
         const Fp8 b = to_fp8(W2, w);
-        scales.push_back(b.scale);
         y = fp8_mm({operand, operand_scale}, {b.codes.t(), b.scale}, at::kBFloat16);
     } else {
         y = at::mm(operand, W2.t());
     }
     if (b2.defined()) y.add_(b2);
-    if (at::SavedTensorDefaultHooks::get_hooks(false).has_value()) scales.clear();
-    return {y, bitmask, prefix, c.start, c.next, scale.defined() ? std::optional<Tensor>(scale) : std::nullopt, scales};
+    return {y, bitmask, prefix, c.start, c.next, scale.defined() ? std::optional<Tensor>(scale) : std::nullopt};
 }
 
 // (dx, dW1, db1, dW2, db2), each where `need` asks for it
@@ -444,10 +428,9 @@ std::vector<std::optional<Tensor>>
 block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const Tensor& vals,
                const Tensor& bitmask, const Tensor& prefix, const Tensor& start, const std::optional<Tensor>& scale,
                bool packed, bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
-               const std::vector<bool>& need, const std::vector<Tensor>& scales)
+               const std::vector<bool>& need)
 {
     const c10::DeviceGuard guard(x.device());
-    auto scale_of = [&](size_t i) { return scales.empty() ? std::nullopt : std::optional<Tensor>(scales[i]); };
     const Held h{vals, bitmask, prefix, start, scale.value_or(Tensor()), x.size(0), W1.size(0), packed, fp8, square, k};
     const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3], need_b2 = need[4];
     std::vector<std::optional<Tensor>> out(5);
@@ -457,7 +440,7 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
     if (fp8) g8 = to_fp8(g, w);
     if (need_W2) out[3] = down_weight_grad(fp8 ? g8.codes : g, g8.scale, h);
     if (!(need_x || need_W1 || need_b1)) return out;
-    Tensor dz = fp8 ? fp8_mm(g8, right_operand(W2, scale_of(2), w), at::kBFloat16) : at::mm(g, W2);
+    Tensor dz = fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
     const bool want8 = fp8 && (need_x || need_W1);
     const bool sums = need_b1 && !at::GradMode::is_enabled();
     Fp8 z8, zt8;
@@ -494,8 +477,8 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
     if (need_b1 && !sums) out[2] = col_sum(dz);
     if (fp8) {
         const at::ScalarType gd = grad_dtype.value_or(at::kFloat8_e4m3fn);
-        if (need_x) out[0] = widened(fp8_mm(z8, right_operand(W1, scale_of(1), w), gd));
-        if (need_W1) out[1] = widened(fp8_mm(zt8, right_operand(x, scale_of(0), w), gd));
+        if (need_x) out[0] = widened(fp8_mm(z8, right_operand(W1, w), gd));
+        if (need_W1) out[1] = widened(fp8_mm(zt8, right_operand(x, w), gd));
     } else {
         if (need_x) out[0] = at::mm(dz, W1);
         if (need_W1) out[1] = at::mm(dz.t(), x);      // W1's own layout, as autograd forms it

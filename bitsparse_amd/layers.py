@@ -257,7 +257,7 @@ class _FFNBlock(Function):
 
     @staticmethod
     def forward(ctx, x, W1, b1, W2, b2, buf, fp8, square):
-        y, bitmask, prefix, start, buf._offset, scale, ctx.scales = native().block_forward(
+        y, bitmask, prefix, start, buf._offset, scale = native().block_forward(
             x, W1, b1, W2, b2, buf.vals, buf._offset, buf.err_flags, buf.inplace_offset, buf.pack_sbit, fp8, square,
             float(RELU2_SCALE))
         M, N = x.shape[0], W1.shape[0]
@@ -276,7 +276,7 @@ class _FFNBlock(Function):
         ctx.h_sparse = None
         grads = native().block_backward(
             grad_output, x, W1, W2, h.vals, h.bitmask, h.prefix, h.vals_offset, h.scale, h.pack_sbit, ctx.fp8,
-            ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE, ctx.needs_input_grad[:5], ctx.scales)
+            ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE, ctx.needs_input_grad[:5])
         return *grads, None, None, None
 
 

@@ -384,22 +384,19 @@ def quantize_t_supported(x: Tensor) -> bool:
             and x.shape[1] % 8 == 0 and x.shape[0] % 4 == 0 and x.data_ptr() % 16 == 0)
 
 
-def quantize_e4m3fn_t(x: Tensor, amax_epoch: int, both: bool,
-                      scale: Tensor | None = None) -> tuple[Tensor | None, Tensor, Tensor]:
+def quantize_e4m3fn_t(x: Tensor, amax_epoch: int, both: bool) -> tuple[Tensor | None, Tensor, Tensor]:
     """(codes of x or None, codes of x.T as a new row-major tensor, fp32 0-d
-    scale) from the amax of ``amax_epoch``, or with ``scale``, x's own scale
-    from an earlier quantization (``quantize_t_supported``); ``both``: the
-    row-major codes too."""
+    scale) from the amax of ``amax_epoch`` (``quantize_t_supported``);
+    ``both``: the row-major codes too."""
     R, C = x.shape
     L = _lib.load()
     ws = _lib.workspace_for(x.device)
     q = torch.empty((R, C), device=x.device, dtype=torch.float8_e4m3fn) if both else None
     qt = torch.empty((C, R), device=x.device, dtype=torch.float8_e4m3fn)
-    out = torch.empty((), device=x.device, dtype=torch.float32) if scale is None else scale
-    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), R, C, ptr(q), qt.data_ptr(), out.data_ptr() if scale is None else None,
-                                 ptr(scale), ws.buf.data_ptr(), ws.nbytes, amax_epoch, stream_handle(x.device)),
-          "bs_quantize_e4m3fn_t")
-    return q, qt, out
+    scale = torch.empty((), device=x.device, dtype=torch.float32)
+    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), R, C, ptr(q), qt.data_ptr(), scale.data_ptr(), ws.buf.data_ptr(),
+                                 ws.nbytes, amax_epoch, stream_handle(x.device)), "bs_quantize_e4m3fn_t")
+    return q, qt, scale
 
 
 def transpose_u8(x: Tensor, out: Tensor | None = None) -> Tensor:

@@ -358,14 +358,11 @@ int bs_amax_relu2_from(void* workspace, int64_t workspace_bytes, uint32_t epoch_
 /*
  * bs_quantize_e4m3fn of a row-major [R, C] matrix with its codes transposed
  * (qt_out: uint8 [C, R], row-major) and, with q_out (nullable), row-major too:
- * bs_quantize_e4m3fn + bs_transpose_u8 in one pass, the same codes.  With
- * scale_in (device fp32, nullable) the scale is that one -- x's own, taken by
- * an earlier quantization of the same x -- instead of the amax slot's; the
- * workspace is then not read and scale_out may be null.  R, C >= 1, C % 8 == 0, R % 4 == 0, x 16-, q_out 8-, qt_out 4-byte aligned, R * C < 2^31.
+ * bs_quantize_e4m3fn + bs_transpose_u8 in one pass, the same codes.  R, C >= 1,
+ * C % 8 == 0, R % 4 == 0, x 16-, q_out 8-, qt_out 4-byte aligned, R * C < 2^31.
  */
 int bs_quantize_e4m3fn_t(const void* x, int64_t R, int64_t C, void* q_out, void* qt_out, float* scale_out,
-                         const float* scale_in, const void* workspace, int64_t workspace_bytes, uint32_t epoch,
-                         void* stream);
+                         const void* workspace, int64_t workspace_bytes, uint32_t epoch, void* stream);
 
 /*
  * out[c * ld_out + r] = in[r * ld_in + c] for an [R, C] byte matrix: the

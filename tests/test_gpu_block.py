@@ -1,5 +1,7 @@
 """The MLP block's single node and its activation / gradient kernels against
 the separate steps they stand for, bit for bit (column sums: fp32 order)."""
+import contextlib
+
 import pytest
 import torch
 
@@ -176,24 +178,51 @@ def test_block_equals_the_separate_nodes(dev, square, store, use_buffer, monkeyp
         assert ((a - b).double().abs() <= 2.0 ** -7 * b.double().abs() + 1e-2).all(), name
 
 
-def test_block_under_saved_tensor_hooks(dev):
-    """Hooks that hand the backward other values than the forward saw: the
-    operands' scales are taken from those values (no code past the format)."""
+def _graph_node(t, name):
+    """The autograd node of that name behind t."""
+    nodes = [t.grad_fn]
+    while nodes:
+        n = nodes.pop()
+        if n is not None and n.name() == name:
+            return n
+        nodes += [m for m, _ in n.next_functions] if n is not None else []
+    raise AssertionError(f"no {name}")
+
+
+@pytest.mark.parametrize("how", ["default_hooks", "node_hooks", "data"])
+@pytest.mark.parametrize("grow", [4.0, 0.25])
+def test_backward_scales_the_values_it_reads(dev, how, grow, monkeypatch):
+    """The backward's operands need not hold what the forward saw: saved-tensor
+    hooks (the default ones, or set on the node afterwards) and writes through
+    .data change them without autograd's notice.  They are quantized with
+    their own scales: no code past the format, none lost below it."""
     from bitsparse_amd.bitsparse import TensorBuffer
+    from bitsparse_amd import config
     from bitsparse_amd.layers import FFNRelu2
+    monkeypatch.setattr(config, "FP8_GRAD_DTYPE", torch.bfloat16)
     g = torch.Generator().manual_seed(21)
     x, W1, W2, dY = (torch.randn(s, generator=g).to(torch.bfloat16).to(dev) * 0.1
                      for s in ((64, 64), (128, 64), (64, 128), (64, 64)))
     grads = []
-    for scaled in (False, True):
+    for factor in (1.0, grow):
         p = [t.clone().requires_grad_() for t in (x, W1, W2)]
         buf = TensorBuffer(64 * 128, device=dev, dtype=E4M3)
-        unpack = (lambda t: t * 4) if scaled else (lambda t: t)
-        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+
+        def unpack(t):
+            return t * factor
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack) if how == "default_hooks" else \
+                contextlib.nullcontext():
             y = FFNRelu2.apply(*p, sparse_data=buf, storage_dtype=E4M3)
+        if how == "node_hooks":
+            for saved in _graph_node(y, "_FFNBlockBackward")._raw_saved_tensors:
+                saved.register_hooks(lambda t: t, unpack)
+        elif how == "data":
+            for t in p:
+                t.data.mul_(factor)
         y.backward(dY)
-        assert all(bool(t.grad.isfinite().all()) for t in p)
-        grads.append(p[0].grad)
-    # dx = (dY W2 ...) W1 with both weights times 4
-    ratio = grads[1].double().norm() / grads[0].double().norm()
-    assert 12 < float(ratio) < 20
+        grads.append([t.grad for t in p])
+    # dx = (dY W2 . 2 r) W1 and dW1 = (dY W2 . 2 r)^T x with all three scaled; r is the
+    # forward's, and a power of two moves no code
+    for i in (0, 1):
+        assert torch.equal(grads[1][i].float(), grads[0][i].float() * grow * grow), i
+    assert torch.equal(grads[1][2], grads[0][2])
