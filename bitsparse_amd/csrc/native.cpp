@@ -340,12 +340,14 @@ Tensor gemm_compressed(const Tensor& a, int64_t M, int64_t K, int64_t lda, int64
 Tensor down_weight_grad(const Tensor& g, const Tensor& g_scale, const Held& h)
 {
     Tensor a = g;
-    if (!h.fp8 && (a.stride(1) != 1 || a.stride(0) % 8 != 0 || (reinterpret_cast<uintptr_t>(a.data_ptr()) & 15))) {
-        const int64_t M = g.size(1);
+    const int64_t M = g.size(1);
+    // rows that overlap (a gradient expanded over the tokens has row stride 0) are copied too
+    if (!h.fp8 && (a.stride(1) != 1 || a.stride(0) % 8 != 0 || a.stride(0) < M ||
+                   (reinterpret_cast<uintptr_t>(a.data_ptr()) & 15))) {
         a = at::zeros({h.M, (M + 7) / 8 * 8}, g.options());
         a.narrow(1, 0, M).copy_(g);
     }
-    return gemm_compressed(a, g.size(1), h.M, a.stride(0), 0, h.fp8 ? std::optional<Tensor>(g_scale) : std::nullopt,
+    return gemm_compressed(a, M, h.M, a.stride(0), 0, h.fp8 ? std::optional<Tensor>(g_scale) : std::nullopt,
                            h.vals, h.fp8 ? at::kFloat8_e4m3fn : at::kBFloat16, h.packed, h.bitmask, h.prefix, h.start,
                            h.N, h.square, h.k, h.fp8 ? std::optional<Tensor>(h.scale) : std::nullopt, std::nullopt);
 }

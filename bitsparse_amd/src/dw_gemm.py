@@ -84,13 +84,14 @@ def gemm_compressed_b(A: Tensor, B_sparse, square: bool) -> Tensor:
         raise ValueError("gemm_compressed_b: unsupported operand combination")
     K, N = B_sparse.shape
     M = A.shape[0]
-    if A.stride(1) == 1 and A.stride(0) % 8 == 0 and A.data_ptr() % 16 == 0 and K % 8 == 0:
+    # rows that overlap (an expanded gradient has row stride 0) are copied too
+    if A.stride(1) == 1 and A.stride(0) % 8 == 0 and A.stride(0) >= K and A.data_ptr() % 16 == 0 and K % 8 == 0:
         a_layout, a_src, lda = 1, A, A.stride(0)          # k contiguous: read in place
     else:
         # the kernel transposes A^T [K, M] (m contiguous; for A = dY.T this
         # is dY itself) into its workspace; rows padded to a multiple of 8
         At = A.t()
-        if At.stride(1) != 1 or At.stride(0) % 8 != 0 or At.data_ptr() % 16 != 0:
+        if At.stride(1) != 1 or At.stride(0) % 8 != 0 or At.stride(0) < M or At.data_ptr() % 16 != 0:
             ld = (M + 7) // 8 * 8
             pad = torch.zeros((K, ld), device=A.device, dtype=A.dtype)
             pad[:, :M] = At

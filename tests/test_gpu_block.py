@@ -226,3 +226,36 @@ def test_backward_scales_the_values_it_reads(dev, how, grow, monkeypatch):
     for i in (0, 1):
         assert torch.equal(grads[1][i].float(), grads[0][i].float() * grow * grow), i
     assert torch.equal(grads[1][2], grads[0][2])
+
+
+@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed"])
+@pytest.mark.parametrize("block", [True, False])
+@pytest.mark.parametrize("layout", ["one_row", "one_value", "column", "transposed", "padded", "misaligned", "overlapping"])
+def test_gradient_layouts(dev, store, block, layout, monkeypatch):
+    """The gradients that y.sum(0), y.mean() and slices of a wider output
+    deliver: expanded, transposed, strided and misaligned ones give what their
+    contiguous copy gives."""
+    from bitsparse_amd import layers
+    from bitsparse_amd.bitsparse import TensorBuffer
+    if not block:
+        monkeypatch.setattr(layers, "_block_ok", lambda *a: False)
+    g = torch.Generator().manual_seed(31)
+    T, D, Hn = 80, 48, 144
+    x, W1, b1, W2, b2, base = (torch.randn(s, generator=g).to(torch.bfloat16).to(dev) * 0.1
+                               for s in ((T, D), (Hn, D), (Hn,), (D, Hn), (D,), (T * (D + 8) + 8,)))
+    strides = {"one_row": (0, 1), "one_value": (0, 0), "column": (1, 0), "transposed": (1, T), "padded": (D + 8, 1),
+               "misaligned": (D, 1), "overlapping": (8, 1)}[layout]
+    dY = base.as_strided((T, D), strides, 1 if layout == "misaligned" else 0)
+    fp8, pack = store == "e4m3", store.endswith("packed")
+    outs = []
+    for grad in (dY, dY.contiguous()):
+        p = [t.clone().requires_grad_() for t in (x, W1, W2, b1, b2)]
+        buf = TensorBuffer(2 * T * Hn + 64, device=dev, dtype=E4M3 if fp8 else torch.bfloat16, pack_sbit=pack)
+        y = layers.FFNRelu.apply(*p, sparse_data=buf, pack_sbit=pack, dtype=E4M3 if fp8 else torch.bfloat16)
+        y.backward(grad)
+        outs.append([t.grad for t in p])
+    for a, b, name in zip(*outs, ("dx", "dW1", "dW2", "db1")):
+        _same(a, b, name)
+    # another summation order where torch sums a strided gradient: fp32 sums, one rounding each
+    a, b = outs[0][4].double(), outs[1][4].double()
+    assert ((a - b).abs() <= 2.0 ** -8 * (a.abs() + b.abs()) + T * 2.0 ** -23 * dY.double().abs().sum(0)).all()
