@@ -2215,7 +2215,7 @@ static int compress_impl(const void* dense, int in_dtype, int64_t M, int64_t N, 
         const unsigned long long v = strtoull(ev, &end, 10);
         if (end != ev) a.patience = (uint64_t)v;
     }
-    if (wb == WB_SQUARE && relu_out == dense) a.patience = kInPlaceSquareTicks;
+    if ((wb == WB_SQUARE || wb == WB_ACT_SQUARE) && relu_out == dense) a.patience = kInPlaceSquareTicks;
     a.gstat = a.status + (T + kStreamU - 1) / kStreamU;
     const int inb = in_dtype == DT_BF16 ? 2 : 1;
     bool vec = (N % 8 == 0) && (((uintptr_t)dense) % (8 * inb) == 0) && vec_rows_fit(N, inb) &&
@@ -2290,8 +2290,8 @@ extern "C" int bs_compress_act(const void* preact, const void* bias, int64_t M, 
     if (quantize ? (codes_out == nullptr || !aligned8(codes_out) || h_out != nullptr) : h_out == nullptr)
         return set_error(BS_ERR_INVALID, "bs_compress_act: quantize writes codes_out (8-byte aligned) and no h_out, "
                                          "else h_out is written");
-    if (h_out == preact && (square || bias != nullptr))
-        return set_error(BS_ERR_INVALID, "bs_compress_act: h_out may alias preact only without a bias or square");
+    if (h_out == preact && bias != nullptr)
+        return set_error(BS_ERR_INVALID, "bs_compress_act: h_out may alias preact only without a bias");
     if (quantize && amax_slot == nullptr) return set_error(BS_ERR_INVALID, "bs_compress_act: null amax slot");
     if ((uint64_t)M * (uint64_t)N >= kMaxElemsUntested)
         return set_error(BS_ERR_INVALID, "bs_compress_act: M*N must be < 2^31");

@@ -402,8 +402,8 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bi
             operand_scale = square ? empty({}, x, at::kFloat) : scale;
             operand = codes = empty({M, N}, x, at::kFloat8_e4m3fn);
         } else {
-            // over z where that leaves a recount of z (the look-back's fallback) right
-            operand = h_out = b1.defined() || square ? at::empty_like(z) : z;
+            // over z, unless the bias would be added again by a recount of z (the look-back's fallback)
+            operand = h_out = b1.defined() ? at::empty_like(z) : z;
         }
         w.ensure(L.bs_compress_workspace_bytes(M, N));
         const int64_t epoch = w.next_epoch(1);
@@ -414,6 +414,7 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bi
                                 ptr<int64_t>(c.next), ptr<int64_t>(c.start_out), ptr<int32_t>(err), w.buf.data_ptr(),
                                 w.nbytes(), epoch, stream_of(x)), "bs_compress_act");
     }
+    z.reset();          // (the down-projection does not need its room)
     Tensor y;
     if (fp8) {
         const Fp8 b = to_fp8(W2, w);
@@ -425,15 +426,18 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bi
     return {y, bitmask, prefix, c.start, c.next, scale.defined() ? std::optional<Tensor>(scale) : std::nullopt};
 }
 
-// (dx, dW1, db1, dW2, db2), each where `need` asks for it
+// (dx, dW1, db1, dW2, db2), each where `need` asks for it.  `held`: (values,
+// bitmask, prefix, start, scale) of the activation, taken out of the list, so
+// that they go once the last kernel that reads them is queued.
 std::vector<std::optional<Tensor>>
-block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const Tensor& vals,
-               const Tensor& bitmask, const Tensor& prefix, const Tensor& start, const std::optional<Tensor>& scale,
-               bool packed, bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
+block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const py::list& held, bool packed,
+               bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
                const std::vector<bool>& need)
 {
     const c10::DeviceGuard guard(x.device());
-    const Held h{vals, bitmask, prefix, start, scale.value_or(Tensor()), x.size(0), W1.size(0), packed, fp8, square, k};
+    Held h{held[0].cast<Tensor>(), held[1].cast<Tensor>(), held[2].cast<Tensor>(), held[3].cast<Tensor>(),
+           held[4].is_none() ? Tensor() : held[4].cast<Tensor>(), x.size(0), W1.size(0), packed, fp8, square, k};
+    held.attr("clear")();
     const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3], need_b2 = need[4];
     std::vector<std::optional<Tensor>> out(5);
     Workspace& w = ws_of(x);
@@ -443,6 +447,7 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
     if (need_W2) out[3] = down_weight_grad(fp8 ? g8.codes : g, g8.scale, h);
     if (!(need_x || need_W1 || need_b1)) return out;
     Tensor dz = fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
+    g8 = Fp8();
     const bool want8 = fp8 && (need_x || need_W1);
     const bool sums = need_b1 && !at::GradMode::is_enabled();
     Fp8 z8, zt8;
@@ -456,11 +461,13 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
         Tensor db1;
         if (sums) out[2] = db1 = empty({h.N}, x, at::kBFloat16);
         const int64_t bytes = L.bs_grad_sums_workspace_bytes(h.M, h.N);
-        const Tensor part = empty({bytes}, x, at::kByte);
-        check(L.bs_act_grad_sums(dz.data_ptr(), h.M, h.N, square, vals.data_ptr(), fp8 ? 1 : 0, vals.numel(), packed,
-                                 ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix), ptr<int64_t>(start), (float)k,
+        Tensor part = empty({bytes}, x, at::kByte);
+        check(L.bs_act_grad_sums(dz.data_ptr(), h.M, h.N, square, h.vals.data_ptr(), fp8 ? 1 : 0, h.vals.numel(),
+                                 packed, ptr<uint8_t>(h.bitmask), ptr<uint32_t>(h.prefix), ptr<int64_t>(h.start), (float)k,
                                  ptr<float>(h.scale), raw(db1), want8 ? w.buf.data_ptr() : nullptr, epoch,
                                  part.data_ptr(), bytes, stream_of(x)), "bs_act_grad_sums");
+        part.reset();
+        h = Held();
         if (want8 && need_W1) {
             const auto [q, t] = quantize_t(dz, epoch, need_x, w);
             z8 = {q, t.scale};
@@ -470,12 +477,13 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
         }
     } else if (square) {
         check((packed ? L.bs_relu2_grad_packed : L.bs_relu2_grad)(
-                  dz.data_ptr(), h.M, h.N, vals.data_ptr(), fp8 ? 1 : 0, vals.numel(), ptr<uint8_t>(bitmask),
-                  ptr<uint32_t>(prefix), ptr<int64_t>(start), (float)k, ptr<float>(h.scale), stream_of(x)),
+                  dz.data_ptr(), h.M, h.N, h.vals.data_ptr(), fp8 ? 1 : 0, h.vals.numel(), ptr<uint8_t>(h.bitmask),
+                  ptr<uint32_t>(h.prefix), ptr<int64_t>(h.start), (float)k, ptr<float>(h.scale), stream_of(x)),
               "bs_relu2_grad");
     } else {
-        check(L.bs_relu_grad(dz.data_ptr(), h.M, h.N, ptr<uint8_t>(bitmask), stream_of(x)), "bs_relu_grad");
+        check(L.bs_relu_grad(dz.data_ptr(), h.M, h.N, ptr<uint8_t>(h.bitmask), stream_of(x)), "bs_relu_grad");
     }
+    h = Held();
     if (need_b1 && !sums) out[2] = col_sum(dz);
     if (fp8) {
         const at::ScalarType gd = grad_dtype.value_or(at::kFloat8_e4m3fn);

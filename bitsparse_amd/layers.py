@@ -274,9 +274,10 @@ class _FFNBlock(Function):
         x, W1, W2 = ctx.saved_tensors
         h: BitsparseTensor = ctx.h_sparse
         ctx.h_sparse = None
+        held, packed = [h.vals, h.bitmask, h.prefix, h.vals_offset, h.scale], h.pack_sbit
+        del h
         grads = native().block_backward(
-            grad_output, x, W1, W2, h.vals, h.bitmask, h.prefix, h.vals_offset, h.scale, h.pack_sbit, ctx.fp8,
-            ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE, ctx.needs_input_grad[:5])
+            grad_output, x, W1, W2, held, packed, ctx.fp8, ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE, ctx.needs_input_grad[:5])
         return *grads, None, None, None
 
 

@@ -546,8 +546,10 @@ int64_t bs_compress_noalloc_max_tiles(void);
  * h = bf16(bf16(r * r) * k), k finite.
  *   bias       bf16 [N], 16-byte aligned; nullable: none
  *   quantize   0: bf16 values; h_out (bf16 [M, N], 16-byte aligned; may alias
- *              preact only without bias and square: a look-back fallback
- *              counts from preact) receives r or h, codes_out is not used.
+ *              preact only without a bias, as a look-back fallback counts from
+ *              preact: with square = 1 in place it waits 10 s before it does
+ *              and then flags bit 2 of *err_flags, as bs_compress_relu2) receives
+ *              r or h, codes_out is not used.
  *              1: e4m3fn values with the scale of amax|r|, which the amax
  *              slot holds under amax_epoch (bs_amax_bias_relu, or
  *              bs_amax_relu without a bias); h_out must be null; codes_out

@@ -259,3 +259,44 @@ def test_gradient_layouts(dev, store, block, layout, monkeypatch):
     # another summation order where torch sums a strided gradient: fp32 sums, one rounding each
     a, b = outs[0][4].double(), outs[1][4].double()
     assert ((a - b).abs() <= 2.0 ** -8 * (a.abs() + b.abs()) + T * 2.0 ** -23 * dY.double().abs().sum(0)).all()
+
+
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed"])
+@pytest.mark.parametrize("bias", [False, True])
+def test_peak_memory(dev, square, store, bias, monkeypatch):
+    """The single node holds no more at its peak than the separate ones, whose
+    square is in place and whose product goes at the bias add (the biased
+    operand is a second [T, H] beside z like theirs, but with the bitmask
+    there already)."""
+    from bitsparse_amd import layers
+    from bitsparse_amd.bitsparse import TensorBuffer
+    g = torch.Generator().manual_seed(41)
+    T, D, Hn = 2048, 128, 2048
+    fp8, pack = store == "e4m3", store.endswith("packed")
+    p = [(torch.randn(s, generator=g).to(torch.bfloat16).to(dev) * 0.1).requires_grad_()
+         for s in ((T, D), (Hn, D), (D, Hn), (Hn,), (D,))]
+    dY = torch.randn((T, D), generator=g).to(torch.bfloat16).to(dev)
+    buf = TensorBuffer(2 * T * Hn + 64, device=dev, dtype=E4M3 if fp8 else torch.bfloat16, pack_sbit=pack)
+    layer, kw = (layers.FFNRelu2, "storage_dtype") if square else (layers.FFNRelu, "dtype")
+    peaks = []
+    for block in (True, False):
+        if not block:
+            monkeypatch.setattr(layers, "_block_ok", lambda *a: False)
+        for _ in range(2):                       # the second has its workspaces
+            buf.reset_buffer()
+            base = torch.cuda.memory_allocated(dev)
+            torch.cuda.reset_peak_memory_stats(dev)
+            y = layer.apply(*p[:3], *(p[3:] if bias else ()), sparse_data=buf, pack_sbit=pack,
+                            **{kw: E4M3 if fp8 else torch.bfloat16})
+            forward = torch.cuda.max_memory_allocated(dev) - base
+            torch.cuda.reset_peak_memory_stats(dev)
+            y.backward(dY)
+            backward = torch.cuda.max_memory_allocated(dev) - base
+            del y
+            for t in p:
+                t.grad = None
+        peaks.append((forward, backward))
+    slack = 64 * 1024                            # rows of N, cursors, scales: each its own 512-byte block
+    assert peaks[0][0] <= peaks[1][0] + slack + (T * Hn // 8 + T * Hn // 1024 if bias else 0), peaks
+    assert peaks[0][1] <= peaks[1][1] + slack, peaks
