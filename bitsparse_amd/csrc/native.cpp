@@ -10,11 +10,11 @@
 #include <ATen/core/grad_mode.h>
 #include <ATen/hip/HIPContext.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include <map>
 #include <memory>
-#include <mutex>
 
 #include "bitsparse_hip.h"
 
@@ -94,20 +94,34 @@ constexpr int64_t kEpochLimit = (int64_t(1) << 30) - 1;
 // Zero-initialised device scratch with an epoch counter.  Each compress / amax
 // call takes a fresh epoch; status words written under older epochs are
 // ignored by the kernels, so the buffer never needs clearing between calls.
-// When the counter wraps the buffer is zeroed again.  `mu` is held while a
-// sequence that passes an amax through the workspace is enqueued (backward
-// threads run without the interpreter lock).
+// When the counter wraps the buffer is zeroed again.
+//
+// Threads: every entry of this module is called from Python and holds the
+// interpreter lock throughout, which is what keeps a sequence that passes an
+// amax through the workspace whole, as long as nothing in it runs Python.  So
+// a sequence allocates its outputs first, then calls `prepare`, and makes no
+// call into torch from there to its last launch; the workspace's own torch
+// calls leave the thread's dispatch modes out.  (No mutex: a thread in a mode's
+// Python code gives the lock away, and one waiting for the mutex would not.)
 struct Workspace {
-    explicit Workspace(c10::Device d) : device(d), buf(at::zeros({0}, at::device(d).dtype(at::kByte))) {}
+    explicit Workspace(c10::Device d) : device(d)
+    {
+        const NoPython guard;
+        buf = at::zeros({0}, at::device(d).dtype(at::kByte));
+    }
     c10::Device device;
     Tensor buf;
     int64_t epoch = 0;
-    std::recursive_mutex mu;
+
+    struct NoPython {
+        c10::impl::ExcludeDispatchKeyGuard guard{c10::DispatchKeySet(
+            {c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::PythonDispatcher})};
+    };
 
     void ensure(int64_t nbytes)
     {
-        std::lock_guard<std::recursive_mutex> g(mu);
         if (buf.numel() >= nbytes) return;
+        const NoPython guard;
         // grow geometrically; the old contents (amax slot, status words of
         // earlier epochs) move along and the new tail is zero, so epochs
         // already handed out stay meaningful
@@ -116,16 +130,19 @@ struct Workspace {
         if (buf.numel()) n.narrow(0, 0, buf.numel()).copy_(buf);
         buf = n;
     }
-    // `reserve`: how many epochs the caller's sequence takes in total (the
-    // amax of a quantizing compress reserves 2), so that the wrap -- which
-    // zeroes the buffer, amax slot included -- never falls inside it
+    // room for a sequence: `nbytes`, and `epochs` that the wrap -- which zeroes
+    // the buffer, amax slot included -- does not fall between
+    void prepare(int64_t nbytes, int64_t epochs)
+    {
+        ensure(nbytes);
+        if (epoch + epochs <= kEpochLimit) return;
+        const NoPython guard;
+        buf.zero_();
+        epoch = 0;
+    }
     int64_t next_epoch(int64_t reserve)
     {
-        std::lock_guard<std::recursive_mutex> g(mu);
-        if (epoch + reserve > kEpochLimit) {
-            buf.zero_();
-            epoch = 0;
-        }
+        prepare(0, reserve);
         return ++epoch;
     }
     int64_t nbytes() const { return buf.numel(); }
@@ -139,24 +156,21 @@ struct Workspace {
 
 std::shared_ptr<Workspace> workspace(int dev)
 {
-    static std::mutex mu;
     static auto* all = new std::map<std::pair<int, void*>, std::shared_ptr<Workspace>>();   // (freed by the process)
     if (dev < 0) dev = c10::hip::current_device();
     void* st = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev).stream();
-    std::lock_guard<std::mutex> g(mu);
     auto& w = (*all)[{dev, st}];
     if (!w) w = std::make_shared<Workspace>(c10::Device(c10::kCUDA, dev));
     return w;
 }
 Workspace& ws_of(const Tensor& t) { return *workspace(t.get_device()); }
 
-using Lock = std::lock_guard<std::recursive_mutex>;
-
-// amax of a bf16 tensor (of its relu, of relu(x + bias)) under a fresh epoch
-int64_t amax(const Tensor& x, bool relu, const Tensor& bias, Workspace& w, int64_t reserve = 2)
+// amax of a bf16 tensor (of its relu, of relu(x + bias)) under the next epoch
+// of a prepared workspace
+constexpr int64_t kAmaxBytes = 256;
+int64_t amax(const Tensor& x, bool relu, const Tensor& bias, Workspace& w)
 {
-    w.ensure(256);
-    const int64_t e = w.next_epoch(reserve);
+    const int64_t e = ++w.epoch;
     void* st = stream_of(x);
     if (bias.defined())
         check(L.bs_amax_bias_relu(x.data_ptr(), x.size(0), x.size(1), bias.data_ptr(), w.buf.data_ptr(), w.nbytes(), e,
@@ -198,18 +212,15 @@ compress(const Tensor& dense, const Tensor& vals, const std::optional<Tensor>& o
     const c10::DeviceGuard guard(dense.device());
     const int64_t M = dense.size(0), N = dense.size(1), T = tiles(M, N);
     Workspace& w = ws_of(dense);
-    Lock lock(w.mu);
     Tensor q, scale;
-    int64_t amax_epoch = 0;
     if (quantize) {
-        amax_epoch = amax(dense, false, Tensor(), w);
         if (dense_out) q = empty({M, N}, dense, at::kFloat8_e4m3fn);
         scale = empty({}, dense, at::kFloat);
     }
     Tensor bitmask = empty({T * 512}, dense, at::kByte), prefix = empty({T + 1}, dense, at::kUInt32);
     Cursor c(offset, in_place, packed, dense);
-    w.ensure(L.bs_compress_workspace_bytes(M, N));
-    const int64_t epoch = w.next_epoch(1);
+    w.prepare(std::max(kAmaxBytes, L.bs_compress_workspace_bytes(M, N)), 2);
+    const int64_t amax_epoch = quantize ? amax(dense, false, Tensor(), w) : 0, epoch = ++w.epoch;
     const uint64_t* slot = quantize ? w.slot() : nullptr;
     if (packed) {
         check(L.bs_compress_packed(dense.data_ptr(), dtype_code(dense.scalar_type()), M, N, quantize, slot, amax_epoch,
@@ -245,40 +256,43 @@ struct Fp8 {
     Tensor codes, scale;
 };
 
-Fp8 quantize_rows(const Tensor& x, int64_t amax_epoch, Workspace& w)
+Fp8 rows_like(const Tensor& x) { return {empty(x.sizes(), x, at::kFloat8_e4m3fn), empty({}, x, at::kFloat)}; }
+Fp8 transposed_like(const Tensor& x)
 {
-    Fp8 o{empty(x.sizes(), x, at::kFloat8_e4m3fn), empty({}, x, at::kFloat)};
+    return {empty({x.size(1), x.size(0)}, x, at::kFloat8_e4m3fn), empty({}, x, at::kFloat)};
+}
+
+// codes of x, whose amax the workspace holds under `amax_epoch`
+void quantize_rows(const Tensor& x, const Fp8& o, int64_t amax_epoch, Workspace& w)
+{
     check(L.bs_quantize_e4m3fn(x.data_ptr(), x.numel(), o.codes.data_ptr(), ptr<float>(o.scale), w.buf.data_ptr(),
                                w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn");
-    return o;
+}
+
+// codes of x.T as a row-major matrix (and, `rows` defined, those of x)
+void quantize_t(const Tensor& x, const Tensor& rows, const Fp8& t, int64_t amax_epoch, Workspace& w)
+{
+    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), x.size(0), x.size(1), raw(rows), t.codes.data_ptr(), ptr<float>(t.scale),
+                                 w.buf.data_ptr(), w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn_t");
 }
 
 // to_fp8 of a row-major matrix
 Fp8 to_fp8(const Tensor& x, Workspace& w)
 {
     const Tensor c = x.contiguous();
-    Lock lock(w.mu);
-    return quantize_rows(c, amax(c, false, Tensor(), w), w);
-}
-
-// codes of x.T as a new row-major tensor (and, `rows`, those of x)
-std::pair<Tensor, Fp8> quantize_t(const Tensor& x, int64_t amax_epoch, bool rows, Workspace& w)
-{
-    const int64_t R = x.size(0), C = x.size(1);
-    Tensor q;
-    if (rows) q = empty({R, C}, x, at::kFloat8_e4m3fn);
-    Fp8 t{empty({C, R}, x, at::kFloat8_e4m3fn), empty({}, x, at::kFloat)};
-    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), R, C, raw(q), t.codes.data_ptr(), ptr<float>(t.scale), w.buf.data_ptr(),
-                                 w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn_t");
-    return {q, t};
+    const Fp8 o = rows_like(c);
+    w.prepare(kAmaxBytes, 1);
+    quantize_rows(c, o, amax(c, false, Tensor(), w), w);
+    return o;
 }
 
 // an operand multiplied from the right: column-major codes
 Fp8 right_operand(const Tensor& x, Workspace& w)
 {
     const Tensor c = x.contiguous();
-    Lock lock(w.mu);
-    Fp8 t = quantize_t(c, amax(c, false, Tensor(), w), false, w).second;
+    const Fp8 t = transposed_like(c);
+    w.prepare(kAmaxBytes, 1);
+    quantize_t(c, Tensor(), t, amax(c, false, Tensor(), w), w);
     return {t.codes.t(), t.scale};
 }
 
@@ -393,27 +407,21 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bi
     Tensor operand, operand_scale, codes, h_out, scale;
     Tensor bitmask = empty({T * 512}, x, at::kByte), prefix = empty({T + 1}, x, at::kUInt32);
     const Cursor c(offset, in_place, packed, x);
-    {
-        Lock lock(w.mu);
-        int64_t amax_epoch = 0;
-        if (fp8) {
-            amax_epoch = amax(z, true, b1, w);
-            scale = empty({}, x, at::kFloat);
-            operand_scale = square ? empty({}, x, at::kFloat) : scale;
-            operand = codes = empty({M, N}, x, at::kFloat8_e4m3fn);
-        } else {
-            // over z, unless the bias would be added again by a recount of z (the look-back's fallback)
-            operand = h_out = b1.defined() ? at::empty_like(z) : z;
-        }
-        w.ensure(L.bs_compress_workspace_bytes(M, N));
-        const int64_t epoch = w.next_epoch(1);
-        check(L.bs_compress_act(z.data_ptr(), raw(b1), M, N, square, (float)k, fp8, fp8 ? w.slot() : nullptr,
-                                amax_epoch, ptr<float>(scale), raw(codes),
-                                square && fp8 ? ptr<float>(operand_scale) : nullptr, raw(h_out), ptr<uint8_t>(bitmask),
-                                ptr<uint32_t>(prefix), vals.data_ptr(), vals.numel(), packed, ptr<int64_t>(c.in),
-                                ptr<int64_t>(c.next), ptr<int64_t>(c.start_out), ptr<int32_t>(err), w.buf.data_ptr(),
-                                w.nbytes(), epoch, stream_of(x)), "bs_compress_act");
+    if (fp8) {
+        scale = empty({}, x, at::kFloat);
+        operand_scale = square ? empty({}, x, at::kFloat) : scale;
+        operand = codes = empty({M, N}, x, at::kFloat8_e4m3fn);
+    } else {
+        // over z, unless the bias would be added again by a recount of z (the look-back's fallback)
+        operand = h_out = b1.defined() ? at::empty_like(z) : z;
     }
+    w.prepare(std::max(kAmaxBytes, L.bs_compress_workspace_bytes(M, N)), 2);
+    const int64_t amax_epoch = fp8 ? amax(z, true, b1, w) : 0, epoch = ++w.epoch;
+    check(L.bs_compress_act(z.data_ptr(), raw(b1), M, N, square, (float)k, fp8, fp8 ? w.slot() : nullptr, amax_epoch,
+                            ptr<float>(scale), raw(codes), square && fp8 ? ptr<float>(operand_scale) : nullptr,
+                            raw(h_out), ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix), vals.data_ptr(), vals.numel(),
+                            packed, ptr<int64_t>(c.in), ptr<int64_t>(c.next), ptr<int64_t>(c.start_out),
+                            ptr<int32_t>(err), w.buf.data_ptr(), w.nbytes(), epoch, stream_of(x)), "bs_compress_act");
     z.reset();          // (the down-projection does not need its room)
     Tensor y;
     if (fp8) {
@@ -452,28 +460,26 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
     const bool sums = need_b1 && !at::GradMode::is_enabled();
     Fp8 z8, zt8;
     if (sums || want8) {
-        Lock lock(w.mu);
-        int64_t epoch = 0;
-        if (want8) {
-            w.ensure(256);
-            epoch = w.next_epoch(2);
-        }
         Tensor db1;
         if (sums) out[2] = db1 = empty({h.N}, x, at::kBFloat16);
         const int64_t bytes = L.bs_grad_sums_workspace_bytes(h.M, h.N);
         Tensor part = empty({bytes}, x, at::kByte);
+        if (want8 && need_x) z8 = need_W1 ? Fp8{empty(dz.sizes(), dz, at::kFloat8_e4m3fn), Tensor()} : rows_like(dz);
+        if (want8 && need_W1) zt8 = transposed_like(dz);
+        int64_t epoch = 0;
+        if (want8) {
+            w.prepare(kAmaxBytes, 1);
+            epoch = ++w.epoch;
+        }
         check(L.bs_act_grad_sums(dz.data_ptr(), h.M, h.N, square, h.vals.data_ptr(), fp8 ? 1 : 0, h.vals.numel(),
                                  packed, ptr<uint8_t>(h.bitmask), ptr<uint32_t>(h.prefix), ptr<int64_t>(h.start), (float)k,
                                  ptr<float>(h.scale), raw(db1), want8 ? w.buf.data_ptr() : nullptr, epoch,
                                  part.data_ptr(), bytes, stream_of(x)), "bs_act_grad_sums");
-        part.reset();
-        h = Held();
         if (want8 && need_W1) {
-            const auto [q, t] = quantize_t(dz, epoch, need_x, w);
-            z8 = {q, t.scale};
-            zt8 = t;
+            quantize_t(dz, z8.codes, zt8, epoch, w);
+            z8.scale = zt8.scale;
         } else if (want8) {
-            z8 = quantize_rows(dz, epoch, w);
+            quantize_rows(dz, z8, epoch, w);
         }
     } else if (square) {
         check((packed ? L.bs_relu2_grad_packed : L.bs_relu2_grad)(
@@ -502,6 +508,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.def("init", &init);
     py::class_<Workspace, std::shared_ptr<Workspace>>(m, "Workspace")
+        .def(py::init<c10::Device>())
         .def_readonly("buf", &Workspace::buf)
         .def_readwrite("epoch", &Workspace::epoch)
         .def_property_readonly("nbytes", &Workspace::nbytes)
