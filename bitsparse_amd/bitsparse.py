@@ -178,6 +178,12 @@ class TensorBuffer:
             return self.offset.clone(), self.offset
         return self.offset, torch.empty(1, device=self.offset.device, dtype=torch.int64)
 
+    def native_cursor(self) -> tuple[Tensor | None, bool]:
+        """(cursor, in place) for one call of the native module, which returns
+        the advanced cursor: None stands for 0, where there is no cursor tensor
+        to advance in place."""
+        return (self.offset, True) if self.inplace_offset else (self._offset, False)
+
     def advance(self, out: Tensor) -> None:
         """Make ``out`` (from ``cursor``) the buffer's cursor."""
         if not self.inplace_offset:

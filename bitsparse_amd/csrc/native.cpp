@@ -192,6 +192,7 @@ struct Cursor {
     Tensor in, next, start, start_out;
     Cursor(const std::optional<Tensor>& offset, bool in_place, bool packed, const Tensor& like)
     {
+        TORCH_CHECK_VALUE(offset || !in_place, "no cursor to advance in place");
         if (offset) in = in_place ? offset->clone() : *offset;
         next = in_place ? *offset : empty({1}, like, at::kLong);
         start = in;

@@ -257,8 +257,9 @@ class _FFNBlock(Function):
 
     @staticmethod
     def forward(ctx, x, W1, b1, W2, b2, buf, fp8, square):
+        offset, in_place = buf.native_cursor()
         y, bitmask, prefix, start, buf._offset, scale = native().block_forward(
-            x, W1, b1, W2, b2, buf.vals, buf._offset, buf.err_flags, buf.inplace_offset, buf.pack_sbit, fp8, square,
+            x, W1, b1, W2, b2, buf.vals, offset, buf.err_flags, in_place, buf.pack_sbit, fp8, square,
             float(RELU2_SCALE))
         M, N = x.shape[0], W1.shape[0]
         ctx.h_sparse = BitsparseTensor(buf.vals, bitmask, prefix, (M, N), torch.float8_e4m3fn if fp8 else torch.bfloat16,

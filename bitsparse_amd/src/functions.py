@@ -241,7 +241,7 @@ def _to_tilesparse(dense: Tensor, scale: Tensor | None, sparse_data: TensorBuffe
 def _compress_into_buffer(dense: Tensor, buf: TensorBuffer, pack_sbit: bool, scale: Tensor | None) -> BitsparseTensor:
     """bs_compress / bs_compress_packed of a non-empty contiguous ``dense``, by the native host path."""
     bitmask, prefix, start, buf._offset, _, _ = native().compress(
-        dense, buf.vals, buf._offset, buf.inplace_offset, buf.err_flags, pack_sbit, False, False)
+        dense, buf.vals, *buf.native_cursor(), buf.err_flags, pack_sbit, False, False)
     grid_m, grid_n, *_ = tile_grid(*dense.shape, BLOCK_M, BLOCK_N)
     return BitsparseTensor(buf.vals, bitmask, prefix, dense.shape, dense.dtype, grid_m, grid_n, BLOCK_M, BLOCK_N,
                            scale=scale, vals_offset=start, pack_sbit=pack_sbit)
@@ -449,8 +449,7 @@ def quantize_and_compress(
         if not pack_sbit and sparse_data.vals.dtype != torch.float8_e4m3fn:
             raise TypeError(f"TensorBuffer stores {sparse_data.vals.dtype}, need float8_e4m3fn")
         bitmask, prefix, start, sparse_data._offset, q, scale = native().compress(
-            dense, sparse_data.vals, sparse_data._offset, sparse_data.inplace_offset, sparse_data.err_flags,
-            pack_sbit, True, dense_out)
+            dense, sparse_data.vals, *sparse_data.native_cursor(), sparse_data.err_flags, pack_sbit, True, dense_out)
         sp = BitsparseTensor(sparse_data.vals, bitmask, prefix, (M, N), torch.float8_e4m3fn, grid_m, grid_n,
                              BLOCK_M, BLOCK_N, scale=scale, vals_offset=start, pack_sbit=pack_sbit)
         return q, scale, sp

@@ -1,0 +1,57 @@
+"""The TensorBuffer's cursor as the native calls are given it (on the CPU: the
+native module is replaced by one that records its arguments)."""
+import types
+
+import pytest
+import torch
+
+from bitsparse_amd import layers
+from bitsparse_amd.bitsparse import TensorBuffer
+from bitsparse_amd.src import functions as F
+
+E4M3 = torch.float8_e4m3fn
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """What the native entry points were called with: (offset, in_place)."""
+    seen = []
+    meta = torch.zeros(1, dtype=torch.int64)
+
+    def compress(dense, vals, offset, in_place, *rest):
+        seen.append((offset, in_place))
+        return meta, meta, meta, offset if in_place else meta, None, None
+
+    def block_forward(x, W1, b1, W2, b2, vals, offset, err, in_place, *rest):
+        seen.append((offset, in_place))
+        return x.new_zeros((x.shape[0], W2.shape[0])), meta, meta, meta, offset if in_place else meta, None
+    stub = types.SimpleNamespace(compress=compress, block_forward=block_forward)
+    monkeypatch.setattr(F, "native", lambda: stub)
+    monkeypatch.setattr(layers, "native", lambda: stub)
+    monkeypatch.setattr(F.ops, "require_device", lambda *a: None)
+    monkeypatch.setattr(layers, "_block_ok", lambda *a: True)
+    return seen
+
+
+def _use(what, buf):
+    x = torch.ones((8, 8), dtype=torch.bfloat16)
+    if what == "compress":
+        F.dense_to_tilesparse(x, None, buf)
+    elif what == "quantize":
+        F.quantize_and_compress(x, buf)
+    else:
+        layers.FFNRelu.apply(x, x, x, sparse_data=buf)
+
+
+@pytest.mark.parametrize("what", ["compress", "quantize", "block"])
+def test_in_place_cursor_chosen_after_a_reset(calls, what):
+    """An in-place call always comes with the cursor tensor it advances."""
+    buf = TensorBuffer(128, device="cpu", dtype=E4M3 if what == "quantize" else torch.bfloat16)
+    buf.reset_buffer()
+    _use(what, buf)
+    assert calls[-1][0] is None and calls[-1][1] is False        # 0, no tensor needed
+    buf.reset_buffer()
+    buf.inplace_offset = True
+    _use(what, buf)
+    offset, in_place = calls[-1]
+    assert in_place is True and offset is buf.offset and int(offset) == 0
