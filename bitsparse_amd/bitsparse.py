@@ -151,6 +151,12 @@ class TensorBuffer:
         self._offset = torch.zeros(1, device=self.device, dtype=torch.int64)
         self.err_flags = torch.zeros(1, device=self.device, dtype=torch.int32)
 
+    def __setstate__(self, state: dict) -> None:
+        state = dict(state)
+        if "offset" in state:                    # saved when the cursor was a plain attribute
+            state["_offset"] = state.pop("offset")
+        self.__dict__.update(state)
+
     @property
     def offset(self) -> Tensor:
         """The cursor, a 1-element int64 tensor (after a reset, made when first asked for)."""

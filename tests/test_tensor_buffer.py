@@ -1,5 +1,7 @@
 """The TensorBuffer's cursor as the native calls are given it (on the CPU: the
 native module is replaced by one that records its arguments)."""
+import copy
+import pickle
 import types
 
 import pytest
@@ -55,3 +57,24 @@ def test_in_place_cursor_chosen_after_a_reset(calls, what):
     _use(what, buf)
     offset, in_place = calls[-1]
     assert in_place is True and offset is buf.offset and int(offset) == 0
+
+
+def test_buffers_of_earlier_files(calls):
+    """A TensorBuffer saved when the cursor was a plain attribute loads with
+    its cursor, and one copied or saved now keeps it, reset or not."""
+    buf = TensorBuffer(128, device="cpu")
+    state = dict(buf.__dict__)
+    state["offset"] = state.pop("_offset") + 5
+    old = TensorBuffer.__new__(TensorBuffer)
+    pickled = pickle.dumps(buf)
+    if hasattr(old, "__setstate__"):
+        old.__setstate__(state)
+    else:
+        old.__dict__.update(state)
+    _use("compress", old)
+    offset, in_place = calls[-1]
+    assert int(offset) == 5 and in_place is False
+    for again in (pickle.loads(pickled), copy.deepcopy(buf)):
+        assert int(again.offset) == 0 and again.offset is not buf.offset
+    buf.reset_buffer()
+    assert pickle.loads(pickle.dumps(buf))._offset is None
