@@ -201,6 +201,14 @@ class TensorBuffer:
         return bool(self.err_flags.item() != 0)
 
 
+def plain_cursor(buf: TensorBuffer) -> bool:
+    """The native calls may move ``buf``'s cursor themselves: its class leaves
+    ``cursor``, ``advance`` and ``offset`` as they are here."""
+    cls = type(buf)
+    return (getattr(cls, "cursor", None) is TensorBuffer.cursor and getattr(cls, "advance", None) is TensorBuffer.advance
+            and getattr(cls, "offset", None) is TensorBuffer.offset)
+
+
 def tile_grid(M: int, N: int, BLOCK_M: int, BLOCK_N: int) -> tuple[int, int, int, int, int]:
     """(grid_m, grid_n, num_tiles, TILE_NUMEL, TILE_BYTES) of a dense shape.
     Reference: lib_sparse/bitsparse.py:120-127."""

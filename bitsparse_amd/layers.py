@@ -17,7 +17,7 @@ from torch import Tensor
 from torch.autograd import Function, forward_ad
 
 from . import config
-from .bitsparse import BitsparseTensor, TensorBuffer
+from .bitsparse import BitsparseTensor, TensorBuffer, plain_cursor
 from .config import BLOCK_M, BLOCK_N, RELU2_SCALE
 from .fp8 import is_fp8, matmul, to_fp8
 from ._lib import native
@@ -222,7 +222,7 @@ def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor |
     TensorBuffer of the stored type, outside autocast, tracing, forward-mode
     AD and the options that choose another path.  Everything else takes the
     layers' separate nodes, with their errors."""
-    if sparse_data is None or not (_plain(x) and _plain(W1) and _plain(W2)):
+    if sparse_data is None or not (_plain(x) and _plain(W1) and _plain(W2) and plain_cursor(sparse_data)):
         return False
     if USE_FUSED_UP or config.CACHE_FP8_MATMUl or not sparse_matmul.USE_LDS_GEMM or not math.isfinite(RELU2_SCALE):
         return False

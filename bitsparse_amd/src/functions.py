@@ -28,7 +28,7 @@ from torch import Tensor
 from . import hip_operators as ops
 from .bitpacking import pack_bits
 from .._lib import native
-from ..bitsparse import BitsparseTensor, TensorBuffer, tile_grid
+from ..bitsparse import BitsparseTensor, TensorBuffer, plain_cursor, tile_grid
 from ..config import BLOCK_M, BLOCK_N
 from ..fp8 import is_fp8
 
@@ -220,7 +220,8 @@ def _to_tilesparse(dense: Tensor, scale: Tensor | None, sparse_data: TensorBuffe
                                vals_offset=vals_offset, pack_sbit=pack_sbit)
 
     _check_buffer(sparse_data, dense.dtype, pack_sbit)
-    if not relu and dense.numel() > 0 and (pack_sbit or sparse_data.vals.dtype == dense.dtype):
+    if (not relu and dense.numel() > 0 and (pack_sbit or sparse_data.vals.dtype == dense.dtype)
+            and plain_cursor(sparse_data)):
         return _compress_into_buffer(dense, sparse_data, pack_sbit, scale)
     fused = dict(relu=True, relu_out=dense) if relu else {}
     if pack_sbit:
@@ -444,7 +445,7 @@ def quantize_and_compress(
     dense = dense.contiguous()
     M, N = dense.shape
     grid_m, grid_n, num_tiles, TILE_NUMEL, TILE_BYTES = tile_grid(M, N, BLOCK_M, BLOCK_N)
-    if sparse_data is not None and not _relu and M * N > 0:
+    if sparse_data is not None and not _relu and M * N > 0 and plain_cursor(sparse_data):
         _check_buffer(sparse_data, torch.float8_e4m3fn, pack_sbit)
         if not pack_sbit and sparse_data.vals.dtype != torch.float8_e4m3fn:
             raise TypeError(f"TensorBuffer stores {sparse_data.vals.dtype}, need float8_e4m3fn")

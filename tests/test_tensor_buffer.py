@@ -12,6 +12,7 @@ from bitsparse_amd.bitsparse import TensorBuffer
 from bitsparse_amd.src import functions as F
 
 E4M3 = torch.float8_e4m3fn
+BLOCK_OK = layers._block_ok
 
 
 @pytest.fixture
@@ -78,3 +79,43 @@ def test_buffers_of_earlier_files(calls):
         assert int(again.offset) == 0 and again.offset is not buf.offset
     buf.reset_buffer()
     assert pickle.loads(pickle.dumps(buf))._offset is None
+
+
+@pytest.mark.parametrize("what", ["compress", "quantize", "block"])
+@pytest.mark.parametrize("hook", ["cursor", "advance", "offset"])
+def test_buffers_with_a_cursor_of_their_own(calls, monkeypatch, what, hook):
+    """A subclass that takes over the cursor's protocol is asked through it:
+    the native calls, which go past it, are for the plain buffer."""
+    used = []
+
+    class Own(TensorBuffer):
+        pass
+    if hook == "offset":
+        def get(self):
+            used.append(hook)
+            return TensorBuffer.offset.fget(self)
+        Own.offset = property(get, TensorBuffer.offset.fset)
+    else:
+        def method(self, *a):
+            used.append(hook)
+            return getattr(TensorBuffer, hook)(self, *a)
+        setattr(Own, hook, method)
+    for op in ("compress_into", "amax_into_workspace"):
+        monkeypatch.setattr(F.ops, op, lambda *a, **k: 1)
+    buf = Own(128, device="cpu", dtype=E4M3 if what == "quantize" else torch.bfloat16)
+    if what == "block":
+        monkeypatch.setattr(layers, "_plain", lambda t: True)
+        x = torch.ones((16, 16), dtype=torch.bfloat16)
+        args = (None, None), (False, torch.bfloat16)
+        assert BLOCK_OK(x, x, x, *args[0], TensorBuffer(512, device="cpu"), *args[1])
+        assert not BLOCK_OK(x, x, x, *args[0], buf, *args[1])
+        return
+    _use(what, buf)
+    assert used and not calls
+
+
+def test_plain_subclass_keeps_the_native_calls(calls):
+    class Plain(TensorBuffer):
+        pass
+    _use("compress", Plain(128, device="cpu"))
+    assert calls
