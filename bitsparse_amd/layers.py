@@ -222,6 +222,8 @@ def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor |
     TensorBuffer of the stored type, outside autocast, tracing, forward-mode
     AD and the options that choose another path.  Everything else takes the
     layers' separate nodes, with their errors."""
+    if torch.compiler.is_compiling():        # first: a tracer does not follow the addresses below
+        return False
     if sparse_data is None or not (_plain(x) and _plain(W1) and _plain(W2) and plain_cursor(sparse_data)):
         return False
     if USE_FUSED_UP or config.CACHE_FP8_MATMUl or not sparse_matmul.USE_LDS_GEMM or not math.isfinite(RELU2_SCALE):
@@ -247,8 +249,7 @@ def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor |
     if not (x.device == W1.device == W2.device == buf.device) or any(
             b is not None and b.device != x.device for b in (b1, b2)):
         return False
-    return (not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
-            and not torch.compiler.is_compiling())
+    return not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
 
 
 class _FFNBlock(Function):
