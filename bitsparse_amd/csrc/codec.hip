@@ -485,7 +485,9 @@ __device__ uint32_t wave_lookback_grouped(const CompressArgs& a, uint32_t u, uin
 #ifndef BS_STREAM_ROUNDS
 #define BS_STREAM_ROUNDS 2
 #endif
-constexpr int kRoundsPerPass = BS_STREAM_ROUNDS;   // rounds written before each store pass (even: ranked in pairs)
+constexpr int kRoundsPerPass = BS_STREAM_ROUNDS;   // rounds written before each store pass
+static_assert(kRoundsPerPass > 0 && kRoundsPerPass % 2 == 0 && 8 % kRoundsPerPass == 0,
+              "rounds are ranked in pairs, and whole passes make up a tile's eight rounds");
 // >= 15 (pending) + 512 per round + 8 (overrun), a multiple of 16
 constexpr int kRingElems = 512 * kRoundsPerPass + 32;
 
