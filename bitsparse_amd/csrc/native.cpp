@@ -26,9 +26,9 @@ using at::Tensor;
 // libbitsparse_hip.so (the path Python loads, so that both use one library)
 // ---------------------------------------------------------------------------
 #define BS_FUNCS(F)                                                                                              \
-    F(bs_last_error) F(bs_compress_workspace_bytes) F(bs_compress) F(bs_compress_relu) F(bs_compress_packed)     \
+    F(bs_abi_version) F(bs_last_error) F(bs_compress_workspace_bytes) F(bs_compress) F(bs_compress_packed)       \
     F(bs_compress_act) F(bs_amax) F(bs_amax_relu) F(bs_amax_bias_relu) F(bs_quantize_e4m3fn)                     \
-    F(bs_quantize_e4m3fn_t) F(bs_transpose_u8) F(bs_widen_e4m3fn) F(bs_decompress) F(bs_decompress_packed)       \
+    F(bs_quantize_e4m3fn_t) F(bs_widen_e4m3fn) F(bs_decompress) F(bs_decompress_packed)                          \
     F(bs_relu_grad) F(bs_relu2_grad) F(bs_relu2_grad_packed) F(bs_grad_sums_workspace_bytes) F(bs_act_grad_sums) \
     F(bs_col_sum_workspace_bytes) F(bs_col_sum) F(bs_gemm_compressed_b_workspace_bytes) F(bs_gemm_compressed_b)  \
     F(bs_gemm_compressed_b_packed_workspace_bytes) F(bs_gemm_compressed_b_packed)                                \
@@ -43,12 +43,18 @@ struct Lib {
 void init(const std::string& path)
 {
     void* h = dlopen(path.c_str(), RTLD_NOW);
-    TORCH_CHECK(h != nullptr, "bitsparse_amd: ", dlerror());
-#define F(name)                                                        \
-    L.name = reinterpret_cast<decltype(&::name)>(dlsym(h, #name));     \
-    TORCH_CHECK(L.name != nullptr, "bitsparse_amd: " #name " missing");
+    if (h == nullptr) throw py::import_error(std::string("bitsparse_amd: ") + dlerror());
+    Lib lib;
+#define F(name)                                                      \
+    lib.name = reinterpret_cast<decltype(&::name)>(dlsym(h, #name)); \
+    if (lib.name == nullptr) throw py::import_error("bitsparse_amd: " #name " missing in " + path);
     BS_FUNCS(F)
 #undef F
+    // the header compiled in here and the library are built apart: one version, or shifted arguments
+    if (lib.bs_abi_version() != BS_ABI_VERSION)
+        throw py::import_error("bitsparse_amd/_native was built for ABI " + std::to_string(BS_ABI_VERSION) + ", " + path +
+                               " has " + std::to_string(lib.bs_abi_version()) + "; rebuild both");
+    L = lib;
 }
 
 void check(int rc, const char* what)
@@ -507,7 +513,9 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
+    m.attr("EPOCH_LIMIT") = kEpochLimit;
     m.def("init", &init);
+    m.def("abi_version", [] { return L.bs_abi_version(); });
     py::class_<Workspace, std::shared_ptr<Workspace>>(m, "Workspace")
         .def(py::init<c10::Device>())
         .def_readonly("buf", &Workspace::buf)

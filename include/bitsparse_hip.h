@@ -48,7 +48,8 @@ extern "C" {
 /* Last error message of the calling thread ("" when none). */
 const char* bs_last_error(void);
 
-/* ABI version of this library (bumped when an entry point changes). */
+/* ABI version (bumped when an entry point changes): of this header, and of a built library. */
+#define BS_ABI_VERSION 17
 int bs_abi_version(void);
 
 /*
