@@ -62,7 +62,9 @@ void check(int rc, const char* what)
     if (rc == BS_OK) return;
     const char* msg = L.bs_last_error();
     if (rc == BS_ERR_INVALID) TORCH_CHECK_VALUE(false, what, ": ", msg);
-    TORCH_CHECK(false, what, " failed (", rc, "): ", msg);
+    py::set_error(py::module_::import("bitsparse_amd._lib").attr("BitsparseHipError"),
+                  (std::string(what) + " failed (" + std::to_string(rc) + "): " + msg).c_str());
+    throw py::error_already_set();
 }
 
 void* stream_of(const Tensor& t)
@@ -515,6 +517,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.attr("EPOCH_LIMIT") = kEpochLimit;
     m.def("init", &init);
+    m.def("check", &check);
     m.def("abi_version", [] { return L.bs_abi_version(); });
     py::class_<Workspace, std::shared_ptr<Workspace>>(m, "Workspace")
         .def(py::init<c10::Device>())

@@ -33,3 +33,17 @@ def test_library_of_another_version_is_refused(tmp_path):
         assert native.abi_version() == _lib.ABI_VERSION          # still bound to the library it had
     finally:
         native.init(_lib.LIB_PATH)
+
+
+@pytest.mark.parametrize("status,error", [(_lib.BS_OK, None), (_lib.BS_ERR_INVALID, ValueError),
+                                          (2, _lib.BitsparseHipError)])
+def test_errors_of_native_calls(status, error):
+    """The native calls raise what the Python ones raise for the same status."""
+    native = _lib.native()
+    for check in (_lib.check, native.check):
+        if error is None:
+            check(status, "bs_compress")
+            continue
+        with pytest.raises(Exception) as e:
+            check(status, "bs_compress")
+        assert type(e.value) is error and str(e.value).startswith("bs_compress")
