@@ -78,6 +78,7 @@ T* ptr(const Tensor& t)
     return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr;
 }
 void* raw(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+std::optional<Tensor> optional(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
 int dtype_code(at::ScalarType t)
 {
@@ -243,8 +244,7 @@ compress(const Tensor& dense, const Tensor& vals, const std::optional<Tensor>& o
                             vals.numel(), ptr<int64_t>(c.in), 0, ptr<int64_t>(c.next), ptr<int64_t>(c.start_out), 1,
                             ptr<int32_t>(err), w.buf.data_ptr(), w.nbytes(), epoch, stream_of(dense)), "bs_compress");
     }
-    return {bitmask, prefix, c.start, c.next, q.defined() ? std::optional<Tensor>(q) : std::nullopt,
-            scale.defined() ? std::optional<Tensor>(scale) : std::nullopt};
+    return {bitmask, prefix, c.start, c.next, optional(q), optional(scale)};
 }
 
 void decompress(const Tensor& vals, at::ScalarType stored, bool packed, const Tensor& bitmask, const Tensor& prefix,
@@ -330,6 +330,16 @@ struct Held {
     double k;
 };
 
+// `held`: (values, bitmask, prefix, start, scale), taken out of the list, so
+// that they go once the last kernel that reads them is queued
+Held take_held(const py::list& held, int64_t M, int64_t N, bool packed, bool fp8, bool square, double k)
+{
+    Held h{held[0].cast<Tensor>(), held[1].cast<Tensor>(), held[2].cast<Tensor>(), held[3].cast<Tensor>(),
+           held[4].is_none() ? Tensor() : held[4].cast<Tensor>(), M, N, packed, fp8, square, k};
+    held.attr("clear")();
+    return h;
+}
+
 // C = A @ op(B), B compressed [K, N]: A row-major (a_layout 1) or A.T
 // row-major (0) in `a` with row stride lda; a_scale: A is e4m3fn
 Tensor gemm_compressed(const Tensor& a, int64_t M, int64_t K, int64_t lda, int64_t a_layout,
@@ -388,6 +398,91 @@ Tensor col_sum(const Tensor& g)
     return out;
 }
 
+// The activation step inside a block, on its up-projection z, which nothing
+// reads afterwards: r = relu(z + bias) compressed, and what the down-projection
+// multiplies -- r or (square) k r^2, in bf16 (over z where that leaves a recount
+// of z, the look-back's fallback, right: no bias to be added again), or (fp8) as
+// e4m3fn codes with their scale, as to_fp8 makes them.
+struct Activation {
+    Tensor operand, operand_scale, bitmask, prefix, start, next, scale;
+};
+
+Activation activate(const Tensor& z, const Tensor& bias, const Tensor& vals, const std::optional<Tensor>& offset,
+                    const Tensor& err, bool in_place, bool packed, bool fp8, bool square, double k)
+{
+    const int64_t M = z.size(0), N = z.size(1), T = tiles(M, N);
+    Workspace& w = ws_of(z);
+    const Cursor c(offset, in_place, packed, z);
+    Activation a;
+    a.bitmask = empty({T * 512}, z, at::kByte);
+    a.prefix = empty({T + 1}, z, at::kUInt32);
+    a.start = c.start;
+    a.next = c.next;
+    if (fp8) {
+        a.scale = empty({}, z, at::kFloat);
+        a.operand_scale = square ? empty({}, z, at::kFloat) : a.scale;
+        a.operand = empty({M, N}, z, at::kFloat8_e4m3fn);
+    } else {
+        a.operand = bias.defined() ? at::empty_like(z) : z;
+    }
+    w.prepare(std::max(kAmaxBytes, L.bs_compress_workspace_bytes(M, N)), 2);
+    const int64_t amax_epoch = fp8 ? amax(z, true, bias, w) : 0, epoch = ++w.epoch;
+    check(L.bs_compress_act(z.data_ptr(), raw(bias), M, N, square, (float)k, fp8, fp8 ? w.slot() : nullptr, amax_epoch,
+                            ptr<float>(a.scale), fp8 ? raw(a.operand) : nullptr,
+                            square && fp8 ? ptr<float>(a.operand_scale) : nullptr, fp8 ? nullptr : raw(a.operand),
+                            ptr<uint8_t>(a.bitmask), ptr<uint32_t>(a.prefix), vals.data_ptr(), vals.numel(), packed,
+                            ptr<int64_t>(c.in), ptr<int64_t>(c.next), ptr<int64_t>(c.start_out), ptr<int32_t>(err),
+                            w.buf.data_ptr(), w.nbytes(), epoch, stream_of(z)), "bs_compress_act");
+    return a;
+}
+
+// The activation's gradient, in place: dz = relu'(.) dh or (square) 2 k r dh,
+// and from the pass that writes it the bias gradient (its column sums) and its
+// e4m3fn codes, row-major (`rows`) and transposed (`cols`), with their scale,
+// each if asked for.  Gives the activation's tensors up once they are read.
+struct ActGrad {
+    Tensor bias;
+    Fp8 rows, cols;
+};
+
+ActGrad act_grad(const Tensor& dz, Held& h, bool bias, bool rows, bool cols)
+{
+    const int stored = h.fp8 ? 1 : 0;
+    ActGrad o;
+    if (bias || rows || cols) {
+        Workspace& w = ws_of(dz);
+        if (bias) o.bias = empty({h.N}, dz, at::kBFloat16);
+        const int64_t bytes = L.bs_grad_sums_workspace_bytes(h.M, h.N);
+        const Tensor part = empty({bytes}, dz, at::kByte);
+        if (rows) o.rows = cols ? Fp8{empty(dz.sizes(), dz, at::kFloat8_e4m3fn), Tensor()} : rows_like(dz);
+        if (cols) o.cols = transposed_like(dz);
+        int64_t epoch = 0;
+        if (rows || cols) {
+            w.prepare(kAmaxBytes, 1);
+            epoch = ++w.epoch;
+        }
+        check(L.bs_act_grad_sums(dz.data_ptr(), h.M, h.N, h.square, h.vals.data_ptr(), stored, h.vals.numel(), h.packed,
+                                 ptr<uint8_t>(h.bitmask), ptr<uint32_t>(h.prefix), ptr<int64_t>(h.start), (float)h.k,
+                                 ptr<float>(h.scale), raw(o.bias), rows || cols ? w.buf.data_ptr() : nullptr, epoch,
+                                 part.data_ptr(), bytes, stream_of(dz)), "bs_act_grad_sums");
+        if (cols) {
+            quantize_t(dz, o.rows.codes, o.cols, epoch, w);
+            o.rows.scale = o.cols.scale;
+        } else if (rows) {
+            quantize_rows(dz, o.rows, epoch, w);
+        }
+    } else if (h.square) {
+        check((h.packed ? L.bs_relu2_grad_packed : L.bs_relu2_grad)(
+                  dz.data_ptr(), h.M, h.N, h.vals.data_ptr(), stored, h.vals.numel(), ptr<uint8_t>(h.bitmask),
+                  ptr<uint32_t>(h.prefix), ptr<int64_t>(h.start), (float)h.k, ptr<float>(h.scale), stream_of(dz)),
+              "bs_relu2_grad");
+    } else {
+        check(L.bs_relu_grad(dz.data_ptr(), h.M, h.N, ptr<uint8_t>(h.bitmask), stream_of(dz)), "bs_relu_grad");
+    }
+    h = Held();
+    return o;
+}
+
 // y = act(x @ W1.T + b1) @ W2.T + b2 with act(z) = relu(z) or k relu(z)^2 saved
 // compressed: the products, quantizations and kernels of the separate nodes
 // (matmul, the bias adds, ReluLinear / Relu2Linear), with their roundings.
@@ -398,13 +493,11 @@ Tensor col_sum(const Tensor& g)
 // has checked the operands.
 // -> (y, bitmask, prefix, start of the values, advanced cursor, scale)
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, std::optional<Tensor>>
-block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bias1, const Tensor& W2,
-              const std::optional<Tensor>& bias2, const Tensor& vals, const std::optional<Tensor>& offset,
+block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& b1, const Tensor& W2,
+              const std::optional<Tensor>& b2, const Tensor& vals, const std::optional<Tensor>& offset,
               const Tensor& err, bool in_place, bool packed, bool fp8, bool square, double k)
 {
     const c10::DeviceGuard guard(x.device());
-    const Tensor b1 = bias1.value_or(Tensor()), b2 = bias2.value_or(Tensor());
-    const int64_t M = x.size(0), N = W1.size(0), T = tiles(M, N);
     Workspace& w = ws_of(x);
     Tensor z;
     if (fp8) {
@@ -413,48 +506,27 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& bi
     } else {
         z = at::mm(x, W1.t());
     }
-    Tensor operand, operand_scale, codes, h_out, scale;
-    Tensor bitmask = empty({T * 512}, x, at::kByte), prefix = empty({T + 1}, x, at::kUInt32);
-    const Cursor c(offset, in_place, packed, x);
-    if (fp8) {
-        scale = empty({}, x, at::kFloat);
-        operand_scale = square ? empty({}, x, at::kFloat) : scale;
-        operand = codes = empty({M, N}, x, at::kFloat8_e4m3fn);
-    } else {
-        // over z, unless the bias would be added again by a recount of z (the look-back's fallback)
-        operand = h_out = b1.defined() ? at::empty_like(z) : z;
-    }
-    w.prepare(std::max(kAmaxBytes, L.bs_compress_workspace_bytes(M, N)), 2);
-    const int64_t amax_epoch = fp8 ? amax(z, true, b1, w) : 0, epoch = ++w.epoch;
-    check(L.bs_compress_act(z.data_ptr(), raw(b1), M, N, square, (float)k, fp8, fp8 ? w.slot() : nullptr, amax_epoch,
-                            ptr<float>(scale), raw(codes), square && fp8 ? ptr<float>(operand_scale) : nullptr,
-                            raw(h_out), ptr<uint8_t>(bitmask), ptr<uint32_t>(prefix), vals.data_ptr(), vals.numel(),
-                            packed, ptr<int64_t>(c.in), ptr<int64_t>(c.next), ptr<int64_t>(c.start_out),
-                            ptr<int32_t>(err), w.buf.data_ptr(), w.nbytes(), epoch, stream_of(x)), "bs_compress_act");
+    const Activation a = activate(z, b1.value_or(Tensor()), vals, offset, err, in_place, packed, fp8, square, k);
     z.reset();          // (the down-projection does not need its room)
     Tensor y;
     if (fp8) {
         const Fp8 b = to_fp8(W2, w);
-        y = fp8_mm({operand, operand_scale}, {b.codes.t(), b.scale}, at::kBFloat16);
+        y = fp8_mm({a.operand, a.operand_scale}, {b.codes.t(), b.scale}, at::kBFloat16);
     } else {
-        y = at::mm(operand, W2.t());
+        y = at::mm(a.operand, W2.t());
     }
-    if (b2.defined()) y.add_(b2);
-    return {y, bitmask, prefix, c.start, c.next, scale.defined() ? std::optional<Tensor>(scale) : std::nullopt};
+    if (b2) y.add_(*b2);
+    return {y, a.bitmask, a.prefix, a.start, a.next, optional(a.scale)};
 }
 
-// (dx, dW1, db1, dW2, db2), each where `need` asks for it.  `held`: (values,
-// bitmask, prefix, start, scale) of the activation, taken out of the list, so
-// that they go once the last kernel that reads them is queued.
+// (dx, dW1, db1, dW2, db2), each where `need` asks for it
 std::vector<std::optional<Tensor>>
 block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const py::list& held, bool packed,
                bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
                const std::vector<bool>& need)
 {
     const c10::DeviceGuard guard(x.device());
-    Held h{held[0].cast<Tensor>(), held[1].cast<Tensor>(), held[2].cast<Tensor>(), held[3].cast<Tensor>(),
-           held[4].is_none() ? Tensor() : held[4].cast<Tensor>(), x.size(0), W1.size(0), packed, fp8, square, k};
-    held.attr("clear")();
+    Held h = take_held(held, x.size(0), W1.size(0), packed, fp8, square, k);
     const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3], need_b2 = need[4];
     std::vector<std::optional<Tensor>> out(5);
     Workspace& w = ws_of(x);
@@ -463,47 +535,15 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
     if (fp8) g8 = to_fp8(g, w);
     if (need_W2) out[3] = down_weight_grad(fp8 ? g8.codes : g, g8.scale, h);
     if (!(need_x || need_W1 || need_b1)) return out;
-    Tensor dz = fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
+    const Tensor dz = fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
     g8 = Fp8();
-    const bool want8 = fp8 && (need_x || need_W1);
     const bool sums = need_b1 && !at::GradMode::is_enabled();
-    Fp8 z8, zt8;
-    if (sums || want8) {
-        Tensor db1;
-        if (sums) out[2] = db1 = empty({h.N}, x, at::kBFloat16);
-        const int64_t bytes = L.bs_grad_sums_workspace_bytes(h.M, h.N);
-        Tensor part = empty({bytes}, x, at::kByte);
-        if (want8 && need_x) z8 = need_W1 ? Fp8{empty(dz.sizes(), dz, at::kFloat8_e4m3fn), Tensor()} : rows_like(dz);
-        if (want8 && need_W1) zt8 = transposed_like(dz);
-        int64_t epoch = 0;
-        if (want8) {
-            w.prepare(kAmaxBytes, 1);
-            epoch = ++w.epoch;
-        }
-        check(L.bs_act_grad_sums(dz.data_ptr(), h.M, h.N, square, h.vals.data_ptr(), fp8 ? 1 : 0, h.vals.numel(),
-                                 packed, ptr<uint8_t>(h.bitmask), ptr<uint32_t>(h.prefix), ptr<int64_t>(h.start), (float)k,
-                                 ptr<float>(h.scale), raw(db1), want8 ? w.buf.data_ptr() : nullptr, epoch,
-                                 part.data_ptr(), bytes, stream_of(x)), "bs_act_grad_sums");
-        if (want8 && need_W1) {
-            quantize_t(dz, z8.codes, zt8, epoch, w);
-            z8.scale = zt8.scale;
-        } else if (want8) {
-            quantize_rows(dz, z8, epoch, w);
-        }
-    } else if (square) {
-        check((packed ? L.bs_relu2_grad_packed : L.bs_relu2_grad)(
-                  dz.data_ptr(), h.M, h.N, h.vals.data_ptr(), fp8 ? 1 : 0, h.vals.numel(), ptr<uint8_t>(h.bitmask),
-                  ptr<uint32_t>(h.prefix), ptr<int64_t>(h.start), (float)k, ptr<float>(h.scale), stream_of(x)),
-              "bs_relu2_grad");
-    } else {
-        check(L.bs_relu_grad(dz.data_ptr(), h.M, h.N, ptr<uint8_t>(h.bitmask), stream_of(x)), "bs_relu_grad");
-    }
-    h = Held();
-    if (need_b1 && !sums) out[2] = col_sum(dz);
+    const ActGrad a = act_grad(dz, h, sums, fp8 && need_x, fp8 && need_W1);
+    if (need_b1) out[2] = sums ? a.bias : col_sum(dz);
     if (fp8) {
         const at::ScalarType gd = grad_dtype.value_or(at::kFloat8_e4m3fn);
-        if (need_x) out[0] = widened(fp8_mm(z8, right_operand(W1, w), gd));
-        if (need_W1) out[1] = widened(fp8_mm(zt8, right_operand(x, w), gd));
+        if (need_x) out[0] = widened(fp8_mm(a.rows, right_operand(W1, w), gd));
+        if (need_W1) out[1] = widened(fp8_mm(a.cols, right_operand(x, w), gd));
     } else {
         if (need_x) out[0] = at::mm(dz, W1);
         if (need_W1) out[1] = at::mm(dz.t(), x);      // W1's own layout, as autograd forms it
@@ -534,4 +574,31 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("gemm_compressed", &gemm_compressed);
     m.def("block_forward", &block_forward);
     m.def("block_backward", &block_backward);
+    // the block's steps by themselves
+    m.def("activate", [](const Tensor& z, const std::optional<Tensor>& bias, const Tensor& vals,
+                         const std::optional<Tensor>& offset, const Tensor& err, bool in_place, bool packed, bool fp8,
+                         bool square, double k) {
+        const c10::DeviceGuard guard(z.device());
+        const Activation a = activate(z, bias.value_or(Tensor()), vals, offset, err, in_place, packed, fp8, square, k);
+        return std::make_tuple(a.operand, optional(a.operand_scale), a.bitmask, a.prefix, a.start, a.next,
+                               optional(a.scale));
+    });
+    m.def("act_grad", [](const Tensor& dz, const py::list& held, bool packed, bool fp8, bool square, double k, bool bias,
+                         bool rows, bool cols) {
+        const c10::DeviceGuard guard(dz.device());
+        Held h = take_held(held, dz.size(0), dz.size(1), packed, fp8, square, k);
+        const ActGrad a = act_grad(dz, h, bias, rows, cols);
+        return std::make_tuple(optional(a.bias), optional(a.rows.codes), optional(a.cols.codes), optional(a.rows.scale),
+                               optional(a.cols.scale));
+    });
+    m.def("col_sum", &col_sum);
+    m.def("quantize_t", [](const Tensor& x, bool rows) {
+        const c10::DeviceGuard guard(x.device());
+        Workspace& w = ws_of(x);
+        const Fp8 t = transposed_like(x);
+        const Tensor q = rows ? empty(x.sizes(), x, at::kFloat8_e4m3fn) : Tensor();
+        w.prepare(kAmaxBytes, 1);
+        quantize_t(x, q, t, amax(x, false, Tensor(), w), w);
+        return std::make_tuple(optional(q), t.codes, t.scale);
+    });
 }

@@ -362,56 +362,6 @@ def relu2_quantize_and_compress(z: Tensor, sparse_data: TensorBuffer,
     return scale, sp, ops.amax_relu2_from(z.device, amax_epoch, k)
 
 
-def activate_ok(z: Tensor, bias: Tensor | None, sparse_data: TensorBuffer | None, k: float) -> bool:
-    """``activate_and_compress`` takes this product: a TensorBuffer to compress
-    into, whole 16-byte chunks in every row, a finite k."""
-    return (sparse_data is not None and z.dim() == 2 and z.is_contiguous() and z.dtype == torch.bfloat16
-            and 0 < z.numel() < 2 ** 31 and z.shape[1] % 8 == 0 and z.shape[1] < 2 ** 28 and z.data_ptr() % 16 == 0
-            and (bias is None or bias.data_ptr() % 16 == 0) and math.isfinite(k))
-
-
-def activate_and_compress(z: Tensor, bias: Tensor | None, sparse_data: TensorBuffer, pack_sbit: bool, fp8: bool,
-                          square: bool) -> tuple[Tensor, Tensor | None, BitsparseTensor]:
-    """The activation step of an MLP block on its up-projection z, which
-    nothing reads afterwards: r = relu(z + bias) compressed into
-    ``sparse_data`` and the down-projection's operand -- r, or with ``square``
-    k r^2; in bf16 (over z, or new), or with ``fp8`` as e4m3fn codes with their
-    scale (``to_fp8`` of it).  Bit for bit the separate bias add,
-    relu_[quantize_]and_compress, square and quantize.  Needs ``activate_ok``.
-    Returns (operand, its scale or None, compressed r)."""
-    stored = torch.float8_e4m3fn if fp8 else torch.bfloat16
-    _check_buffer(sparse_data, stored, pack_sbit)
-    if not pack_sbit and sparse_data.vals.dtype != stored:
-        raise TypeError(f"TensorBuffer stores {sparse_data.vals.dtype} but the values are {stored}")
-    M, N = z.shape
-    dev = z.device
-    grid_m, grid_n, num_tiles, TILE_NUMEL, TILE_BYTES = tile_grid(M, N, BLOCK_M, BLOCK_N)
-    bitmask = torch.empty(num_tiles * TILE_BYTES, device=dev, dtype=torch.uint8)
-    prefix = torch.empty(num_tiles + 1, device=dev, dtype=torch.uint32)
-    start = torch.empty(1, device=dev, dtype=torch.int64) if pack_sbit else None
-    cursor, advanced = sparse_data.cursor()
-    scale = operand_scale = None
-    fused = {}
-    if fp8:
-        epoch = (ops.amax_into_workspace(z, relu=True) if bias is None
-                 else ops.amax_bias_relu_into_workspace(z, bias))
-        scale = torch.empty((), device=dev, dtype=torch.float32)
-        operand_scale = torch.empty((), device=dev, dtype=torch.float32) if square else scale
-        operand = torch.empty((M, N), device=dev, dtype=stored)
-        fused = dict(codes_out=operand, scale_out=scale, amax_epoch=epoch,
-                     codes_scale_out=operand_scale if square else None)
-    else:
-        # over z where that leaves a recount of z (the look-back's fallback) right
-        operand = z if bias is None and not square else torch.empty_like(z)
-        fused = dict(h_out=operand)
-    ops.compress_act_into(z, bias, square, bitmask, prefix, sparse_data.vals, pack_sbit, cursor, advanced, start,
-                          sparse_data.err_flags, **fused)
-    sparse_data.advance(advanced)
-    sp = BitsparseTensor(sparse_data.vals, bitmask, prefix, (M, N), stored, grid_m, grid_n, BLOCK_M, BLOCK_N,
-                         scale=scale, vals_offset=start if pack_sbit else cursor, pack_sbit=pack_sbit)
-    return operand, operand_scale, sp
-
-
 def relu_quantize_and_compress(
     z: Tensor, sparse_data: TensorBuffer | None = None, pack_sbit: bool = False,
     dense_out: bool = True,

@@ -302,42 +302,6 @@ def amax_into_workspace(x: Tensor, relu: bool = False, reserve: int = 2) -> int:
     return epoch
 
 
-def amax_bias_relu_into_workspace(z: Tensor, bias: Tensor) -> int:
-    """amax of relu(z + bias) into the stream's workspace; returns the epoch
-    that tags it (the compress that reads it takes the next one)."""
-    M, N = z.shape
-    L = _lib.load()
-    ws = _lib.workspace_for(z.device)
-    ws.ensure(256)
-    epoch = ws.next_epoch(reserve=2)
-    check(L.bs_amax_bias_relu(z.data_ptr(), M, N, bias.data_ptr(), ws.buf.data_ptr(), ws.nbytes, epoch,
-                              stream_handle(z.device)), "bs_amax_bias_relu")
-    return epoch
-
-
-def compress_act_into(z: Tensor, bias: Tensor | None, square: bool, bitmask: Tensor, prefix: Tensor, vals: Tensor,
-                      packed: bool, vals_offset_in: Tensor | None, vals_offset_out: Tensor | None,
-                      vals_start_out: Tensor | None, err_flags: Tensor | None, h_out: Tensor | None = None,
-                      codes_out: Tensor | None = None, scale_out: Tensor | None = None,
-                      codes_scale_out: Tensor | None = None, amax_epoch: int = 0) -> None:
-    """The activation step of an MLP block (bs_compress_act): relu(z + bias)
-    compressed, and the down-projection's operand written -- h_out (bf16), or
-    with ``codes_out`` its e4m3fn codes (values then e4m3fn, the amax under
-    ``amax_epoch``)."""
-    M, N = z.shape
-    quantize = codes_out is not None
-    L = _lib.load()
-    ws = _lib.workspace_for(z.device)
-    ws.ensure(L.bs_compress_workspace_bytes(M, N))
-    epoch = ws.next_epoch()
-    check(L.bs_compress_act(z.data_ptr(), ptr(bias), M, N, int(square), float(RELU2_SCALE), int(quantize),
-                            ws.amax_slot_ptr() if quantize else None, amax_epoch, ptr(scale_out), ptr(codes_out),
-                            ptr(codes_scale_out), ptr(h_out), bitmask.data_ptr(), prefix.data_ptr(), vals.data_ptr(),
-                            vals.numel(), int(packed), ptr(vals_offset_in), ptr(vals_offset_out), ptr(vals_start_out),
-                            ptr(err_flags), ws.buf.data_ptr(), ws.nbytes, epoch, stream_handle(z.device)),
-          "bs_compress_act")
-
-
 def amax_relu2_from(device: torch.device, epoch_in: int, k: float) -> int:
     """amax|bf16(bf16(r * r) * k)| from the amax|r| of ``epoch_in`` (r = relu(z),
     bs_amax_relu2_from) into the stream's workspace; returns the epoch that
@@ -377,26 +341,6 @@ def quantize_e4m3fn(x: Tensor, amax_epoch: int) -> tuple[Tensor, Tensor]:
                                ws.buf.data_ptr(), ws.nbytes, amax_epoch,
                                stream_handle(x.device)), "bs_quantize_e4m3fn")
     return q, scale
-
-
-def quantize_t_supported(x: Tensor) -> bool:
-    return (x.dim() == 2 and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and 0 < x.numel() < 2 ** 31
-            and x.shape[1] % 8 == 0 and x.shape[0] % 4 == 0 and x.data_ptr() % 16 == 0)
-
-
-def quantize_e4m3fn_t(x: Tensor, amax_epoch: int, both: bool) -> tuple[Tensor | None, Tensor, Tensor]:
-    """(codes of x or None, codes of x.T as a new row-major tensor, fp32 0-d
-    scale) from the amax of ``amax_epoch`` (``quantize_t_supported``);
-    ``both``: the row-major codes too."""
-    R, C = x.shape
-    L = _lib.load()
-    ws = _lib.workspace_for(x.device)
-    q = torch.empty((R, C), device=x.device, dtype=torch.float8_e4m3fn) if both else None
-    qt = torch.empty((C, R), device=x.device, dtype=torch.float8_e4m3fn)
-    scale = torch.empty((), device=x.device, dtype=torch.float32)
-    check(L.bs_quantize_e4m3fn_t(x.data_ptr(), R, C, ptr(q), qt.data_ptr(), scale.data_ptr(), ws.buf.data_ptr(),
-                                 ws.nbytes, amax_epoch, stream_handle(x.device)), "bs_quantize_e4m3fn_t")
-    return q, qt, scale
 
 
 def transpose_u8(x: Tensor, out: Tensor | None = None) -> Tensor:
@@ -504,60 +448,6 @@ def _check_grad(grad: Tensor, sparse: BitsparseTensor, what: str) -> None:
         raise TypeError(f"{what}: grad must be bfloat16")
     if tuple(grad.shape) != tuple(sparse.shape):
         raise ValueError(f"{what}: grad shape {tuple(grad.shape)} != {tuple(sparse.shape)}")
-
-
-def act_grad_sums_supported(grad: Tensor, sparse: BitsparseTensor, square: bool) -> bool:
-    """Whether ``act_grad_sums_`` takes this gradient and activation."""
-    if not (grad.is_contiguous() and grad.dtype == torch.bfloat16 and grad.numel() > 0 and grad.numel() < 2 ** 31
-            and grad.shape[1] % 8 == 0 and grad.data_ptr() % 16 == 0):
-        return False
-    if not square:
-        return True
-    stored = sparse.dtype if sparse.pack_sbit else sparse.vals.dtype
-    return (stored, sparse.scale is None) in ((torch.bfloat16, True), (torch.float8_e4m3fn, False))
-
-
-def act_grad_sums_(grad: Tensor, sparse: BitsparseTensor, square: bool, bias_grad: bool,
-                   amax: bool) -> tuple[Tensor | None, int]:
-    """``relu2_grad_sparse_`` (square) or ``mask_with_bitmask_`` in place, and
-    from the same pass (bias gradient = the column sums of the result, epoch
-    that tags its amax in the stream's workspace), each if asked for."""
-    _check_grad(grad, sparse, "act_grad_sums_")
-    M, N = sparse.shape
-    L = _lib.load()
-    out = torch.empty(N, device=grad.device, dtype=torch.bfloat16) if bias_grad else None
-    need = L.bs_grad_sums_workspace_bytes(M, N)
-    part = torch.empty(need, device=grad.device, dtype=torch.uint8)
-    ws, epoch = None, 0
-    if amax:
-        ws = _lib.workspace_for(grad.device)
-        ws.ensure(256)
-        epoch = ws.next_epoch(reserve=2)
-    stored = sparse.dtype if sparse.pack_sbit else sparse.vals.dtype
-    check(L.bs_act_grad_sums(grad.data_ptr(), M, N, int(square), sparse.vals.data_ptr(), dtype_code(stored),
-                             sparse.vals.numel(), int(sparse.pack_sbit), sparse.bitmask.data_ptr(),
-                             sparse.prefix.data_ptr(), sparse.vals_offset.data_ptr(), float(RELU2_SCALE),
-                             ptr(sparse.scale), ptr(out), ws.buf.data_ptr() if ws else None, epoch, part.data_ptr(),
-                             need, stream_handle(grad.device)), "bs_act_grad_sums")
-    return out, epoch
-
-
-def col_sum_supported(x: Tensor) -> bool:
-    """Whether ``col_sum`` takes x as it is."""
-    return (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and x.is_contiguous() and x.shape[0] > 0
-            and x.shape[1] > 0 and x.shape[1] % 8 == 0 and x.data_ptr() % 16 == 0 and x.numel() < 2 ** 31)
-
-
-def col_sum(x: Tensor) -> Tensor:
-    """x.sum(0) of a bf16 matrix (``col_sum_supported``), in fp32, rounded once."""
-    R, C = x.shape
-    L = _lib.load()
-    out = torch.empty(C, device=x.device, dtype=torch.bfloat16)
-    need = L.bs_col_sum_workspace_bytes(R, C)
-    part = torch.empty(need, device=x.device, dtype=torch.uint8)
-    check(L.bs_col_sum(x.data_ptr(), R, C, out.data_ptr(), part.data_ptr(), need, stream_handle(x.device)),
-          "bs_col_sum")
-    return out
 
 
 def mask_with_bitmask_(grad: Tensor, sparse: BitsparseTensor) -> Tensor:

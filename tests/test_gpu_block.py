@@ -1,6 +1,8 @@
 """The MLP block's single node and its activation / gradient kernels against
 the separate steps they stand for, bit for bit (column sums: fp32 order)."""
 import contextlib
+import itertools
+import threading
 
 import pytest
 import torch
@@ -27,54 +29,73 @@ def _same(a, b, what):
     assert a.shape == b.shape and torch.equal(a.view(torch.uint8), b.view(torch.uint8)), what
 
 
+def _buffer(n, dev, store):
+    """A TensorBuffer with room for n values: store is a value type and _packed or not."""
+    from bitsparse_amd.bitsparse import TensorBuffer
+    fp8, pack = store.startswith("e4m3"), store.endswith("packed")
+    size = (n * (7 if fp8 else 15) + 7) // 8 + 16 if pack else n * (1 if fp8 else 2)
+    return TensorBuffer(size, device=dev, dtype=E4M3 if fp8 else torch.bfloat16, pack_sbit=pack)
+
+
+def _activate(z, bias, buf, square, k=1.0):
+    """The native activation step: (operand, its scale, bitmask, prefix, start, scale)."""
+    from bitsparse_amd._lib import native
+    offset, in_place = buf.native_cursor()
+    operand, oscale, bitmask, prefix, start, buf.offset, scale = native().activate(
+        z, bias, buf.vals, offset, buf.err_flags, in_place, buf.pack_sbit, buf.dtype == E4M3, square, k)
+    return operand, oscale, bitmask, prefix, start, scale
+
+
+def _separate_activation(z, bias, buf, square, k=1.0):
+    """The same by the layers' separate steps."""
+    from bitsparse_amd.fp8 import to_fp8
+    from bitsparse_amd.src import functions as F
+    z = z + bias if bias is not None else z.clone()
+    if buf.dtype == E4M3:
+        operand, oscale, sp = F.relu_quantize_and_compress(z, buf, buf.pack_sbit)
+        if square:
+            operand, oscale = to_fp8(z.square().mul_(k))
+    else:
+        operand, sp = F.relu_and_compress(z, buf, buf.pack_sbit)
+        oscale = None
+        if square:
+            operand = operand.square().mul_(k)
+    return operand, oscale, sp.bitmask, sp.prefix, sp.vals_offset, sp.scale
+
+
+def _same_step(want, got, bufs):
+    for a, b, name in zip(want, got, ("operand", "operand scale", "bitmask", "prefix", "start", "scale")):
+        assert (a is None) == (b is None), name
+        if a is not None:
+            _same(a.reshape(1) if a.numel() == 1 else a, b.reshape(1) if b.numel() == 1 else b, name)
+    _same(bufs[0].vals, bufs[1].vals, "values")
+    _same(bufs[0].offset, bufs[1].offset, "cursor")
+
+
+STORES = ["bf16", "e4m3", "bf16_packed", "e4m3_packed"]
+
+
 # one tile, short last tile rows and columns, a row of several workgroups
 @pytest.mark.parametrize("shape", [(1, 8), (64, 64), (65, 72), (80, 1416), (304, 528), (1000, 1024)])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("square", [False, True])
-@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed", "e4m3_packed"])
+@pytest.mark.parametrize("store", STORES)
 @pytest.mark.parametrize("special", [False, True])
 def test_activation_step(dev, shape, bias, square, store, special):
-    from bitsparse_amd.bitsparse import TensorBuffer
-    from bitsparse_amd.fp8 import to_fp8
-    from bitsparse_amd.src import functions as F
-    fp8, pack = store.startswith("e4m3"), store.endswith("packed")
     z, b = _z(shape, 3, special, dev)
-    n = z.numel()
-    size = (n * (7 if fp8 else 15) + 7) // 8 + 16 if pack else n * (1 if fp8 else 2)
-    bufs = [TensorBuffer(size, device=dev, dtype=E4M3 if fp8 else torch.bfloat16, pack_sbit=pack) for _ in range(2)]
-    zz = z + b if bias else z.clone()
-    if fp8:
-        q, scale, want = F.relu_quantize_and_compress(zz, bufs[0], pack)
-        operand, oscale = (q, scale) if not square else to_fp8(zz.square().mul_(1.0))
-    else:
-        operand, want = F.relu_and_compress(zz, bufs[0], pack)
-        oscale = None
-        if square:
-            operand = operand.square().mul_(1.0)
-    assert F.activate_ok(z, b if bias else None, bufs[1], 1.0)
-    got_operand, got_scale, got = F.activate_and_compress(z, b if bias else None, bufs[1], pack, fp8, square)
-    _same(want.bitmask, got.bitmask, "bitmask")
-    _same(want.prefix, got.prefix, "prefix")
-    _same(bufs[0].vals, bufs[1].vals, "values")
-    _same(bufs[0].offset, bufs[1].offset, "cursor")
-    _same(want.vals_offset.reshape(1), got.vals_offset.reshape(1), "start")
-    _same(operand, got_operand, "operand")
-    if fp8:
-        _same(want.scale.reshape(1), got.scale.reshape(1), "stored scale")
-        _same(oscale.reshape(1), got_scale.reshape(1), "operand scale")
+    bufs = [_buffer(z.numel(), dev, store) for _ in range(2)]
+    b = b if bias else None
+    want = _separate_activation(z, b, bufs[0], square)
+    _same_step(want, _activate(z, b, bufs[1], square), bufs)
 
 
 @pytest.mark.parametrize("value", [2.0e25, 3.0e-25, float("inf"), float("nan"), -float("nan"), None])
 @pytest.mark.parametrize("k", [1.0, 0.37, -2.0, 0.0])
-def test_codes_of_the_square(dev, value, k, monkeypatch):
-    """The codes of h = k r^2 over the whole range of scales: a square past
+@pytest.mark.parametrize("store", STORES)
+def test_codes_of_the_square(dev, value, k, store):
+    """h = k r^2 over the whole range of scales: a square past
     bf16's range (an infinite scale), all squares underflowing, Inf, NaN of
     either sign, an all-negative pre-activation; k of either sign and 0."""
-    from bitsparse_amd.bitsparse import TensorBuffer
-    from bitsparse_amd.fp8 import to_fp8
-    from bitsparse_amd.src import functions as F
-    from bitsparse_amd.src import hip_operators as H
-    monkeypatch.setattr(H, "RELU2_SCALE", k)
     z, _ = _z((70, 136), 4, False, dev)
     if value is None:
         z = -z.abs()
@@ -82,111 +103,285 @@ def test_codes_of_the_square(dev, value, k, monkeypatch):
         z = z * value
     else:
         z[3, 5] = value
-    bufs = [TensorBuffer(z.numel(), device=dev, dtype=E4M3) for _ in range(2)]
-    r = z.clone()
-    want_sp = F.relu_quantize_and_compress(r, bufs[0], False)[2]
-    want, wscale = to_fp8(r.square().mul_(k))
-    got, gscale, sp = F.activate_and_compress(z, None, bufs[1], False, True, True)
-    _same(wscale.reshape(1), gscale.reshape(1), "scale of h")
-    _same(want, got, "codes of h")
-    _same(want_sp.scale.reshape(1), sp.scale.reshape(1), "scale")
-    _same(want_sp.bitmask, sp.bitmask, "bitmask")
-    _same(bufs[0].vals, bufs[1].vals, "values")
+    bufs = [_buffer(z.numel(), dev, store) for _ in range(2)]
+    want = _separate_activation(z, None, bufs[0], True, k)
+    _same_step(want, _activate(z, None, bufs[1], True, k), bufs)
 
 
-@pytest.mark.parametrize("store", ["bf16", "e4m3"])
-def test_activation_step_lookback_fallback(dev, store, monkeypatch):
-    """With no patience every wait counts its predecessors from the dense
-    input, where the bias has to be added too (and rows past the matrix, whose
+# (over z without a bias, where a recount sees the relu of z; the square of a
+# z written over is waited for instead)
+@pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("bias,square", [(True, True), (True, False), (False, False), (False, True)])
+def test_activation_step_lookback_fallback(dev, store, bias, square, monkeypatch):
+    """With no patience a unit that finds a predecessor unpublished counts it
+    from the dense input, where the bias has to be added too (and rows past the matrix, whose
     bias alone may be positive, count nothing)."""
-    from bitsparse_amd.bitsparse import TensorBuffer
-    from bitsparse_amd.src import functions as F
-    z, b = _z((72, 64 * 40), 12, False, dev)
-    b = b.abs()
-    dt = E4M3 if store == "e4m3" else torch.bfloat16
-    outs = []
+    from bitsparse_amd import _lib
+    z, b = _z((8008, 4096), 12, False, dev)         # 1000 units: some meet an unpublished predecessor
+    b = b.abs() if bias else None
+    ws = _lib.workspace_for(z.device)
+    outs, bufs, counted = [], [], []
     for patience in (None, "0"):
         if patience is not None:
             monkeypatch.setenv("BITSPARSE_LOOKBACK_PATIENCE", patience)
-        buf = TensorBuffer(2 * z.numel(), device=dev, dtype=dt)
-        sp = F.activate_and_compress(z.clone(), b, buf, False, store == "e4m3", True)[2]
-        outs.append((sp.prefix, buf.vals, buf.offset))
-    for x, y, what in zip(*outs, ("prefix", "values", "cursor")):
-        _same(x, y, what)
+        bufs.append(_buffer(z.numel(), dev, store))
+        before = ws.fallback_count()
+        outs.append(_activate(z.clone(), b, bufs[-1], square))
+        counted.append(ws.fallback_count() - before)
+    in_place = square and not bias and not store.startswith("e4m3")
+    assert counted[0] == 0 and (counted[1] > 0) == (not in_place), counted
+    _same_step(*outs, bufs)
+    assert not bufs[1].overflowed()
 
 
 @pytest.mark.parametrize("shape", [(1, 8), (64, 64), (65, 72), (80, 1416), (1000, 1024), (4100, 192)])
-@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed", "e4m3_packed"])
+@pytest.mark.parametrize("store", STORES)
 @pytest.mark.parametrize("square", [False, True])
 @pytest.mark.parametrize("zeros", [0.0, 0.5, 1.0])
-def test_gradient_sums(dev, shape, store, square, zeros):
+def test_gradient_step(dev, shape, store, square, zeros):
+    """The activation's gradient with every set of what rides on it: the
+    gradient and its codes bit for bit, the bias gradient to its rounding."""
+    from bitsparse_amd._lib import native
     from bitsparse_amd.src import functions as F
     from bitsparse_amd.src import hip_operators as H
     z, _ = _z(shape, 6, False, dev)
     z = z.abs() + 1 if zeros == 0.0 else (-z.abs() if zeros == 1.0 else z)
-    pack = store.endswith("packed")
-    if store.startswith("e4m3"):
+    fp8, pack = store.startswith("e4m3"), store.endswith("packed")
+    if fp8:
         sp = F.quantize_and_compress(z.relu(), None, pack)[2]
     else:
         sp = F.dense_to_tilesparse(z.relu(), None, None, pack)
-    g = torch.randn(shape, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to(dev)
-    want = g.clone()
+    g0 = torch.randn(shape, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to(dev)
+    want = g0.clone()
     (H.relu2_grad_sparse_ if square else H.mask_with_bitmask_)(want, sp)
-    assert H.act_grad_sums_supported(g, sp, square)
-    sums, epoch = H.act_grad_sums_(g, sp, square, True, True)
-    q, scale = H.quantize_e4m3fn(g, epoch)
-    _same(want, g, "gradient")
     wq, wscale = H.quantize_e4m3fn(want, H.amax_into_workspace(want))
-    _same(wscale.reshape(1), scale.reshape(1), "scale")
-    _same(wq, q, "codes")
     w64 = want.double().sum(0)
     bound = shape[0] * 2.0 ** -24 * want.double().abs().sum(0) + 2.0 ** -8 * w64.abs() + 1e-30
-    assert ((sums.double() - w64).abs() <= bound).all()
+    # transposed codes: rows in whole groups of 4
+    for bias, rows, cols in itertools.product((False, True), (False, fp8), (False, fp8 and shape[0] % 4 == 0)):
+        g, held = g0.clone(), [sp.vals, sp.bitmask, sp.prefix, sp.vals_offset, sp.scale]
+        sums, q, qt, scale, scale_t = native().act_grad(g, held, pack, fp8, square, 1.0, bias, rows, cols)
+        assert held == []
+        _same(want, g, "gradient")
+        assert (sums is not None, q is not None, qt is not None) == (bias, rows, cols)
+        if bias:
+            assert ((sums.double() - w64).abs() <= bound).all()
+        for codes, s, t in ((q, scale, wq), (qt, scale_t, wq.view(torch.uint8).t().contiguous())):
+            if codes is not None:
+                _same(wscale.reshape(1), s.reshape(1), "scale")
+                _same(t.view(torch.uint8), codes.view(torch.uint8), "codes")
+
+
+# ---------------------------------------------------------------------------
+# the whole block against the separate nodes
+# ---------------------------------------------------------------------------
+NAMES = ("x", "W1", "W2", "b1", "b2")
+
+
+def _operands(dev, T, D, Hn, O, biases=("b1", "b2"), seed=11):
+    """(operands by name, gradient of y)"""
+    g = torch.Generator().manual_seed(seed)
+
+    def r(*s, mul=0.1):
+        return (mul * torch.randn(s, generator=g)).to(torch.bfloat16).to(dev)
+    p = dict(x=r(T, D, mul=1.0), W1=r(Hn, D), W2=r(O, Hn), b1=r(Hn), b2=r(O))
+    dY = r(T, O, mul=1.0)
+    return {k: v if k in biases or k[0] != "b" else None for k, v in p.items()}, dY
+
+
+def _block(p, store, square, block, buf=None):
+    """y of the layer on operands p, as one node or by the separate ones."""
+    from bitsparse_amd import layers
+    layer, kw = (layers.FFNRelu2, "storage_dtype") if square else (layers.FFNRelu, "dtype")
+    buf = buf or _buffer(p["x"].shape[:-1].numel() * p["W1"].shape[0], p["x"].device, store)
+    with pytest.MonkeyPatch.context() as m:
+        if not block:
+            m.setattr(layers, "_block_ok", lambda *a: False)
+        y = layer.apply(p["x"], p["W1"], p["W2"], p["b1"], p["b2"], sparse_data=buf,
+                        pack_sbit=store.endswith("packed"), **{kw: E4M3 if store.startswith("e4m3") else torch.bfloat16})
+    if y.requires_grad:
+        taken = any(n.name() == "_FFNBlockBackward" for n in _graph_nodes(y))
+        assert taken == block, "the node that was asked for"
+    return y
+
+
+def _params(p, need=NAMES):
+    return {k: None if t is None else t.clone().requires_grad_(k in need) for k, t in p.items()}
+
+
+def _compare(got, want, T):
+    """y, dx, dW1, dW2 bit for bit; the bias gradients (fp32 sums of T values in
+    another order, rounded once each) to their rounding."""
+    assert got.keys() == want.keys()
+    for name, a in got.items():
+        b = want[name]
+        if name in ("b1", "b2"):
+            assert ((a - b).double().abs() <= 2.0 ** -7 * b.double().abs() + 1e-2).all(), name
+        else:
+            _same(a, b, name)
+
+
+def _step(p, dY, store, square, block, need=NAMES, buf=None):
+    q = _params(p, need)
+    y = _block(q, store, square, block, buf)
+    out = {"y": y.detach()}
+    if need:
+        y.backward(dY)
+        out.update({k: t.grad for k, t in q.items() if t is not None and k in need})
+    return out
+
+
+# tokens, in, hidden, out: ordinary; one token; rows and columns that end inside a tile and a
+# GEMM's tile, in != out; (fp8: multiples of 16)
+@pytest.mark.parametrize("shape", [(208, 144, 528, 144), (1, 8, 8, 8), (67, 20, 136, 12), (300, 72, 1416, 40),
+                                   (16, 48, 32, 80)])
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("biases", [(), ("b1",), ("b2",), ("b1", "b2")])
+def test_block_equals_the_separate_nodes(dev, shape, square, store, biases):
+    if store.startswith("e4m3") and any(n % 16 for n in shape):
+        shape = tuple(-(-n // 16) * 16 for n in shape)
+    p, dY = _operands(dev, *shape, biases)
+    _compare(_step(p, dY, store, square, True), _step(p, dY, store, square, False), shape[0])
 
 
 @pytest.mark.parametrize("square", [False, True])
-@pytest.mark.parametrize("store", ["bf16", "e4m3", "bf16_packed"])
-@pytest.mark.parametrize("use_buffer", [False, True])
-def test_block_equals_the_separate_nodes(dev, square, store, use_buffer, monkeypatch):
-    """y, dx, dW1, dW2 bit for bit; the bias gradients to their rounding."""
-    from bitsparse_amd import layers
-    from bitsparse_amd.bitsparse import TensorBuffer
-    g = torch.Generator().manual_seed(11)
-    T, D, Hn = 208, 144, 528
-    fp8, pack = store == "e4m3", store.endswith("packed")
-    x = torch.randn((2, T // 2, D), generator=g).to(torch.bfloat16).to(dev)
-    W1 = (0.1 * torch.randn((Hn, D), generator=g)).to(torch.bfloat16).to(dev)
-    W2 = (0.1 * torch.randn((D, Hn), generator=g)).to(torch.bfloat16).to(dev)
-    b1 = (0.1 * torch.randn(Hn, generator=g)).to(torch.bfloat16).to(dev)
-    b2 = (0.1 * torch.randn(D, generator=g)).to(torch.bfloat16).to(dev)
-    dY = torch.randn((2, T // 2, D), generator=g).to(torch.bfloat16).to(dev)
-    dt = E4M3 if fp8 else torch.bfloat16
-    layer, kw = (layers.FFNRelu2, "storage_dtype") if square else (layers.FFNRelu, "dtype")
+@pytest.mark.parametrize("store", STORES)
+def test_block_with_frozen_operands(dev, square, store):
+    """Every subset of the operands that may ask for a gradient."""
+    p, dY = _operands(dev, 80, 48, 144, 32)
+    for n in range(len(NAMES) + 1):
+        for need in itertools.combinations(NAMES, n):
+            _compare(_step(p, dY, store, square, True, need), _step(p, dY, store, square, False, need), 80)
+
+
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan"), 3.0e38, 1.0e-38])
+def test_block_special_values(dev, square, store, value):
+    p, dY = _operands(dev, 80, 48, 144, 32)
+    p["x"][3, 5] = value
+    got, want = (_step(p, dY, store, square, block) for block in (True, False))
+    for name in ("y", "x", "W1", "W2"):
+        a, b = got[name], want[name]
+        assert torch.equal(a.isnan(), b.isnan()), name
+        _same(a.nan_to_num(1.5), b.nan_to_num(1.5), name)
+    for name in ("b1", "b2"):
+        a, b = got[name], want[name]
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), name
+        ok = a.isfinite()
+        assert ((a[ok] - b[ok]).double().abs() <= 2.0 ** -7 * b[ok].double().abs() + 1e-2).all(), name
+
+
+@pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("layout", ["3d", "transposed", "padded", "one_row"])
+def test_block_input_layouts(dev, store, layout):
+    p, dY = _operands(dev, 96, 48, 144, 48)
+    base, view = {"3d": (p["x"].reshape(2, 48, 48), lambda t: t),
+                  "transposed": (p["x"].t().contiguous(), lambda t: t.t()),
+                  "padded": (torch.nn.functional.pad(p["x"], (0, 16)), lambda t: t[:, :48]),
+                  "one_row": (p["x"][:1], lambda t: t.expand(96, 48))}[layout]
     outs = []
     for block in (True, False):
-        if not block:
-            monkeypatch.setattr(layers, "_block_ok", lambda *a: False)
-        p = [t.clone().requires_grad_() for t in (x, W1, W2, b1, b2)]
-        buf = TensorBuffer(2 * T * Hn + 64, device=dev, dtype=dt, pack_sbit=pack) if use_buffer else None
-        y = layer.apply(p[0], p[1], p[2], p[3], p[4], sparse_data=buf, pack_sbit=pack, **{kw: dt})
-        y.backward(dY)
-        outs.append([y.detach()] + [t.grad for t in p])
-    for a, b, name in zip(outs[0][:4], outs[1][:4], ("y", "dx", "dW1", "dW2")):
-        _same(a, b, name)
-    for a, b, name in zip(outs[0][4:], outs[1][4:], ("db1", "db2")):
-        # two bf16 roundings of fp32 sums
-        assert ((a - b).double().abs() <= 2.0 ** -7 * b.double().abs() + 1e-2).all(), name
+        q = _params(p)
+        leaf = base.clone().requires_grad_()
+        q["x"] = view(leaf)
+        y = _block(q, store, True, block)
+        y.backward(dY.reshape(y.shape))
+        outs.append({"y": y.detach(), "x": leaf.grad, **{k: q[k].grad for k in NAMES[1:]}})
+    _compare(*outs, 96)
 
 
-def _graph_node(t, name):
-    """The autograd node of that name behind t."""
-    nodes = [t.grad_fn]
+@pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("in_place", [False, True])
+def test_blocks_of_one_buffer(dev, store, in_place):
+    """Blocks appended to one buffer, backwards in the reverse order; then
+    over again after a reset."""
+    ps = [_operands(dev, 80, 48, 144, 48, seed=s) for s in (1, 2, 3)]
+    want = [_step(p, dY, store, True, False) for p, dY in ps]
+    buf = _buffer(4 * 80 * 144, dev, store)
+    buf.inplace_offset = in_place
+    for _ in range(2):
+        buf.reset_buffer()
+        qs = [_params(p) for p, _ in ps]
+        ys = [_block(q, store, True, True, buf) for q in qs]
+        for y, (_, dY) in reversed(list(zip(ys, ps))):
+            y.backward(dY)
+        for q, y, w in zip(qs, ys, want):
+            _compare({"y": y.detach(), **{k: t.grad for k, t in q.items()}}, w, 80)
+    assert not buf.overflowed()
+
+
+@pytest.mark.parametrize("store", STORES)
+def test_epoch_wrap_inside_a_block(dev, store):
+    """The workspace's counter wraps (and clears the amax slot) at every place
+    inside a forward and backward."""
+    from bitsparse_amd import _lib
+    p, dY = _operands(dev, 80, 48, 144, 32)
+    want = _step(p, dY, store, True, False)
+    ws = _lib.workspace_for(p["x"].device)
+    _step(p, dY, store, True, True)
+    before = ws.epoch
+    _step(p, dY, store, True, True)
+    took = ws.epoch - before
+    for left in range(took + 2):
+        ws.buf.zero_()                   # (the counter is set back: no word of a later epoch)
+        ws.epoch = _lib._EPOCH_LIMIT - left
+        _compare(_step(p, dY, store, True, True), want, 80)
+        assert 0 < ws.epoch <= _lib._EPOCH_LIMIT
+
+
+@pytest.mark.parametrize("store", STORES)
+def test_block_on_another_stream(dev, store):
+    p, dY = _operands(dev, 304, 64, 528, 64)
+    want = _step(p, dY, store, True, False)
+    s = torch.cuda.Stream(dev)
+    for _ in range(3):
+        s.wait_stream(torch.cuda.current_stream(dev))
+        with torch.cuda.stream(s):
+            got = _step(p, dY, store, True, True)
+        torch.cuda.current_stream(dev).wait_stream(s)
+        _compare(got, want, 304)
+
+
+@pytest.mark.parametrize("own_streams", [False, True])
+@pytest.mark.parametrize("store", ["bf16", "e4m3"])
+def test_blocks_of_two_threads(dev, store, own_streams):
+    """Two threads, on one stream (one workspace) or on a stream each."""
+    jobs = [_operands(dev, 144, 64, 272, 64, seed=s) for s in (1, 2)]
+    want = [_step(p, dY, store, True, True) for p, dY in jobs]
+    torch.cuda.synchronize(dev)
+    errors = []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream(dev) if own_streams else torch.cuda.current_stream(dev)
+            with torch.cuda.device(dev), torch.cuda.stream(stream):
+                got = [_step(*jobs[i], store, True, True) for _ in range(20)]
+                stream.synchronize()
+            for g in got:
+                for k in g:
+                    _same(g[k], want[i][k], k)
+        except BaseException as e:      # noqa: B036 (handed to the test's thread)
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[0]
+
+
+def _graph_nodes(t):
+    """Every autograd node behind t."""
+    nodes, seen = [t.grad_fn], set()
     while nodes:
         n = nodes.pop()
-        if n is not None and n.name() == name:
-            return n
-        nodes += [m for m, _ in n.next_functions] if n is not None else []
-    raise AssertionError(f"no {name}")
+        if n is None or n in seen:
+            continue
+        seen.add(n)
+        yield n
+        nodes += [m for m, _ in n.next_functions]
 
 
 @pytest.mark.parametrize("how", ["default_hooks", "node_hooks", "data"])
@@ -214,7 +409,7 @@ def test_backward_scales_the_values_it_reads(dev, how, grow, monkeypatch):
                 contextlib.nullcontext():
             y = FFNRelu2.apply(*p, sparse_data=buf, storage_dtype=E4M3)
         if how == "node_hooks":
-            for saved in _graph_node(y, "_FFNBlockBackward")._raw_saved_tensors:
+            for saved in next(n for n in _graph_nodes(y) if n.name() == "_FFNBlockBackward")._raw_saved_tensors:
                 saved.register_hooks(lambda t: t, unpack)
         elif how == "data":
             for t in p:
