@@ -144,6 +144,16 @@ __device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b)
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(s, bf16x2));
 }
 
+// two bf16 values with every NaN as 0x7fc0, the one torch's rounding to bf16
+// gives (the hardware's keeps sign and payload)
+__device__ __forceinline__ uint32_t quiet_nan_bf16x2(uint32_t w)
+{
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const u16x2 m = __builtin_bit_cast(u16x2, w) & (u16x2)(unsigned short)0x7fff;
+    const uint32_t nan = __builtin_bit_cast(uint32_t, m > (u16x2)(unsigned short)0x7f80);
+    return (w & ~nan) | (0x7fc07fc0u & nan);
+}
+
 // e4m3fn bits -> fp32 (exact). 0x7f / 0xff are NaN.
 __device__ __forceinline__ float e4m3_to_f32(uint32_t b)
 {

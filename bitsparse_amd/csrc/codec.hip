@@ -847,6 +847,36 @@ void compress_stream_kernel(CompressArgs a)
 #pragma unroll
                 for (int k = 0; k < 8; k++) d[k] = relu_chunk<IN_T>(d[k]);
             }
+            if constexpr (WB == WB_ACT) {
+                // what is written beside the compressed form: torch's z + b
+                // turns every NaN into 0x7fc0.  The quantizer's scale tells of
+                // one; else r >= 0, where a larger half is a NaN (one packed
+                // maximum per pair)
+                if (a.bias != nullptr) {
+                    bool nan = false;
+                    if constexpr (QUANT) {
+                        nan = scale != scale;
+                    } else {
+                        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+                        u16x2 m = {0, 0};
+#pragma unroll
+                        for (int k = 0; k < 8; k++)
+                            m = __builtin_elementwise_max(
+                                __builtin_elementwise_max(
+                                    __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, d[k].x)),
+                                    __builtin_bit_cast(u16x2, d[k].y)),
+                                __builtin_elementwise_max(__builtin_bit_cast(u16x2, d[k].z),
+                                                          __builtin_bit_cast(u16x2, d[k].w)));
+                        nan = max(m.x, m.y) > 0x7f80;
+                    }
+                    if (nan) {
+#pragma unroll
+                        for (int k = 0; k < 8; k++)
+                            d[k] = uint4{quiet_nan_bf16x2(d[k].x), quiet_nan_bf16x2(d[k].y), quiet_nan_bf16x2(d[k].z),
+                                         quiet_nan_bf16x2(d[k].w)};
+                    }
+                }
+            }
         }
 
         // ---- masks, bitmask bytes, round totals

@@ -127,6 +127,7 @@ __global__ __launch_bounds__(kFp8Threads) void amax_bias_relu_kernel(const uint1
     __syncthreads();
     if (tid == 0) {
         for (int w = 1; w < kFp8Threads / 64; w++) m = max(m, s_w[w]);
+        if (m > 0x7f80u) m = 0x7fc0u;                  // the NaN that torch's add makes of any
         atomicMax((unsigned long long*)slot, (unsigned long long)(((uint64_t)epoch << 32) | m));
     }
 }

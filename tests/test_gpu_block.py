@@ -16,12 +16,13 @@ def _z(shape, seed, special, dev):
     g = torch.Generator().manual_seed(seed)
     z = torch.randn(shape, generator=g).to(torch.bfloat16)
     b = (0.5 * torch.randn(shape[1], generator=g)).to(torch.bfloat16)
-    if special:
-        f = z.view(torch.int16).view(-1)
-        n = f.numel()
-        # -0, +Inf, -Inf, largest finite, a value whose square overflows, denormals
-        for i, v in enumerate((-32768, 0x7f80, -128, 0x7f7f, 0x5f80, 1, 0x0080)):
-            f[(i * 977 + 13) % n] = v
+    # -0, +Inf, -Inf, largest finite, a value whose square overflows, denormals; NaNs of either
+    # sign and any payload
+    values = {"inf": (-32768, 0x7f80, -128, 0x7f7f, 0x5f80, 1, 0x0080),
+              "nan": (-1, -64, 0x7fff, 0x7f81, -127, 0x7fc0, -32768)}.get(special, ())
+    f = z.view(torch.int16).view(-1)
+    for i, v in enumerate(values):
+        f[(i * 977 + 13) % f.numel()] = v
     return z.to(dev), b.to(dev)
 
 
@@ -80,7 +81,7 @@ STORES = ["bf16", "e4m3", "bf16_packed", "e4m3_packed"]
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("square", [False, True])
 @pytest.mark.parametrize("store", STORES)
-@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("special", [None, "inf", "nan"])
 def test_activation_step(dev, shape, bias, square, store, special):
     z, b = _z(shape, 3, special, dev)
     bufs = [_buffer(z.numel(), dev, store) for _ in range(2)]
@@ -96,7 +97,7 @@ def test_codes_of_the_square(dev, value, k, store):
     """h = k r^2 over the whole range of scales: a square past
     bf16's range (an infinite scale), all squares underflowing, Inf, NaN of
     either sign, an all-negative pre-activation; k of either sign and 0."""
-    z, _ = _z((70, 136), 4, False, dev)
+    z, _ = _z((70, 136), 4, None, dev)
     if value is None:
         z = -z.abs()
     elif value == 3.0e-25:
@@ -117,7 +118,7 @@ def test_activation_step_lookback_fallback(dev, store, bias, square, monkeypatch
     from the dense input, where the bias has to be added too (and rows past the matrix, whose
     bias alone may be positive, count nothing)."""
     from bitsparse_amd import _lib
-    z, b = _z((8008, 4096), 12, False, dev)         # 1000 units: some meet an unpublished predecessor
+    z, b = _z((8008, 4096), 12, None, dev)         # 1000 units: some meet an unpublished predecessor
     b = b.abs() if bias else None
     ws = _lib.workspace_for(z.device)
     outs, bufs, counted = [], [], []
@@ -144,7 +145,7 @@ def test_gradient_step(dev, shape, store, square, zeros):
     from bitsparse_amd._lib import native
     from bitsparse_amd.src import functions as F
     from bitsparse_amd.src import hip_operators as H
-    z, _ = _z(shape, 6, False, dev)
+    z, _ = _z(shape, 6, None, dev)
     z = z.abs() + 1 if zeros == 0.0 else (-z.abs() if zeros == 1.0 else z)
     fp8, pack = store.startswith("e4m3"), store.endswith("packed")
     if fp8:
