@@ -519,11 +519,13 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& b1
     return {y, a.bitmask, a.prefix, a.start, a.next, optional(a.scale)};
 }
 
-// (dx, dW1, db1, dW2, db2), each where `need` asks for it
+// (dx, dW1, db1, dW2, db2), each where `need` asks for it.  `dh`: the product
+// g W2 formed by the caller, where its graph is wanted and the operations here
+// would not record one (it is overwritten).
 std::vector<std::optional<Tensor>>
 block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const py::list& held, bool packed,
                bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
-               const std::vector<bool>& need)
+               const std::vector<bool>& need, const std::optional<Tensor>& dh)
 {
     const c10::DeviceGuard guard(x.device());
     Held h = take_held(held, x.size(0), W1.size(0), packed, fp8, square, k);
@@ -535,7 +537,7 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
     if (fp8) g8 = to_fp8(g, w);
     if (need_W2) out[3] = down_weight_grad(fp8 ? g8.codes : g, g8.scale, h);
     if (!(need_x || need_W1 || need_b1)) return out;
-    const Tensor dz = fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
+    const Tensor dz = dh ? *dh : fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
     g8 = Fp8();
     const bool sums = need_b1 && !at::GradMode::is_enabled();
     const ActGrad a = act_grad(dz, h, sums, fp8 && need_x, fp8 && need_W1);

@@ -496,3 +496,30 @@ def test_peak_memory(dev, square, store, bias, monkeypatch):
     slack = 64 * 1024                            # rows of N, cursors, scales: each its own 512-byte block
     assert peaks[0][0] <= peaks[1][0] + slack + (T * Hn // 8 + T * Hn // 1024 if bias else 0), peaks
     assert peaks[0][1] <= peaks[1][1] + slack, peaks
+
+
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", STORES)
+def test_gradients_with_a_graph(dev, square, store):
+    """create_graph: the same gradients have a graph as those of the separate
+    nodes, and it leads to the same second gradients."""
+    p, dY = _operands(dev, 80, 48, 144, 32)
+    outs = []
+    for block in (True, False):
+        q = _params(p)
+        gy = dY.clone().requires_grad_()
+        y = _block(q, store, square, block)
+        leaves = [*q.values(), gy]
+        first = torch.autograd.grad(y, list(q.values()), gy, create_graph=True)
+        loss = sum((t.float() ** 2).sum() for t in first if t.requires_grad)
+        second = torch.autograd.grad(loss, leaves, allow_unused=True)
+        outs.append((first, second))
+    (f1, s1), (f2, s2) = outs
+    assert [t.requires_grad for t in f1] == [t.requires_grad for t in f2]
+    assert [t is None for t in s1] == [t is None for t in s2]
+    for name, a, b in zip(NAMES, f1, f2):
+        err = (a.double() - b.double()).norm() / b.double().norm()
+        assert float(err) <= (2.0 ** -7 if name in ("b1", "b2") else 0.0), name
+    # bf16 sums of a few contributions each, in the order the engine comes by them: 2^-9 an addition
+    for name, a, b in zip((*NAMES, "gy"), s1, s2):
+        assert a is None or float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -7, name
