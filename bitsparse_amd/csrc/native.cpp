@@ -127,9 +127,22 @@ struct Workspace {
             {c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::PythonDispatcher})};
     };
 
+    // A graph would record the zero fills below instead of running them, and
+    // what is captured with an epoch is refused anyway.
+    void refuse_capture() const
+    {
+        if (!device.is_cuda()) return;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        const hipError_t e = hipStreamIsCapturing(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index()).stream(), &cs);
+        if (e != hipSuccess) (void)hipGetLastError();
+        TORCH_CHECK_VALUE(e != hipSuccess || cs == hipStreamCaptureStatusNone,
+                          "bitsparse_amd: compress and amax cannot be captured into a HIP graph: their device state is "
+                          "tagged with a per-call epoch that a replay would repeat");
+    }
     void ensure(int64_t nbytes)
     {
         if (buf.numel() >= nbytes) return;
+        refuse_capture();
         const NoPython guard;
         // grow geometrically; the old contents (amax slot, status words of
         // earlier epochs) move along and the new tail is zero, so epochs
@@ -145,6 +158,7 @@ struct Workspace {
     {
         ensure(nbytes);
         if (epoch + epochs <= kEpochLimit) return;
+        refuse_capture();
         const NoPython guard;
         buf.zero_();
         epoch = 0;
@@ -563,7 +577,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("abi_version", [] { return L.bs_abi_version(); });
     py::class_<Workspace, std::shared_ptr<Workspace>>(m, "Workspace")
         .def(py::init<c10::Device>())
-        .def_readonly("buf", &Workspace::buf)
+        .def_readwrite("buf", &Workspace::buf)
         .def_readwrite("epoch", &Workspace::epoch)
         .def_property_readonly("nbytes", &Workspace::nbytes)
         .def("ensure", &Workspace::ensure)

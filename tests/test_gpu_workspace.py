@@ -58,6 +58,52 @@ def test_epoch_tagged_entry_points_refuse_graph_capture(dev):
     assert torch.equal(again.vals[:x.numel()], ref.vals[:x.numel()])
 
 
+@pytest.mark.parametrize("what", ["compress", "quantize", "amax", "block", "block_fp8"])
+def test_refused_capture_leaves_no_workspace(dev, what):
+    """A capture that is refused must not have made the stream's workspace: its
+    zero fill would only have been recorded, and later calls on that stream
+    would take the memory's old contents for status words."""
+    import torch
+    from bitsparse_amd import _lib
+    from bitsparse_amd.bitsparse import TensorBuffer
+    from bitsparse_amd.layers import FFNRelu
+    from bitsparse_amd.src import hip_operators as H
+    from bitsparse_amd.src.functions import dense_to_tilesparse, quantize_and_compress
+    from tests.helpers import relu_input
+    x = relu_input((256, 512), 0.5, seed=90).to(dev)
+    W1, W2 = x[:128].contiguous(), x[:128, :128].contiguous()
+    dtype = torch.float8_e4m3fn if what in ("quantize", "block_fp8") else torch.bfloat16
+    buf = TensorBuffer(2 * x.numel(), device=dev, dtype=dtype)
+    calls = {"compress": lambda: dense_to_tilesparse(x, None, buf),
+             "quantize": lambda: quantize_and_compress(x, buf),
+             "amax": lambda: H.amax_into_workspace(x),
+             "block": lambda: FFNRelu.apply(x, W1, W2, sparse_data=buf, dtype=dtype),
+             "block_fp8": lambda: FFNRelu.apply(x, W1, W2, sparse_data=buf, dtype=dtype)}
+    fn = calls[what]
+    fn()
+    buf.reset_buffer()
+    want = fn()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        ws = _lib.workspace_for(x.device)
+        ws.buf, ws.epoch = ws.buf[:0], 0                 # (a stream of the pool may have been here before)
+    g = torch.cuda.CUDAGraph()
+    with pytest.raises(ValueError, match="captured into a HIP graph"):
+        with torch.cuda.graph(g, stream=side):
+            fn()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        assert ws.nbytes == 0 and _lib.workspace_for(x.device) is ws
+        buf.reset_buffer()
+        again = fn()
+        side.synchronize()
+    if what.startswith("block"):
+        assert torch.equal(again, want)
+    elif what == "compress":
+        assert torch.equal(again.bitmask, want.bitmask) and torch.equal(again.prefix, want.prefix)
+
+
 def test_epoch_wrap_between_amax_and_compress(dev):
     """The workspace epoch wraps (buffer zeroed) only where no amax is
     pending: an amax taken at the last epoch still reaches its compress."""
