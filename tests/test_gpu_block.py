@@ -313,6 +313,22 @@ def test_blocks_of_one_buffer(dev, store, in_place):
     assert not buf.overflowed()
 
 
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", STORES)
+def test_block_in_a_buffer_too_small(dev, square, store):
+    """Values that do not fit are dropped and flagged; y does not depend on them."""
+    p, _ = _operands(dev, 208, 48, 528, 48)
+    outs, bufs = [], []
+    for block in (True, False):
+        bufs.append(_buffer(208 * 528 // 5 // 32 * 32, dev, store))
+        with torch.no_grad():
+            outs.append(_block(p, store, square, block, bufs[-1]))
+    _same(*outs, "y")
+    _same(bufs[0].vals, bufs[1].vals, "values")
+    _same(bufs[0].offset, bufs[1].offset, "cursor")
+    assert bufs[0].overflowed() and bufs[1].overflowed()
+
+
 @pytest.mark.parametrize("store", STORES)
 def test_epoch_wrap_inside_a_block(dev, store):
     """The workspace's counter wraps (and clears the amax slot) at every place
