@@ -461,6 +461,8 @@ struct ActGrad {
 
 ActGrad act_grad(const Tensor& dz, Held& h, bool bias, bool rows, bool cols)
 {
+    // (the product behind dz may have come in another type, under autocast)
+    TORCH_CHECK_TYPE(dz.scalar_type() == at::kBFloat16, "the activation's gradient: grad must be bfloat16");
     const int stored = h.fp8 ? 1 : 0;
     ActGrad o;
     if (bias || rows || cols) {

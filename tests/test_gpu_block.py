@@ -313,6 +313,25 @@ def test_blocks_of_one_buffer(dev, store, in_place):
     assert not buf.overflowed()
 
 
+@pytest.mark.parametrize("block", [True, False])
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("store", ["bf16", "e4m3"])
+def test_backward_under_autocast(dev, block, square, store):
+    """A backward that runs inside autocast: in bfloat16 nothing changes, in
+    float16 the bf16 products would come in a type the activation's gradient
+    does not take, and are refused (the fp8 ones are not autocast)."""
+    p, dY = _operands(dev, 80, 48, 144, 32)
+    want = _step(p, dY, store, square, block)
+    for dtype in (torch.bfloat16, torch.float16):
+        q = _params(p)
+        y = _block(q, store, square, block)
+        refused = dtype == torch.float16 and store == "bf16"
+        with torch.autocast("cuda", dtype=dtype), pytest.raises(TypeError) if refused else contextlib.nullcontext():
+            y.backward(dY)
+        if not refused:
+            _compare({"y": y.detach(), **{k: t.grad for k, t in q.items()}}, want, 80)
+
+
 @pytest.mark.parametrize("square", [False, True])
 @pytest.mark.parametrize("store", STORES)
 def test_block_in_a_buffer_too_small(dev, square, store):
