@@ -299,10 +299,21 @@ void quantize_t(const Tensor& x, const Tensor& rows, const Fp8& t, int64_t amax_
                                  w.buf.data_ptr(), w.nbytes(), amax_epoch, stream_of(x)), "bs_quantize_e4m3fn_t");
 }
 
-// to_fp8 of a row-major matrix
-Fp8 to_fp8(const Tensor& x, Workspace& w)
+// x as the kernels read it: a bf16 matrix on the GPU (the backward's operands
+// come from autograd, whose saved-tensor hooks may hand back anything)
+Tensor operand(const Tensor& x)
 {
-    const Tensor c = x.contiguous();
+    TORCH_CHECK(x.is_cuda(), "bitsparse_amd runs on a ROCm GPU; got a tensor on ", x.device());
+    TORCH_CHECK_TYPE(x.scalar_type() == at::kBFloat16, "expected a bfloat16 tensor, got ", x.scalar_type());
+    TORCH_CHECK_VALUE(x.dim() == 2, "expected a matrix, got ", x.dim(), " dimensions");
+    return x.contiguous();
+}
+
+// to_fp8 of a row-major matrix
+Fp8 to_fp8(const Tensor& x)
+{
+    const Tensor c = operand(x);
+    Workspace& w = ws_of(c);
     const Fp8 o = rows_like(c);
     w.prepare(kAmaxBytes, 1);
     quantize_rows(c, o, amax(c, false, Tensor(), w), w);
@@ -310,9 +321,10 @@ Fp8 to_fp8(const Tensor& x, Workspace& w)
 }
 
 // an operand multiplied from the right: column-major codes
-Fp8 right_operand(const Tensor& x, Workspace& w)
+Fp8 right_operand(const Tensor& x)
 {
-    const Tensor c = x.contiguous();
+    const Tensor c = operand(x);
+    Workspace& w = ws_of(c);
     const Fp8 t = transposed_like(c);
     w.prepare(kAmaxBytes, 1);
     quantize_t(c, Tensor(), t, amax(c, false, Tensor(), w), w);
@@ -461,8 +473,10 @@ struct ActGrad {
 
 ActGrad act_grad(const Tensor& dz, Held& h, bool bias, bool rows, bool cols)
 {
-    // (the product behind dz may have come in another type, under autocast)
+    // (the product behind dz may have come in another type, under autocast, or of other operands than the forward's)
     TORCH_CHECK_TYPE(dz.scalar_type() == at::kBFloat16, "the activation's gradient: grad must be bfloat16");
+    TORCH_CHECK_VALUE(dz.dim() == 2 && dz.size(0) == h.M && dz.size(1) == h.N && dz.is_contiguous(),
+                      "the activation's gradient: grad shape ", dz.sizes(), " != ", at::IntArrayRef({h.M, h.N}));
     const int stored = h.fp8 ? 1 : 0;
     ActGrad o;
     if (bias || rows || cols) {
@@ -514,10 +528,9 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& b1
               const Tensor& err, bool in_place, bool packed, bool fp8, bool square, double k)
 {
     const c10::DeviceGuard guard(x.device());
-    Workspace& w = ws_of(x);
     Tensor z;
     if (fp8) {
-        const Fp8 a = to_fp8(x, w), b = to_fp8(W1, w);
+        const Fp8 a = to_fp8(x), b = to_fp8(W1);
         z = fp8_mm(a, {b.codes.t(), b.scale}, at::kBFloat16);
     } else {
         z = at::mm(x, W1.t());
@@ -526,7 +539,7 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& b1
     z.reset();          // (the down-projection does not need its room)
     Tensor y;
     if (fp8) {
-        const Fp8 b = to_fp8(W2, w);
+        const Fp8 b = to_fp8(W2);
         y = fp8_mm({a.operand, a.operand_scale}, {b.codes.t(), b.scale}, at::kBFloat16);
     } else {
         y = at::mm(a.operand, W2.t());
@@ -539,29 +552,29 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& b1
 // g W2 formed by the caller, where its graph is wanted and the operations here
 // would not record one (it is overwritten).
 std::vector<std::optional<Tensor>>
-block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const py::list& held, bool packed,
-               bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
+block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const py::list& held, int64_t M,
+               int64_t N, bool packed, bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
                const std::vector<bool>& need, const std::optional<Tensor>& dh)
 {
-    const c10::DeviceGuard guard(x.device());
-    Held h = take_held(held, x.size(0), W1.size(0), packed, fp8, square, k);
+    const c10::DeviceGuard guard(g.device());
+    Held h = take_held(held, M, N, packed, fp8, square, k);
+    TORCH_CHECK_VALUE(g.dim() == 2 && g.size(0) == M, "the gradient's rows are not the activation's");
     const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3], need_b2 = need[4];
     std::vector<std::optional<Tensor>> out(5);
-    Workspace& w = ws_of(x);
     if (need_b2) out[4] = col_sum(g);
     Fp8 g8;
-    if (fp8) g8 = to_fp8(g, w);
+    if (fp8) g8 = to_fp8(g);
     if (need_W2) out[3] = down_weight_grad(fp8 ? g8.codes : g, g8.scale, h);
     if (!(need_x || need_W1 || need_b1)) return out;
-    const Tensor dz = dh ? *dh : fp8 ? fp8_mm(g8, right_operand(W2, w), at::kBFloat16) : at::mm(g, W2);
+    const Tensor dz = dh ? *dh : fp8 ? fp8_mm(g8, right_operand(W2), at::kBFloat16) : at::mm(g, W2);
     g8 = Fp8();
     const bool sums = need_b1 && !at::GradMode::is_enabled();
     const ActGrad a = act_grad(dz, h, sums, fp8 && need_x, fp8 && need_W1);
     if (need_b1) out[2] = sums ? a.bias : col_sum(dz);
     if (fp8) {
         const at::ScalarType gd = grad_dtype.value_or(at::kFloat8_e4m3fn);
-        if (need_x) out[0] = widened(fp8_mm(a.rows, right_operand(W1, w), gd));
-        if (need_W1) out[1] = widened(fp8_mm(a.cols, right_operand(x, w), gd));
+        if (need_x) out[0] = widened(fp8_mm(a.rows, right_operand(W1), gd));
+        if (need_W1) out[1] = widened(fp8_mm(a.cols, right_operand(x), gd));
     } else {
         if (need_x) out[0] = at::mm(dz, W1);
         if (need_W1) out[1] = at::mm(dz.t(), x);      // W1's own layout, as autograd forms it

@@ -276,7 +276,7 @@ class _FFNBlock(Function):
         x, W1, W2 = ctx.saved_tensors
         h: BitsparseTensor = ctx.h_sparse
         ctx.h_sparse = None
-        held, packed = [h.vals, h.bitmask, h.prefix, h.vals_offset, h.scale], h.pack_sbit
+        held, shape, packed = [h.vals, h.bitmask, h.prefix, h.vals_offset, h.scale], h.shape, h.pack_sbit
         del h
         dh = None
         # create_graph: the fp8 product has its graph from MatmulFp8
@@ -284,7 +284,7 @@ class _FFNBlock(Function):
             g8, scale = to_fp8(grad_output)
             dh = matmul(g8, W2, True, a_scale=scale)
         grads = native().block_backward(
-            grad_output, x, W1, W2, held, packed, ctx.fp8, ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE,
+            grad_output, x, W1, W2, held, *shape, packed, ctx.fp8, ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE,
             ctx.needs_input_grad[:5], dh)
         return *grads, None, None, None
 

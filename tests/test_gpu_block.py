@@ -332,6 +332,33 @@ def test_backward_under_autocast(dev, block, square, store):
             _compare({"y": y.detach(), **{k: t.grad for k, t in q.items()}}, want, 80)
 
 
+@pytest.mark.parametrize("block", [True, False])
+@pytest.mark.parametrize("store", ["bf16", "e4m3"])
+@pytest.mark.parametrize("name", ["x", "W1", "W2"])
+@pytest.mark.parametrize("kind", ["float32", "float16", "cpu", "flat", "wider", "longer"])
+def test_saved_tensors_of_another_kind(dev, block, store, name, kind):
+    """A saved-tensor hook that hands the backward an operand in another type,
+    on another device or of another shape: an error, and nothing read as what
+    it is not."""
+    p, dY = _operands(dev, 80, 48, 144, 32)
+    q = _params(p)
+    shape = tuple(q[name].shape)
+
+    def unpack(t):
+        # (x @ W1.T saves W1 as a transposed view)
+        if tuple(t.shape) not in (shape, shape[::-1]):
+            return t
+        # (zeros around it: other shapes, all fp8 products of them possible by themselves)
+        pad = torch.nn.functional.pad
+        return {"float32": t.float, "float16": t.half, "cpu": t.cpu, "flat": t.flatten,
+                "wider": lambda: pad(t, (0, 64)), "longer": lambda: pad(t, (0, 0, 0, 64))}[kind]()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = _block(q, store, False, block)
+    with pytest.raises((RuntimeError, TypeError, ValueError, IndexError, AssertionError)):
+        y.backward(dY)
+    torch.cuda.synchronize(dev)
+
+
 @pytest.mark.parametrize("square", [False, True])
 @pytest.mark.parametrize("store", STORES)
 def test_block_in_a_buffer_too_small(dev, square, store):
