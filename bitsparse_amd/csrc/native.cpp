@@ -323,7 +323,8 @@ Fp8 to_fp8(const Tensor& x)
 // an operand multiplied from the right: column-major codes
 Fp8 right_operand(const Tensor& x)
 {
-    const Tensor c = operand(x);
+    Tensor c = operand(x);
+    if (reinterpret_cast<uintptr_t>(c.data_ptr()) & 15) c = c.clone();      // the kernel loads 16 bytes
     Workspace& w = ws_of(c);
     const Fp8 t = transposed_like(c);
     w.prepare(kAmaxBytes, 1);

@@ -359,6 +359,26 @@ def test_saved_tensors_of_another_kind(dev, block, store, name, kind):
     torch.cuda.synchronize(dev)
 
 
+@pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("layout", ["misaligned", "transposed", "padded"])
+def test_saved_tensors_in_another_layout(dev, store, layout):
+    """... and one that hands back the same values at another address (a view
+    into a flat buffer) or with other strides changes nothing."""
+    p, dY = _operands(dev, 80, 48, 144, 32)
+    want = _step(p, dY, store, False, False)
+
+    def unpack(t):
+        t = t.contiguous()
+        if layout == "misaligned":
+            return torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)
+        return t.t().contiguous().t() if layout == "transposed" else torch.nn.functional.pad(t, (0, 8))[:, :t.shape[1]]
+    q = _params(p)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = _block(q, store, False, True)
+    y.backward(dY)
+    _compare({"y": y.detach(), **{k: t.grad for k, t in q.items()}}, want, 80)
+
+
 @pytest.mark.parametrize("square", [False, True])
 @pytest.mark.parametrize("store", STORES)
 def test_block_in_a_buffer_too_small(dev, square, store):
