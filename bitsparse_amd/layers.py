@@ -222,7 +222,8 @@ def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor |
     TensorBuffer of the stored type, outside autocast, tracing, forward-mode
     AD and the options that choose another path.  Everything else takes the
     layers' separate nodes, with their errors."""
-    if torch.compiler.is_compiling():        # first: a tracer does not follow the addresses below
+    # first: neither tracers nor function transforms follow the addresses below
+    if torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active():
         return False
     if sparse_data is None or not (_plain(x) and _plain(W1) and _plain(W2) and plain_cursor(sparse_data)):
         return False
