@@ -98,7 +98,7 @@ class FFNRelu:
 
         if _block_ok(x, W1, W2, b1, b2, sparse_data, pack_sbit, dtype):
             y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, is_fp8(dtype), False)
-            return y.reshape(*bs_dims, y.shape[-1])
+            return _block_result(y, bs_dims, b2)
         if not is_fp8(dtype) and not pack_sbit and USE_FUSED_UP and fused_linear_relu_ok(x, W1, b1, sparse_data):
             y = _UpReluLinear.apply(x, W1, b1, W2, sparse_data, False)
         else:
@@ -193,7 +193,7 @@ class FFNRelu2:
         x = x.reshape(-1, x.shape[-1])
         if _block_ok(x, W1, W2, b1, b2, sparse_data, pack_sbit, storage_dtype):
             y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, is_fp8(storage_dtype), True)
-            return y.reshape(*bs_dims, y.shape[-1])
+            return _block_result(y, bs_dims, b2)
         if (not is_fp8(storage_dtype) and not pack_sbit and USE_FUSED_UP
                 and fused_linear_relu_ok(x, W1, b1, sparse_data)):
             y = _UpReluLinear.apply(x, W1, b1, W2, sparse_data, True)
@@ -251,6 +251,14 @@ def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor |
             b is not None and b.device != x.device for b in (b1, b2)):
         return False
     return not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
+
+
+def _block_result(y: Tensor, bs_dims: torch.Size, b2: Tensor | None) -> Tensor:
+    """The block's y in the shape of its input: a view, or with b2 a tensor of
+    its own, as the bias add makes it (a view refuses ``detach_()``)."""
+    if b2 is None:
+        return y.reshape(*bs_dims, y.shape[-1])
+    return y if len(bs_dims) == 1 else torch.ops.aten._unsafe_view(y, (*bs_dims, y.shape[-1]))
 
 
 class _FFNBlock(Function):

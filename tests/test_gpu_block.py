@@ -294,6 +294,28 @@ def test_block_input_layouts(dev, store, layout):
 
 
 @pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("biases", [(), ("b1",), ("b2",), ("b1", "b2")])
+@pytest.mark.parametrize("dims", [2, 3])
+def test_block_result_changed_in_place(dev, store, biases, dims):
+    """In-place calls on y: what the separate nodes' result allows, with their gradients."""
+    p, dY = _operands(dev, 96, 48, 144, 48, biases)
+    if dims == 3:
+        p["x"], dY = p["x"].reshape(2, 48, 48), dY.reshape(2, 48, 48)
+    outs, views = [], []
+    for block in (True, False):
+        q = _params(p)
+        y = _block(q, store, False, block)
+        views.append(y._is_view())
+        if "b2" in biases:
+            assert not _block(q, store, False, block).detach_().requires_grad
+        y.mul_(2.0)
+        y.backward(dY)
+        outs.append({"y": y.detach(), **{k: t.grad for k, t in q.items() if t is not None}})
+    assert views[0] == views[1]
+    _compare(*outs, 96)
+
+
+@pytest.mark.parametrize("store", STORES)
 @pytest.mark.parametrize("in_place", [False, True])
 def test_blocks_of_one_buffer(dev, store, in_place):
     """Blocks appended to one buffer, backwards in the reverse order; then
