@@ -1870,7 +1870,7 @@ __global__ __launch_bounds__(kThreads) void relu2_grad_kernel(GatherArgs a)
     // Memory still moves the 128-byte line of a tile row whenever any of its
     // eight chunks is read, so the skip saves no HBM traffic below whole
     // rows, but it keeps the unused chunks out of the CU: reading every chunk
-    // of a live row measured 55.7 against 51.7 us at the configs[3] shape.
+    // of a live row measured 55.7 against 51.7 us at 4096 x 16384.
     const int64_t vo = a.vals_offset ? *a.vals_offset : 0;
     float sc = 1.0f;
     if constexpr (HAS_SCALE) sc = *a.scale;

@@ -878,7 +878,7 @@ static int64_t apk_bytes(int64_t M, int64_t K) { return (M + 31) / 32 * apk_nkb(
 
 // Launch plan: 512-row workgroups when they cover M with no more padding
 // than 256-row ones (half the decode work per MFMA); else 256 x 128 with two
-// workgroups per CU (configs[1]'s 768 x 8192 x 3072: 78 us per call against
+// workgroups per CU (768 x 8192 x 3072: 78 us per call against
 // 87 us with one 256 x 256 workgroup per CU, and 104 us with 768 x 64
 // workgroups, which decode each B tile once but re-read A for every 64
 // columns).  BITSPARSE_DW_CFG (256 / 512 / 768 / 2561 for 256h / 2562 for
