@@ -62,6 +62,7 @@ void check(int rc, const char* what)
     if (rc == BS_OK) return;
     const char* msg = L.bs_last_error();
     if (rc == BS_ERR_INVALID) TORCH_CHECK_VALUE(false, what, ": ", msg);
+    const py::gil_scoped_acquire gil;       // (a C++ node's backward has no interpreter lock)
     py::set_error(py::module_::import("bitsparse_amd._lib").attr("BitsparseHipError"),
                   (std::string(what) + " failed (" + std::to_string(rc) + "): " + msg).c_str());
     throw py::error_already_set();
@@ -105,13 +106,14 @@ constexpr int64_t kEpochLimit = (int64_t(1) << 30) - 1;
 // ignored by the kernels, so the buffer never needs clearing between calls.
 // When the counter wraps the buffer is zeroed again.
 //
-// Threads: every entry of this module is called from Python and holds the
-// interpreter lock throughout, which is what keeps a sequence that passes an
-// amax through the workspace whole, as long as nothing in it runs Python.  So
-// a sequence allocates its outputs first, then calls `prepare`, and makes no
-// call into torch from there to its last launch; the workspace's own torch
-// calls leave the thread's dispatch modes out.  (No mutex: a thread in a mode's
-// Python code gives the lock away, and one waiting for the mutex would not.)
+// Threads: every use of a workspace is in a call from Python and holds the
+// interpreter lock throughout (Biased's backward does not, and has no use of
+// one), which is what keeps a sequence that passes an amax through the
+// workspace whole, as long as nothing in it runs Python.  So a sequence
+// allocates its outputs first, then calls `prepare`, and makes no call into
+// torch from there to its last launch; the workspace's own torch calls leave
+// the thread's dispatch modes out.  (No mutex: a thread in a mode's Python code
+// gives the lock away, and one waiting for the mutex would not.)
 struct Workspace {
     explicit Workspace(c10::Device d) : device(d)
     {
@@ -414,9 +416,9 @@ Tensor down_weight_grad(const Tensor& g, const Tensor& g_scale, const Held& h)
 
 Tensor col_sum(const Tensor& g)
 {
-    // a graph of this gradient (create_graph), or a layout the kernel does not
-    // take: torch's own sum
-    if (at::GradMode::is_enabled() || !g.is_contiguous() || g.size(1) % 8 != 0 || g.numel() == 0 ||
+    // a graph of this gradient (create_graph), a batch of them (no storage of
+    // its own), or a layout the kernel does not take: torch's own sum
+    if (at::GradMode::is_enabled() || !g.has_storage() || g.scalar_type() != at::kBFloat16 || !g.is_contiguous() || g.size(1) % 8 != 0 || g.numel() == 0 ||
         (reinterpret_cast<uintptr_t>(g.data_ptr()) & 15) || g.numel() >= (int64_t(1) << 31))
         return g.sum(0);
     const int64_t R = g.size(0), C = g.size(1), need = L.bs_col_sum_workspace_bytes(R, C);
@@ -424,6 +426,24 @@ Tensor col_sum(const Tensor& g)
     check(L.bs_col_sum(g.data_ptr(), R, C, out.data_ptr(), part.data_ptr(), need, stream_of(g)), "bs_col_sum");
     return out;
 }
+
+// The block's y, b2 added, as a node of b2's own: the sum is there already, and
+// forward gives y in the shape of the block's input, as a tensor of its own (a
+// view refuses detach_()).  b2's gradient needs nothing of the block, so a walk
+// for b2 alone leaves the compressed activation to a later one.
+struct Biased : torch::autograd::Function<Biased> {
+    static Tensor forward(torch::autograd::AutogradContext*, const Tensor& y, const Tensor& /*b2*/,
+                          const std::vector<int64_t>& shape)
+    {
+        return at::_unsafe_view(y, shape);
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                   const torch::autograd::variable_list& grads)
+    {
+        const Tensor g = grads[0].reshape({-1, grads[0].size(-1)});
+        return {ctx->needs_input_grad(0) ? g : Tensor(), ctx->needs_input_grad(1) ? col_sum(g) : Tensor(), Tensor()};
+    }
+};
 
 // The activation step inside a block, on its up-projection z, which nothing
 // reads afterwards: r = relu(z + bias) compressed, and what the down-projection
@@ -549,7 +569,7 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& b1
     return {y, a.bitmask, a.prefix, a.start, a.next, optional(a.scale)};
 }
 
-// (dx, dW1, db1, dW2, db2), each where `need` asks for it.  `dh`: the product
+// (dx, dW1, db1, dW2), each where `need` asks for it.  `dh`: the product
 // g W2 formed by the caller, where its graph is wanted and the operations here
 // would not record one (it is overwritten).
 std::vector<std::optional<Tensor>>
@@ -560,9 +580,8 @@ block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor&
     const c10::DeviceGuard guard(g.device());
     Held h = take_held(held, M, N, packed, fp8, square, k);
     TORCH_CHECK_VALUE(g.dim() == 2 && g.size(0) == M, "the gradient's rows are not the activation's");
-    const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3], need_b2 = need[4];
-    std::vector<std::optional<Tensor>> out(5);
-    if (need_b2) out[4] = col_sum(g);
+    const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3];
+    std::vector<std::optional<Tensor>> out(4);
     Fp8 g8;
     if (fp8) g8 = to_fp8(g);
     if (need_W2) out[3] = down_weight_grad(fp8 ? g8.codes : g, g8.scale, h);
@@ -606,6 +625,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("gemm_compressed", &gemm_compressed);
     m.def("block_forward", &block_forward);
     m.def("block_backward", &block_backward);
+    m.def("biased", [](const Tensor& y, const Tensor& b2, const std::vector<int64_t>& shape) {
+        return Biased::apply(y, b2, shape);
+    });
     // the block's steps by themselves
     m.def("activate", [](const Tensor& z, const std::optional<Tensor>& bias, const Tensor& vals,
                          const std::optional<Tensor>& offset, const Tensor& err, bool in_place, bool packed, bool fp8,

@@ -97,8 +97,7 @@ class FFNRelu:
         x = x.reshape(-1, x.shape[-1])
 
         if _block_ok(x, W1, W2, b1, b2, sparse_data, pack_sbit, dtype):
-            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, is_fp8(dtype), False)
-            return _block_result(y, bs_dims, b2)
+            return _block(x, W1, b1, W2, b2, bs_dims, sparse_data, is_fp8(dtype), False)
         if not is_fp8(dtype) and not pack_sbit and USE_FUSED_UP and fused_linear_relu_ok(x, W1, b1, sparse_data):
             y = _UpReluLinear.apply(x, W1, b1, W2, sparse_data, False)
         else:
@@ -192,8 +191,7 @@ class FFNRelu2:
         bs_dims = x.shape[:-1]
         x = x.reshape(-1, x.shape[-1])
         if _block_ok(x, W1, W2, b1, b2, sparse_data, pack_sbit, storage_dtype):
-            y = _FFNBlock.apply(x, W1, b1, W2, b2, sparse_data, is_fp8(storage_dtype), True)
-            return _block_result(y, bs_dims, b2)
+            return _block(x, W1, b1, W2, b2, bs_dims, sparse_data, is_fp8(storage_dtype), True)
         if (not is_fp8(storage_dtype) and not pack_sbit and USE_FUSED_UP
                 and fused_linear_relu_ok(x, W1, b1, sparse_data)):
             y = _UpReluLinear.apply(x, W1, b1, W2, sparse_data, True)
@@ -253,12 +251,13 @@ def _block_ok(x: Tensor, W1: Tensor, W2: Tensor, b1: Tensor | None, b2: Tensor |
     return not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
 
 
-def _block_result(y: Tensor, bs_dims: torch.Size, b2: Tensor | None) -> Tensor:
-    """The block's y in the shape of its input: a view, or with b2 a tensor of
-    its own, as the bias add makes it (a view refuses ``detach_()``)."""
+def _block(x, W1, b1, W2, b2, bs_dims, sparse_data: TensorBuffer, fp8: bool, square: bool) -> Tensor:
+    """The block's y in the shape of its input.  The node adds b2; b2's
+    gradient, which needs nothing of the node, has one of its own."""
+    y = _FFNBlock.apply(x, W1, b1, W2, (b2,), sparse_data, fp8, square)     # (in a tuple: no edge to b2)
     if b2 is None:
         return y.reshape(*bs_dims, y.shape[-1])
-    return y if len(bs_dims) == 1 else torch.ops.aten._unsafe_view(y, (*bs_dims, y.shape[-1]))
+    return native().biased(y, b2, (*bs_dims, y.shape[-1]))
 
 
 class _FFNBlock(Function):
@@ -269,7 +268,7 @@ class _FFNBlock(Function):
     def forward(ctx, x, W1, b1, W2, b2, buf, fp8, square):
         offset, in_place = buf.native_cursor()
         y, bitmask, prefix, start, buf._offset, scale = native().block_forward(
-            x, W1, b1, W2, b2, buf.vals, offset, buf.err_flags, in_place, buf.pack_sbit, fp8, square,
+            x, W1, b1, W2, b2[0], buf.vals, offset, buf.err_flags, in_place, buf.pack_sbit, fp8, square,
             float(RELU2_SCALE))
         M, N = x.shape[0], W1.shape[0]
         ctx.h_sparse = BitsparseTensor(buf.vals, bitmask, prefix, (M, N), torch.float8_e4m3fn if fp8 else torch.bfloat16,
@@ -294,8 +293,8 @@ class _FFNBlock(Function):
             dh = matmul(g8, W2, True, a_scale=scale)
         grads = native().block_backward(
             grad_output, x, W1, W2, held, *shape, packed, ctx.fp8, ctx.square, float(RELU2_SCALE), config.FP8_GRAD_DTYPE,
-            ctx.needs_input_grad[:5], dh)
-        return *grads, None, None, None
+            ctx.needs_input_grad[:4], dh)
+        return *grads, None, None, None, None
 
 
 # ------------------------------------------------------------

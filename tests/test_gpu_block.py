@@ -201,7 +201,8 @@ def _block(p, store, square, block, buf=None):
         y = layer.apply(p["x"], p["W1"], p["W2"], p["b1"], p["b2"], sparse_data=buf,
                         pack_sbit=store.endswith("packed"), **{kw: E4M3 if store.startswith("e4m3") else torch.bfloat16})
     if y.requires_grad:
-        taken = any(n.name() == "_FFNBlockBackward" for n in _graph_nodes(y))
+        # (a block none of whose operands but b2 asks for a gradient leaves b2's node alone)
+        taken = any(n.name() == "_FFNBlockBackward" or n.name().endswith("Biased>") for n in _graph_nodes(y))
         assert taken == block, "the node that was asked for"
     return y
 
@@ -312,6 +313,29 @@ def test_block_result_changed_in_place(dev, store, biases, dims):
         y.backward(dY)
         outs.append({"y": y.detach(), **{k: t.grad for k, t in q.items() if t is not None}})
     assert views[0] == views[1]
+    _compare(*outs, 96)
+
+
+@pytest.mark.parametrize("store", STORES)
+@pytest.mark.parametrize("dims", [2, 3])
+def test_gradient_of_b2_alone(dev, store, dims):
+    """A walk for b2 alone, for one gradient and for a batch of them, needs nothing of
+    the block: the whole walk after it finds the compressed activation."""
+    p, dY = _operands(dev, 96, 48, 144, 48)
+    if dims == 3:
+        p["x"], dY = p["x"].reshape(2, 48, 48), dY.reshape(2, 48, 48)
+    outs = []
+    for block in (True, False):
+        q = _params(p)
+        y = _block(q, store, True, block)
+        one, = torch.autograd.grad(y, q["b2"], dY, retain_graph=True)
+        batch, = torch.autograd.grad(y, q["b2"], torch.stack([dY, 2 * dY]), retain_graph=True, is_grads_batched=True)
+        y.backward(dY)
+        bound = 2.0 ** -8 * one.double().abs() + 1e-2          # sums in another order, rounded once
+        assert ((q["b2"].grad - one).double().abs() <= bound).all()
+        assert ((batch[0] - one).double().abs() <= bound).all()
+        assert ((batch[1] - 2 * one).double().abs() <= 2 * bound).all()
+        outs.append({"y": y.detach(), **{k: t.grad for k, t in q.items()}})
     _compare(*outs, 96)
 
 
