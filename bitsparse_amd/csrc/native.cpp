@@ -569,17 +569,34 @@ block_forward(const Tensor& x, const Tensor& W1, const std::optional<Tensor>& b1
     return {y, a.bitmask, a.prefix, a.start, a.next, optional(a.scale)};
 }
 
-// (dx, dW1, db1, dW2), each where `need` asks for it.  `dh`: the product
+// `need` (x, W1, b1, W2 ask for gradients) without those that this walk is not
+// after (torch.autograd.grad or backward(inputs=) of some of them): the separate
+// nodes' products were left out by the engine itself.
+std::vector<bool> asked_for(std::vector<bool> need)
+{
+    const std::shared_ptr<torch::autograd::Node> node = torch::autograd::get_current_node();
+    if (!node || node->name() != "_FFNBlockBackward") return need;
+    size_t edge = 0;
+    for (size_t i = 0; i < need.size(); i++) {
+        if (i == 2 && node->num_outputs() < need.size()) continue;      // no b1, no edge to it
+        need[i] = need[i] && node->task_should_compute_output(edge);
+        edge++;
+    }
+    return need;
+}
+
+// (dx, dW1, db1, dW2), each where `wanted` and this walk ask for it.  `dh`: the product
 // g W2 formed by the caller, where its graph is wanted and the operations here
 // would not record one (it is overwritten).
 std::vector<std::optional<Tensor>>
 block_backward(const Tensor& g, const Tensor& x, const Tensor& W1, const Tensor& W2, const py::list& held, int64_t M,
                int64_t N, bool packed, bool fp8, bool square, double k, const std::optional<at::ScalarType>& grad_dtype,
-               const std::vector<bool>& need, const std::optional<Tensor>& dh)
+               const std::vector<bool>& wanted, const std::optional<Tensor>& dh)
 {
     const c10::DeviceGuard guard(g.device());
     Held h = take_held(held, M, N, packed, fp8, square, k);
     TORCH_CHECK_VALUE(g.dim() == 2 && g.size(0) == M, "the gradient's rows are not the activation's");
+    const std::vector<bool> need = asked_for(wanted);
     const bool need_x = need[0], need_W1 = need[1], need_b1 = need[2], need_W2 = need[3];
     std::vector<std::optional<Tensor>> out(4);
     Fp8 g8;

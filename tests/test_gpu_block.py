@@ -339,6 +339,40 @@ def test_gradient_of_b2_alone(dev, store, dims):
     _compare(*outs, 96)
 
 
+@pytest.mark.parametrize("store", ["bf16", "e4m3"])
+@pytest.mark.parametrize("biases", [("b2",), ("b1", "b2")])
+@pytest.mark.parametrize("leaf", [True, False])
+def test_walks_for_some_operands(dev, store, biases, leaf, monkeypatch):
+    """Walks after some of the operands' gradients form those alone, with the values of
+    a whole walk; all operands ask for gradients."""
+    from bitsparse_amd._lib import native
+    p, dY = _operands(dev, 96, 48, 144, 48, biases)
+    names = [n for n in NAMES if p[n] is not None]
+    whole = _step(p, dY, store, True, True)
+    inner, formed = native().block_backward, []
+
+    def spy(*args):
+        out = inner(*args)
+        formed.append({n for n, t in zip(("x", "W1", "b1", "W2"), out) if t is not None})
+        return out
+    monkeypatch.setattr(native(), "block_backward", spy)
+    for n in range(1, len(names) + 1):
+        for ask in itertools.combinations(names, n):
+            for walk in ("grad", "backward") if leaf else ("grad",):     # (backward's inputs are leaves here)
+                q = _params(p)
+                if not leaf:
+                    q["x"] = q["x"] * 1
+                y = _block(q, store, True, True)
+                formed.clear()
+                if walk == "grad":
+                    got = dict(zip(ask, torch.autograd.grad(y, [q[k] for k in ask], dY)))
+                else:
+                    torch.autograd.backward(y, dY, inputs=[q[k] for k in ask])
+                    got = {k: q[k].grad for k in ask}
+                _compare(got, {k: whole[k] for k in ask}, 96)
+                assert formed == ([set(ask) - {"b2"}] if set(ask) != {"b2"} else []), ask
+
+
 @pytest.mark.parametrize("store", STORES)
 @pytest.mark.parametrize("in_place", [False, True])
 def test_blocks_of_one_buffer(dev, store, in_place):
